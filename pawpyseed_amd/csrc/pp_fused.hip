@@ -83,11 +83,11 @@ __global__ __launch_bounds__(256) void k_fft_x_sphere(
     const int *__restrict__ site_pt, const int *__restrict__ site_np, const long *__restrict__ tab_off,
     const cplx<float> *__restrict__ phase, const float *__restrict__ table, int NB, cplx<float> *__restrict__ partial) {
   static_assert(NBW == 16, "lanes are 16 bands x 2 points x 2 projector halves");
-  constexpr int P = FX_PMAX, PH = FX_PMAX / 2, S = FX_S, G = FX_G;
+  constexpr int P = FX_PMAX, TS = FX_TS, PH = FX_PMAX / 2, S = FX_S, G = FX_G;
   extern __shared__ unsigned char smem_raw[];
   __shared__ int2 s_seg[FX_BL * G];  // per (line, slot): first point, length << 16 | x of the first point
-  __shared__ long s_tbase[G];        // table row of point p of the slot's site: s_tbase + p * np
-  __shared__ int s_np[G];
+  __shared__ long s_tbase[G];        // table row of point p of the slot's site: s_tbase + p * stride
+  __shared__ int s_np[G], s_ts[G];   // its projectors and its table row stride
   const int bid = blockIdx.x, xcd = bid & 7, r8 = bid >> 3;
   const int slice = r8 % nslices, item = (r8 / nslices) * 8 + xcd;
   if (item >= nitems)
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void k_fft_x_sphere(
   cplx<float> *buf = reinterpret_cast<cplx<float> *>(smem_raw);
   cplx<float> *twl = buf + tot;
   cplx<float> *s_ph = twl + twlen;                                     // [G][maxlen]
-  float *s_tab = reinterpret_cast<float *>(s_ph + (long)G * maxlen);  // [G][maxlen][np]
+  float *s_tab = reinterpret_cast<float *>(s_ph + (long)G * maxlen);  // [G][maxlen][stride]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, b = lane % NBW;
   const int pq = (lane / NBW) & 1, j0 = (lane / NBW >> 1) * PH;
   stage_twiddles<float, 256>(twl, tw, twlen);
@@ -113,8 +113,10 @@ __global__ __launch_bounds__(256) void k_fft_x_sphere(
   if (tid < G) {
     const int site = isites[item * G + tid];
     const int np = site >= 0 ? (FULL ? P : site_np[site]) : 0;
+    const int ts = table_stride(np, true);
     s_np[tid] = np;
-    s_tbase[tid] = site >= 0 ? tab_off[site] - (long)site_pt[site] * np : 0;
+    s_ts[tid] = ts;
+    s_tbase[tid] = site >= 0 ? tab_off[site] - (long)site_pt[site] * ts : 0;
   }
   int lo = -(1 << 30), hi = 1 << 30;
   if (bd.xb) {
@@ -156,8 +158,8 @@ __global__ __launch_bounds__(256) void k_fft_x_sphere(
         const int2 sv = s_seg[ln * G + s];
         len[r] = sv.y >> 16;
         p0[r] = sv.x;
-        nfl[r] = len[r] * s_np[s];
-        src[r] = table + s_tbase[s] + (long)sv.x * s_np[s];
+        nfl[r] = len[r] * s_ts[s];
+        src[r] = table + s_tbase[s] + (long)sv.x * s_ts[s];
       }
       const int most = max(nfl[0], max(nfl[1], nfl[2]));
       for (int e0 = 0; e0 < most; e0 += 64 * FX_STAGE) {
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(256) void k_fft_x_sphere(
           for (int k = 0; k < FX_STAGE; k++) {
             const int e = e0 + lane + 64 * k;
             if (e < nfl[r])
-              s_tab[(long)(wave + 4 * r) * maxlen * P + e] = v[r][k];
+              s_tab[(long)(wave + 4 * r) * maxlen * TS + e] = v[r][k];
           }
       }
 #pragma unroll
@@ -192,15 +194,15 @@ __global__ __launch_bounds__(256) void k_fft_x_sphere(
       const int len = sv.y >> 16;
       if (len == 0)
         continue;
-      const int np = FULL ? P : s_np[s];
-      const float *tp = s_tab + (long)s * maxlen * P + j0;
+      const int np = FULL ? P : s_np[s], ts = FULL ? TS : s_ts[s];
+      const float *tp = s_tab + (long)s * maxlen * TS + j0;
       const cplx<float> *ph = s_ph + s * maxlen;
       int x = (sv.y & 0xffff) + pq;
       if (x >= n)
         x -= n;
       for (int i = pq; i < len; i += 2) {
         const cplx<float> v = buf[x * NBW + b] * ph[i];
-        const float *t = tp + i * np;
+        const float *t = tp + i * ts;
 #pragma unroll
         for (int j = 0; j < PH; j++)
           if (FULL || j0 + j < np) {
@@ -445,7 +447,7 @@ static int basic_twlen(const AxisPlan &ap) { return ap.nstc > 0 ? ap.twoffc[0] :
 // staging of FX_G sites x fx_maxlen points
 static size_t fused_lds(const AxisPlan &ap, const pp_sphere *sp) {
   return ((size_t)ap.n * 16 + basic_twlen(ap) + (size_t)FX_G * sp->fx_maxlen) * sizeof(cplx<float>) +
-         (size_t)FX_G * sp->fx_maxlen * FX_PMAX * sizeof(float);
+         (size_t)FX_G * sp->fx_maxlen * FX_TS * sizeof(float);
 }
 
 // Work lists of the current tables, built on first use.
@@ -488,7 +490,7 @@ int fused_x_sums(pp_ctx *ctx, FftPlan *pl, pp_sphere *sp, const cplx<float> *gri
   const long nwg = (long)((sp->fx_nitems + 7) / 8) * 8 * nslices;
   const long es = (long)n1 * n2 * NB, s1 = (long)n2 * NB, s2 = NB;
   const cplx<float> *tw = fft_twiddles<float>(pl, 0);
-  const bool full = sp->pmin == FX_PMAX;
+  const bool full = *std::min_element(sp->nproj_site.begin(), sp->nproj_site.end()) == FX_PMAX;
   hipEvent_t ev;
   tbegin(ctx, K_FFT_X_SPHERE, &ev);
 #define PP_FX(MB, RM, FULL)                                                                                      \

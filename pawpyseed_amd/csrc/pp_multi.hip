@@ -29,11 +29,11 @@ const int *sphere_fftg(pp_sphere *sp);
 long sphere_generation(pp_sphere *sp);
 const unsigned *sphere_xmask(pp_sphere *sp, int *words);
 template <typename T> int make_phase(pp_ctx *ctx, pp_sphere *sp, const double *kfrac, cplx<T> *phase, bool expand);
-int sphere_pm_of(pp_sphere *sp, bool *full);
+int sphere_pm_of(pp_sphere *sp);
+long sphere_reduce_blocks(int nsites, int nbc);
 void sphere_item_fields(pp_ctx *ctx, pp_sphere *sp, ChunkItem &it);
 template <typename T>
-int sphere_sums_items(pp_ctx *ctx, const ChunkItem *items, int nitems, int NB, int PM, bool full, long maxblk,
-                      long maxred);
+int sphere_sums_items(pp_ctx *ctx, const ChunkItem *items, int nitems, int NB, int PM, long maxblk, long maxred);
 template <typename T>
 int fft_items(pp_ctx *ctx, FftPlan *pl, const ChunkItem *items, int nitems, int NB, int maxw, long maxzl,
               long maxyl);
@@ -54,8 +54,8 @@ struct MultiBatch {
 
 struct MultiState {
   FftPlan *pl = nullptr;
-  int NB = 64, PM = 8;
-  bool full = true, two = false;
+  int NB = 64, PM = 4;
+  bool two = false;
   ChunkItem *d_items = nullptr;
   std::vector<MultiBatch> batches;
 };
@@ -95,19 +95,10 @@ static int multi_prepare(pp_ctx *ctx, const MultiArgs &a, const MultiBufs &mb, M
     return PP_ERR_UNSUPPORTED;
   // plans: phases offsets, projector slots
   std::vector<long> ph_off(a.nstruct * a.nk + 1, 0);
-  S.PM = 8;
-  S.full = true;
   for (int s = 0; s < a.nstruct; s++) {
-    bool full = false;
-    const int pm = sphere_pm_of(a.plans[s], &full);
-    S.PM = std::max(S.PM, pm);
+    S.PM = std::max(S.PM, sphere_pm_of(a.plans[s]));
     for (int k = 0; k < a.nk; k++)
       ph_off[s * a.nk + k + 1] = ph_off[s * a.nk + k] + std::max<long>(1, sphere_npts(a.plans[s]));
-  }
-  for (int s = 0; s < a.nstruct; s++) {
-    bool full = false;
-    const int pm = sphere_pm_of(a.plans[s], &full);
-    S.full = S.full && full && pm == S.PM;
   }
   // plane-wave bounds of every k (one host synchronisation)
   const int nbnd = 2 * n0 * n1 + 2 * n0 + 3;
@@ -206,7 +197,7 @@ static int multi_prepare(pp_ctx *ctx, const MultiArgs &a, const MultiBufs &mb, M
   for (int s = 0; s < a.nstruct; s++) {
     ChunkItem tmp;
     sphere_item_fields(ctx, a.plans[s], tmp);
-    part_bytes = std::max(part_bytes, sizeof(cplx<double>) * (size_t)tmp.nsites * tmp.nparts * NB * S.PM);
+    part_bytes = std::max(part_bytes, sizeof(cplx<T>) * (size_t)tmp.nsites * tmp.nparts * NB * S.PM);
   }
   part_bytes = (std::max<size_t>(part_bytes, 256) + 255) / 256 * 256;
   const size_t grid_bytes = (sizeof(cplx<T>) * (size_t)npts_grid * NB + 255) / 256 * 256;
@@ -226,7 +217,7 @@ static int multi_prepare(pp_ctx *ctx, const MultiArgs &a, const MultiBufs &mb, M
       bt.maxzl = std::max<long>(bt.maxzl, it.nzl);
       bt.maxyl = std::max<long>(bt.maxyl, it.nyl);
       bt.maxblk = std::max<long>(bt.maxblk, (long)it.nsites * it.nparts);
-      bt.maxred = std::max<long>(bt.maxred, (long)it.nsites * it.nbc * S.PM);
+      bt.maxred = std::max(bt.maxred, sphere_reduce_blocks(it.nsites, it.nbc));
     }
     S.batches.push_back(bt);
   }
@@ -262,7 +253,7 @@ template <typename T> static int multi_launch(pp_ctx *ctx, const MultiState &S) 
     const ChunkItem *it = S.d_items + bt.first;
     st = fft_items<T>(ctx, S.pl, it, bt.count, S.NB, bt.maxw, bt.maxzl, bt.maxyl);
     if (st == PP_OK)
-      st = sphere_sums_items<T>(ctx, it, bt.count, S.NB, S.PM, S.full, bt.maxblk, bt.maxred);
+      st = sphere_sums_items<T>(ctx, it, bt.count, S.NB, S.PM, bt.maxblk, bt.maxred);
     if (st != PP_OK)
       break;
   }

@@ -23,6 +23,21 @@ struct SiteGeo {
   int chan_off;  // offset into the channel-l array
 };
 
+// Projector slots per point of a site's table rows: its projector count
+// rounded up to one of the counts the sum kernels are compiled for, the
+// slots past the last projector zero, so that the kernels' projector loops
+// carry no guards (with a guard per projector the sums of a plan with two
+// species took 116 us per chunk where the unguarded ones take a fifth).  FP32
+// rows hold whole groups of four, the rows of one 4x4x1 MFMA operand.
+__host__ __device__ inline int table_stride(int np, bool fp32) {
+  if (fp32)
+    return np <= 4 ? 4 : np <= 24 ? (np + 3) / 4 * 4 : np <= 32 ? 32 : np <= 48 ? 48 : 64;
+  return np <= 4 ? 4 : np <= 8 ? 8 : np <= 9 ? 9 : np <= 12 ? 12 : np <= 16 ? 16 : np <= 18 ? 18 : np <= 24 ? 24
+         : np <= 32 ? 32 : np <= 48 ? 48 : 64;
+}
+#define PP_STRIDES_F32(X) X(4) X(8) X(12) X(16) X(20) X(24) X(32) X(48) X(64)
+#define PP_STRIDES_F64(X) X(4) X(8) X(9) X(12) X(16) X(18) X(24) X(32) X(48) X(64)
+
 // R0, rmax, ngrid and the candidate box (g, c) of a site whose coord is
 // set (pp_sphere.hip).
 void site_box(const double *lattice, const int *fftg, double rmax, int ngrid, SiteGeo &g);
@@ -33,6 +48,7 @@ void site_box(const double *lattice, const int *fftg, double rmax, int ngrid, Si
 constexpr int FX_BY = 4, FX_BZ = 4, FX_BL = FX_BY * FX_BZ;
 constexpr int FX_S = 3, FX_G = 4 * FX_S;
 constexpr int FX_PMAX = 18;  // projectors per site the fused kernel holds
+constexpr int FX_TS = 20;    // table_stride(FX_PMAX, true)
 
 // Work lists of the fused x pass (host).  items: (y0, z0, sites, 0) per
 // item; isites: FX_G slots per item (site or -1); bitem: items of block b
@@ -60,7 +76,7 @@ struct pp_sphere {
   std::vector<double> rmax;
   std::vector<int> nproj_site, proj_off;  // host
   std::vector<int> site_pt_h;
-  int ptot = 0, pmax = 0, pmin = 0;
+  int ptot = 0, pmax = 0;
   long npts = 0;
   long gen = 0;  // build count: graphs captured against older tables refuse to replay
   // device

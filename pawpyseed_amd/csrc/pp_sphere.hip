@@ -251,7 +251,8 @@ __global__ __launch_bounds__(256) void k_site_values(const SiteGeo *__restrict__
   const double ct = cos(theta);
   const int n = s.ngrid;
   const double *x = spl + s.spl_off;
-  T *out = table + tab_off[s_id] + (long)i * s.nproj;
+  const int ts = table_stride(s.nproj, sizeof(T) == 4);
+  T *out = table + tab_off[s_id] + (long)i * ts;
   int p = 0;
   for (int ch = 0; ch < s.nchan; ch++) {
     const int l = chan_l[s.chan_off + ch];
@@ -283,6 +284,8 @@ __global__ __launch_bounds__(256) void k_site_values(const SiteGeo *__restrict__
       out[p] = (T)(m < 0 ? pl * sn : pl * cs);
     }
   }
+  for (; p < ts; p++)
+    out[p] = (T)0;
 }
 
 // phase[pt] = dv / sqrt(V) * exp(i kc . path)
@@ -298,64 +301,50 @@ __global__ __launch_bounds__(256) void k_phase(long npts, const double *__restri
   phase[i] = mk<T>((T)(scl * cs), (T)(scl * sn));
 }
 
-// One work-group (4 wavefronts) per (site, part of its points); lane b
-// of every wavefront accumulates the site's projectors for band b of the
-// chunk.  Tiles of TP points stage their projector values, phases and grid
-// indices in LDS with coalesced loads; each wavefront then takes every
-// fourth point of the tile, four points per step with their grid loads in
-// flight together, and reads the projector values as LDS broadcasts.  The
-// four wavefronts' sums are added in LDS at the end.
-template <typename T, int PMAX, bool FULL, int U>
-__device__ __forceinline__ void sphere_sum_block(const cplx<T> *__restrict__ g, int NB,
-                                                 const int *__restrict__ site_pt, const int *__restrict__ site_np,
-                                                 const long *__restrict__ tab_off, const int *__restrict__ pidx,
-                                                 const cplx<T> *__restrict__ phase, const T *__restrict__ table,
-                                                 int nparts, cplx<double> *__restrict__ partial, int streaming,
-                                                 int blk) {
+// Sphere sums of one (site, part of its points) by a work-group of 4
+// wavefronts, FP64; lane b of every wavefront accumulates the site's PM
+// table slots for band b of the chunk.  Tiles of TP points stage their
+// table rows, phases and grid indices in LDS with coalesced loads; each
+// wavefront then takes every fourth point of the tile, U points per step
+// with their grid loads in flight together, and reads the table values as
+// LDS broadcasts.  The four wavefronts' sums are added in LDS at the end;
+// partial[(blk * PMX + j) * NB + b].
+template <typename T, int PM, int U>
+__device__ __forceinline__ void sphere_sum_valu(const cplx<T> *__restrict__ g, int NB, int p0, int len,
+                                                const int *__restrict__ pidx, const cplx<T> *__restrict__ phase,
+                                                const T *__restrict__ tsite, int a, int e,
+                                                cplx<T> *__restrict__ partial, int streaming,
+                                                T *__restrict__ s_tab, cplx<T> *__restrict__ s_ph,
+                                                int *__restrict__ s_idx) {
   constexpr int TP = 64;
-  __shared__ __align__(16) T s_tab[TP * PMAX];
-  __shared__ cplx<T> s_ph[TP];
-  __shared__ int s_idx[TP];
-  const int s = blk / nparts, part = blk % nparts;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int p0 = site_pt[s], p1 = site_pt[s + 1];
-  const int np = FULL ? PMAX : site_np[s];  // FULL: every site has PMAX projectors
-  const int len = p1 - p0;
-  const int chunk = (len + nparts - 1) / nparts;
-  const int a = p0 + part * chunk;
-  const int e = min(p1, a + chunk);
   const bool active = lane < NB;
-  cplx<T> acc[PMAX];
+  cplx<T> acc[PM];
 #pragma unroll
-  for (int j = 0; j < PMAX; j++)
+  for (int j = 0; j < PM; j++)
     acc[j] = mk<T>(0, 0);
-  const T *tsite = table + tab_off[s];
   // a tile's table values, indices and phases: every load of a thread is
   // issued before any is written to LDS, so they are in flight together
-  constexpr int SL = (TP * PMAX + 255) / 256;
+  constexpr int SL = (TP * PM + 255) / 256;
   T tv[SL];
   int iv = 0;
   cplx<T> pv = mk<T>(0, 0);
-  auto fetch = [&](int f0) {
-    const int fn = min(TP, e - f0);
-    const T *tsrc = tsite + (long)(f0 - p0) * np;
-#pragma unroll
-    for (int u = 0; u < SL; u++) {
-      const int q = tid + u * 256;
-      tv[u] = q < fn * np ? tsrc[q] : (T)0;
-    }
-    if (tid < fn) {
-      iv = pidx[f0 + tid];
-      pv = phase[f0 + tid];
-    }
-  };
   for (int t0 = a; t0 < e; t0 += TP) {
     const int n = min(TP, e - t0);
-    fetch(t0);
+    const T *tsrc = tsite + (long)(t0 - p0) * PM;
 #pragma unroll
     for (int u = 0; u < SL; u++) {
       const int q = tid + u * 256;
-      if (q < n * np)
+      tv[u] = q < n * PM ? tsrc[q] : (T)0;
+    }
+    if (tid < n) {
+      iv = pidx[t0 + tid];
+      pv = phase[t0 + tid];
+    }
+#pragma unroll
+    for (int u = 0; u < SL; u++) {
+      const int q = tid + u * 256;
+      if (q < n * PM)
         s_tab[q] = tv[u];
     }
     if (tid < n) {
@@ -374,133 +363,295 @@ __device__ __forceinline__ void sphere_sum_block(const cplx<T> *__restrict__ g, 
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const cplx<T> xv = x[u] * s_ph[i + 4 * u];
-        const T *tp = s_tab + (i + 4 * u) * np;
+        const T *tp = s_tab + (i + 4 * u) * PM;
 #pragma unroll
-        for (int j = 0; j < PMAX; j++)
-          if (FULL || j < np) {
-            acc[j].x += tp[j] * xv.x;
-            acc[j].y += tp[j] * xv.y;
-          }
+        for (int j = 0; j < PM; j++) {
+          acc[j].x += tp[j] * xv.x;
+          acc[j].y += tp[j] * xv.y;
+        }
       }
     }
     for (; i < n; i += 4) {
       cplx<T> xv = active ? g[(long)s_idx[i] * NB + lane] : mk<T>(0, 0);
       xv = xv * s_ph[i];
-      const T *tp = s_tab + i * np;
+      const T *tp = s_tab + i * PM;
 #pragma unroll
-      for (int j = 0; j < PMAX; j++)
-        if (FULL || j < np) {
-          acc[j].x += tp[j] * xv.x;
-          acc[j].y += tp[j] * xv.y;
-        }
+      for (int j = 0; j < PM; j++) {
+        acc[j].x += tp[j] * xv.x;
+        acc[j].y += tp[j] * xv.y;
+      }
     }
     __syncthreads();
   }
-  // add the four wavefronts' sums, PMAX/2 projectors at a time through the
-  // table tile (TP * PMAX reals = 64 lanes x PMAX/2 complex)
+  // add the four wavefronts' sums, half of the slots at a time through the
+  // table tile (at least 64 lanes x (PM + 1) / 2 complex)
   cplx<T> *red = reinterpret_cast<cplx<T> *>(s_tab);
-  constexpr int JH = PMAX / 2;
+  constexpr int JH = (PM + 1) / 2;
   for (int w = 1; w < 4; w++) {
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       if (wave == w) {
 #pragma unroll
         for (int j = 0; j < JH; j++)
-          red[j * 64 + lane] = acc[h * JH + j];
+          if (h * JH + j < PM)
+            red[j * 64 + lane] = acc[h * JH + j];
       }
       __syncthreads();
       if (wave == 0) {
 #pragma unroll
         for (int j = 0; j < JH; j++)
-          acc[h * JH + j] = acc[h * JH + j] + red[j * 64 + lane];
+          if (h * JH + j < PM)
+            acc[h * JH + j] = acc[h * JH + j] + red[j * 64 + lane];
       }
       __syncthreads();
     }
   }
   if (wave == 0 && active) {
-    cplx<double> *o = partial + ((long)blk * NB + lane) * PMAX;
 #pragma unroll
-    for (int j = 0; j < PMAX; j++)
-      if (FULL || j < np)
-        o[j] = cvt<double>(acc[j]);
+    for (int j = 0; j < PM; j++)
+      partial[(long)j * NB + lane] = acc[j];
   }
 }
-template <typename T, int PMAX, bool FULL, int U>
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// MFMA operand: value `v` of the 64 table values a wavefront holds in one
+// register is broadcast to all 16 blocks of the 4x4x1 MFMA, value group
+// ABID (4 table slots of one point) against the lane's band.
+template <int ABID> __device__ __forceinline__ floatx4 mfma_quad(float tab, float x, floatx4 acc) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(tab, x, acc, 4, ABID, 0);
+}
+template <int I, int Q, int N = 0>
+__device__ __forceinline__ void mfma_point(const float (&tab)[Q], float xr, float xi, floatx4 (&ar)[Q],
+                                           floatx4 (&ai)[Q]) {
+  if constexpr (N < Q) {
+    constexpr int q = I * Q + N;  // quad q of the group's 16 points x Q quads
+    ar[N] = mfma_quad<q % 16>(tab[q / 16], xr, ar[N]);
+    ai[N] = mfma_quad<q % 16>(tab[q / 16], xi, ai[N]);
+    mfma_point<I, Q, N + 1>(tab, xr, xi, ar, ai);
+  }
+}
+template <int Q, int I = 0>
+__device__ __forceinline__ void mfma_group(const float (&tab)[Q], const cplx<float> (&x)[16], cplx<float> ph,
+                                           floatx4 (&ar)[Q], floatx4 (&ai)[Q]) {
+  if constexpr (I < 16) {
+    const float pr = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ph.x), I));
+    const float pi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ph.y), I));
+    const cplx<float> v = x[I] * mk<float>(pr, pi);
+    mfma_point<I, Q>(tab, v.x, v.y, ar, ai);
+    mfma_group<Q, I + 1>(tab, x, ph, ar, ai);
+  }
+}
+
+// The FP32 sphere sums on the matrix cores.  A wavefront takes groups of 16
+// points: the group's 16 x 4Q table values are Q coalesced register loads,
+// its 16 grid runs one 512-byte load each (lane = band), and every (point,
+// quad of table slots) is one 4x4x1 16-block MFMA per component, the table
+// quad broadcast to the 16 blocks (CBSZ = 4, ABID = the quad's place in the
+// register), the blocks' columns the 64 bands: no LDS, no barrier and no
+// projector guard in the loop, and 2Q MFMAs of 8 cycles per point where the
+// VALU form issued 8Q FMAs of 4.  Register v of accumulator q holds table
+// slot 4q + v of the lane's band.  A group's tail points repeat the last
+// point with phase 0 (the table values past the site's rows are other
+// sites' rows or the buffer's padding, both finite).
+template <int Q>
+__device__ __forceinline__ void sphere_sum_mfma(const cplx<float> *__restrict__ g, int NB, int p0, int len,
+                                                const int *__restrict__ pidx, const cplx<float> *__restrict__ phase,
+                                                const float *__restrict__ tsite, int a, int e,
+                                                cplx<float> *__restrict__ partial, int streaming,
+                                                float *__restrict__ red) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15;
+  const int band = lane < NB ? lane : 0;
+  floatx4 ar[Q], ai[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+    ar[q] = ai[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+  int idx = 0;
+  cplx<float> ph = mk<float>(0, 0);
+  float tab[Q];
+  auto fetch = [&](int g0) {
+    const int n = min(16, e - g0);
+    const int pt = g0 + (l16 < n ? l16 : n - 1);
+    idx = pidx[pt];
+    const cplx<float> v = phase[pt];
+    ph = l16 < n ? v : mk<float>(0, 0);
+    const float *ts = tsite + (long)(g0 - p0) * (4 * Q) + lane;
+#pragma unroll
+    for (int r = 0; r < Q; r++)
+      tab[r] = ts[r * 64];
+  };
+  int g0 = a + wave * 16;
+  if (g0 < e)
+    fetch(g0);
+  for (; g0 < e; g0 += 64) {
+    cplx<float> x[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const cplx<float> *gp = g + (long)__builtin_amdgcn_readlane(idx, i) * NB + band;
+      x[i] = streaming ? load_nt(gp) : *gp;
+    }
+    // the next group's table, phases and indices are loaded during this
+    // group's sums
+    float tc[Q];
+#pragma unroll
+    for (int r = 0; r < Q; r++)
+      tc[r] = tab[r];
+    const cplx<float> pc = ph;
+    if (g0 + 64 < e)
+      fetch(g0 + 64);
+    mfma_group<Q>(tc, x, pc, ar, ai);
+  }
+  // add the four wavefronts' sums: 2, 3 onto 0, 1, then 1 onto 0
+  auto put = [&](float *dst) {
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        dst[((4 * q + v) * 2) * 64 + lane] = ar[q][v];
+        dst[((4 * q + v) * 2 + 1) * 64 + lane] = ai[q][v];
+      }
+  };
+  auto add = [&](const float *src) {
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        ar[q][v] += src[((4 * q + v) * 2) * 64 + lane];
+        ai[q][v] += src[((4 * q + v) * 2 + 1) * 64 + lane];
+      }
+  };
+  for (int w = 3; w > 0; w--) {
+    if (wave == w)
+      put(red);
+    __syncthreads();
+    if (wave == 0)
+      add(red);
+    __syncthreads();
+  }
+  if (wave == 0 && lane < NB) {
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        partial[(long)(4 * q + v) * NB + lane] = mk<float>(ar[q][v], ai[q][v]);
+  }
+}
+
+// One work-group per (site, part of its points).  PM: the widest table row
+// of the plan; a site's own row width picks the body (uniform over the
+// work-group), so a plan that mixes species sums each at its own width.
+template <typename T, int PM, int U>
+__device__ __forceinline__ void sphere_sum_block(const cplx<T> *__restrict__ g, int NB,
+                                                 const int *__restrict__ site_pt, const int *__restrict__ site_np,
+                                                 const long *__restrict__ tab_off, const int *__restrict__ pidx,
+                                                 const cplx<T> *__restrict__ phase, const T *__restrict__ table,
+                                                 int nparts, cplx<T> *__restrict__ partial, int streaming, int blk) {
+  const int s = blk / nparts, part = blk % nparts;
+  const int p0 = site_pt[s], p1 = site_pt[s + 1];
+  const int len = p1 - p0;
+  const int chunk = (len + nparts - 1) / nparts;
+  const int a = p0 + part * chunk;
+  const int e = min(p1, a + chunk);
+  const T *tsite = table + tab_off[s];
+  const int ts = table_stride(site_np[s], sizeof(T) == 4);
+  cplx<T> *o = partial + (long)blk * PM * NB;
+  if constexpr (sizeof(T) == 4) {
+    __shared__ float red[PM * 2 * 64];
+#define PP_BODY(C)                                                                                         if constexpr (C <= PM) {                                                                                   if (ts == C) {                                                                                             sphere_sum_mfma<C / 4>(g, NB, p0, len, pidx, phase, tsite, a, e, o, streaming, red);                     return;                                                                                                }                                                                                                      }
+    PP_STRIDES_F32(PP_BODY)
+#undef PP_BODY
+  } else {
+    __shared__ __align__(16) T s_tab[64 * (PM + 1)];
+    __shared__ cplx<T> s_ph[64];
+    __shared__ int s_idx[64];
+#define PP_BODY(C)                                                                                         if constexpr (C <= PM) {                                                                                   if (ts == C) {                                                                                             sphere_sum_valu<T, C, U>(g, NB, p0, len, pidx, phase, tsite, a, e, o, streaming, s_tab, s_ph, s_idx);       return;                                                                                                }                                                                                                      }
+    PP_STRIDES_F64(PP_BODY)
+#undef PP_BODY
+  }
+}
+template <typename T, int PM, int U>
 __global__ __launch_bounds__(256) void k_sphere_sum(const cplx<T> *__restrict__ g, int NB,
                                                     const int *__restrict__ site_pt, const int *__restrict__ site_np,
                                                     const long *__restrict__ tab_off, const int *__restrict__ pidx,
                                                     const cplx<T> *__restrict__ phase, const T *__restrict__ table,
-                                                    int nparts, cplx<double> *__restrict__ partial, int streaming) {
-  sphere_sum_block<T, PMAX, FULL, U>(g, NB, site_pt, site_np, tab_off, pidx, phase, table, nparts, partial, streaming,
-                                     blockIdx.x);
+                                                    int nparts, cplx<T> *__restrict__ partial, int streaming) {
+  sphere_sum_block<T, PM, U>(g, NB, site_pt, site_np, tab_off, pidx, phase, table, nparts, partial, streaming,
+                             blockIdx.x);
 }
 // The sphere sums of a batch of work items (one per blockIdx.y), each with
 // its own chunk, plan and phases.
-template <typename T, int PMAX, bool FULL, int U>
+template <typename T, int PM, int U>
 __global__ __launch_bounds__(256) void k_sphere_sum_items(const ChunkItem *__restrict__ items, int NB, int streaming) {
   const ChunkItem &it = items[blockIdx.y];
   const int blk = blockIdx.x;
   if (blk >= it.nsites * it.nparts)
     return;
-  sphere_sum_block<T, PMAX, FULL, U>((const cplx<T> *)it.grid, NB, (const int *)it.site_pt,
-                                     (const int *)it.site_np, (const long *)it.tab_off, (const int *)it.pidx,
-                                     (const cplx<T> *)it.phase, (const T *)it.table, it.nparts,
-                                     (cplx<double> *)it.partial, streaming, blk);
+  sphere_sum_block<T, PM, U>((const cplx<T> *)it.grid, NB, (const int *)it.site_pt, (const int *)it.site_np,
+                             (const long *)it.tab_off, (const int *)it.pidx, (const cplx<T> *)it.phase,
+                             (const T *)it.table, it.nparts, (cplx<T> *)it.partial, streaming, blk);
 }
 
-// Sum the parts of every (site, band, projector) in FP64 and form the
-// complex projections from the real-harmonic sums: thread (s, b, j) with
-// m_j >= 0 writes slot j and, for m_j > 0, its partner slot j - 2 m_j.
-__device__ __forceinline__ void sphere_reduce_one(const cplx<double> *__restrict__ partial, int NB, int nbc,
-                                                  int PMAX, int nparts, int nsites, const int *__restrict__ site_np,
-                                                  const int *__restrict__ proj_off, const int *__restrict__ proj_m,
-                                                  long ptot, cplx<double> *__restrict__ out, long t) {
-  long total = (long)nsites * nbc * PMAX;
-  if (t >= total)
+// Sum the parts of every (site, slot, band) in FP64 and form the complex
+// projections from the real-harmonic sums.  One work-group per site and 16
+// bands: the part sums are read with the bands on consecutive lanes (as
+// the sum kernels wrote them) into an LDS tile, and the projections written
+// with the slots on consecutive lanes (as the output rows hold them), so
+// both sides move whole lines.
+constexpr int RED_NB = 16;
+template <typename T>
+__device__ __forceinline__ void sphere_reduce_block(const cplx<T> *__restrict__ partial, int NB, int nbc, int PM,
+                                                    int nparts, int nsites, const int *__restrict__ site_np,
+                                                    const int *__restrict__ proj_off, const int *__restrict__ proj_m,
+                                                    long ptot, cplx<double> *__restrict__ out, int blk) {
+  __shared__ cplx<double> tile[64][RED_NB + 1];
+  const int ng = (nbc + RED_NB - 1) / RED_NB;
+  const int s = blk / ng, b0 = (blk % ng) * RED_NB;
+  if (s >= nsites)
     return;
-  int j = (int)(t % PMAX);
-  long r = t / PMAX;
-  int b = (int)(r % nbc);
-  int s = (int)(r / nbc);
-  if (j >= site_np[s])
-    return;
-  const int m = proj_m[proj_off[s] + j];
-  if (m < 0)
-    return;
-  cplx<double> c = mk<double>(0, 0), sn = mk<double>(0, 0);
-  const cplx<double> *ps = partial + ((long)s * nparts * NB + b) * PMAX;
-  // the partner slot of m > 0 (m = 0 reads its own slot again and leaves
-  // the sum unused), loaded without a branch and unrolled, so that several
-  // parts' loads are in flight together; the sums keep their order
-  const int jo = m > 0 ? j - 2 * m : j;
+  const int np = site_np[s], po = proj_off[s];
+  const int bl = threadIdx.x % RED_NB, j0 = threadIdx.x / RED_NB;
+  if (b0 + bl < nbc)
+    for (int j = j0; j < np; j += 256 / RED_NB) {
+      cplx<double> c = mk<double>(0, 0);
+      const cplx<T> *ps = partial + ((long)s * nparts * PM + j) * NB + b0 + bl;
 #pragma unroll 4
-  for (int q = 0; q < nparts; q++) {
-    c = c + ps[(long)q * NB * PMAX + j];
-    sn = sn + ps[(long)q * NB * PMAX + jo];
-  }
-  cplx<double> *o = out + (long)b * ptot + proj_off[s];
-  if (m == 0) {
-    o[j] = c;
-  } else {
-    const double sg = (m & 1) ? -1.0 : 1.0;
-    o[j] = mk<double>(c.x + sn.y, c.y - sn.x);
-    o[j - 2 * m] = mk<double>(sg * (c.x - sn.y), sg * (c.y + sn.x));
+      for (int q = 0; q < nparts; q++)
+        c = c + cvt<double>(ps[(long)q * PM * NB]);
+      tile[j][bl] = c;
+    }
+  __syncthreads();
+  for (int t = threadIdx.x; t < np * RED_NB; t += 256) {
+    const int b = t / np, j = t - b * np;
+    if (b0 + b >= nbc)
+      break;
+    const int m = proj_m[po + j];
+    const cplx<double> own = tile[j][b];
+    cplx<double> r = own;
+    if (m > 0) {  // s_(l,m) - i s_(l,-m)
+      const cplx<double> sn = tile[j - 2 * m][b];
+      r = mk<double>(own.x + sn.y, own.y - sn.x);
+    } else if (m < 0) {  // (-1)^m (s_(l,m) + i s_(l,-m))
+      const cplx<double> c = tile[j - 2 * m][b];
+      const double sg = (m & 1) ? -1.0 : 1.0;
+      r = mk<double>(sg * (c.x - own.y), sg * (c.y + own.x));
+    }
+    out[(long)(b0 + b) * ptot + po + j] = r;
   }
 }
-__global__ __launch_bounds__(256) void k_sphere_reduce(const cplx<double> *__restrict__ partial, int NB, int nbc,
-                                                       int PMAX, int nparts, int nsites,
-                                                       const int *__restrict__ site_np,
+template <typename T>
+__global__ __launch_bounds__(256) void k_sphere_reduce(const cplx<T> *__restrict__ partial, int NB, int nbc, int PM,
+                                                       int nparts, int nsites, const int *__restrict__ site_np,
                                                        const int *__restrict__ proj_off,
                                                        const int *__restrict__ proj_m, long ptot,
                                                        cplx<double> *__restrict__ out) {
-  sphere_reduce_one(partial, NB, nbc, PMAX, nparts, nsites, site_np, proj_off, proj_m, ptot, out,
-                    (long)blockIdx.x * 256 + threadIdx.x);
+  sphere_reduce_block<T>(partial, NB, nbc, PM, nparts, nsites, site_np, proj_off, proj_m, ptot, out, blockIdx.x);
 }
-__global__ __launch_bounds__(256) void k_sphere_reduce_items(const ChunkItem *__restrict__ items, int NB, int PMAX) {
+template <typename T>
+__global__ __launch_bounds__(256) void k_sphere_reduce_items(const ChunkItem *__restrict__ items, int NB, int PM) {
   const ChunkItem &it = items[blockIdx.y];
-  sphere_reduce_one((const cplx<double> *)it.partial, NB, it.nbc, PMAX, it.nparts, it.nsites,
-                    (const int *)it.site_np, (const int *)it.proj_off, (const int *)it.proj_m, it.ptot,
-                    (cplx<double> *)it.out, (long)blockIdx.x * 256 + threadIdx.x);
+  sphere_reduce_block<T>((const cplx<T> *)it.partial, NB, it.nbc, PM, it.nparts, it.nsites, (const int *)it.site_np,
+                         (const int *)it.proj_off, (const int *)it.proj_m, it.ptot, (cplx<double> *)it.out,
+                         blockIdx.x);
 }
 
 // Coefficients of the real-harmonic table slots for the expansion
@@ -555,7 +706,7 @@ __global__ __launch_bounds__(256) void k_sphere_expand(cplx<T> *__restrict__ g, 
   const int s = blockIdx.x / nparts, part = blockIdx.x % nparts;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int p0 = site_pt[s], len = site_pt[s + 1] - p0;
-  const int np = site_np[s];
+  const int np = site_np[s], ts = table_stride(np, sizeof(T) == 4);
   const int chunk = (len + nparts - 1) / nparts;
   const int a = p0 + part * chunk, e = min(p0 + len, a + chunk);
   if (lane >= nbc)
@@ -566,7 +717,7 @@ __global__ __launch_bounds__(256) void k_sphere_expand(cplx<T> *__restrict__ g, 
     q[j] = j < np ? Q[((long)s * PMAX + j) * NB + lane] : mk<T>(0, 0);
   const T *tsite = table + tab_off[s];
   for (int i = a + wave; i < e; i += 4) {
-    const T *tp = tsite + (long)(i - p0) * np;
+    const T *tp = tsite + (long)(i - p0) * ts;
     cplx<T> v = mk<T>(0, 0);
 #pragma unroll
     for (int j = 0; j < PMAX; j++)
@@ -676,8 +827,6 @@ static int sphere_build(pp_sphere *sp) {
     sp->proj_off[s + 1] = sp->proj_off[s] + np;
     if (np > sp->pmax)
       sp->pmax = np;
-    if (s == 0 || np < sp->pmin)
-      sp->pmin = np;
   }
   sp->ptot = sp->proj_off[ns];
   PP_REQUIRE(sp->pmax <= 64, PP_ERR_UNSUPPORTED, "more than 64 projectors on one site");
@@ -717,7 +866,7 @@ static int sphere_build(pp_sphere *sp) {
     sp->site_pt_h[s + 1] = sp->site_pt_h[s] + counts[s];
     sp->seg_off_h[s + 1] = sp->seg_off_h[s] + counts[ns + s];
     tab_off[s] = to;
-    to += (long)counts[s] * sp->nproj_site[s];
+    to += (long)counts[s] * table_stride(sp->nproj_site[s], sp->precision != PP_FP64);
     if (counts[s] > maxcount)
       maxcount = counts[s];
   }
@@ -730,7 +879,10 @@ static int sphere_build(pp_sphere *sp) {
   PP_TRY(sp->d_proj_off.ensure(sizeof(int) * (ns + 1)));
   PP_TRY(sp->d_pidx.ensure(sizeof(int) * std::max<long>(1, sp->npts)));
   PP_TRY(sp->d_path.ensure(sizeof(double) * 3 * std::max<long>(1, sp->npts)));
-  PP_TRY(sp->d_table.ensure(csz * std::max<long>(1, to)));
+  // the FP32 sums read whole groups of 16 rows: padding past the last row
+  const long tpad = 16 * 64;
+  PP_TRY(sp->d_table.ensure(csz * (to + tpad)));
+  PP_TRY(zero_async(ctx, (char *)sp->d_table.p + csz * to, csz * tpad));
   PP_TRY(sp->d_seg_off.ensure(sizeof(int) * (ns + 1)));
   PP_TRY(sp->d_seg.ensure(sizeof(int4) * std::max<long>(1, sp->nseg)));
   PP_TRY(sp->d_segline.ensure(sizeof(int) * std::max<long>(1, sp->nseg)));
@@ -787,31 +939,24 @@ static int sphere_build(pp_sphere *sp) {
   return ctx->tune_fused ? fused_plan(sp, geo) : PP_OK;
 }
 
-template <typename T, int PMAX>
+// Sum kernel of a plan whose widest table row is PM (one of the strides of
+// table_stride); the FP32 form has no unroll variants.
+template <typename T, int PM>
 static void launch_sum(pp_ctx *ctx, pp_sphere *sp, const cplx<T> *grid, int NB, const cplx<T> *phase, int nparts,
-                       cplx<double> *partial) {
-#define PP_SS(FULL, U)                                                                                            \
-  hipLaunchKernelGGL((k_sphere_sum<T, PMAX, FULL, U>), dim3(sp->nsites * nparts), dim3(256), 0, ctx->stream, grid,  \
-                     NB, (const int *)sp->d_site_pt.p, (const int *)sp->d_site_np.p, (const long *)sp->d_tab_off.p, \
-                     (const int *)sp->d_pidx.p, phase, (const T *)sp->d_table.p, nparts, partial,             \
-                     ctx->tune_sphere_nt)
-  const bool u8 = ctx->tune_sphere_unroll == 8;
-  if (sp->pmin == PMAX) {
-    if (u8)
-      PP_SS(true, 8);
-    else
-      PP_SS(true, 4);
-  } else {
-    if (u8)
-      PP_SS(false, 8);
-    else
-      PP_SS(false, 4);
-  }
+                       cplx<T> *partial) {
+#define PP_SS(U)                                                                                                    \
+  hipLaunchKernelGGL((k_sphere_sum<T, PM, U>), dim3(sp->nsites * nparts), dim3(256), 0, ctx->stream, grid, NB,     \
+                     (const int *)sp->d_site_pt.p, (const int *)sp->d_site_np.p, (const long *)sp->d_tab_off.p,    \
+                     (const int *)sp->d_pidx.p, phase, (const T *)sp->d_table.p, nparts, partial, ctx->tune_sphere_nt)
+  if (sizeof(T) == 4 || ctx->tune_sphere_unroll == 8)
+    PP_SS(8);
+  else
+    PP_SS(4);
 #undef PP_SS
 }
 
 int sphere_parts_of(pp_ctx *ctx, pp_sphere *sp);
-int sphere_pm_of(pp_sphere *sp, bool *full);
+int sphere_pm_of(pp_sphere *sp);
 
 template <typename T>
 int sphere_sums(pp_ctx *ctx, pp_sphere *sp, const cplx<T> *grid, int NB, int nbc, const cplx<T> *phase,
@@ -819,60 +964,47 @@ int sphere_sums(pp_ctx *ctx, pp_sphere *sp, const cplx<T> *grid, int NB, int nbc
   if (sp->nsites == 0 || nbc == 0)
     return PP_OK;
   const int nparts = sphere_parts_of(ctx, sp);
-  const int PM = sphere_pm_of(sp, nullptr);
+  const int PM = sphere_pm_of(sp);
   DevBuf &pbuf = ctx->slot ? ctx->partial2 : ctx->partial;
-  PP_TRY(pbuf.ensure(sizeof(cplx<double>) * (size_t)sp->nsites * nparts * NB * PM));
-  cplx<double> *partial = (cplx<double> *)pbuf.p;
+  PP_TRY(pbuf.ensure(sizeof(cplx<T>) * (size_t)sp->nsites * nparts * NB * PM));
+  cplx<T> *partial = (cplx<T> *)pbuf.p;
   hipEvent_t ev;
   tbegin(ctx, K_SPHERE_SUM, &ev);
-  switch (PM) {
-  case 8:
-    launch_sum<T, 8>(ctx, sp, grid, NB, phase, nparts, partial);
+#define PP_SUM(P)                                                     \
+  case P:                                                             \
+    launch_sum<T, P>(ctx, sp, grid, NB, phase, nparts, partial);      \
     break;
-  case 18:
-    launch_sum<T, 18>(ctx, sp, grid, NB, phase, nparts, partial);
-    break;
-  case 32:
-    launch_sum<T, 32>(ctx, sp, grid, NB, phase, nparts, partial);
-    break;
-  default:
-    launch_sum<T, 64>(ctx, sp, grid, NB, phase, nparts, partial);
+  if constexpr (sizeof(T) == 4) {
+    switch (PM) { PP_STRIDES_F32(PP_SUM) }
+  } else {
+    switch (PM) { PP_STRIDES_F64(PP_SUM) }
   }
+#undef PP_SUM
   tend(ctx, K_SPHERE_SUM, ev);
   PP_CHECK_HIP(hipGetLastError());
-  long total = (long)sp->nsites * nbc * PM;
+  const long nblk = (long)sp->nsites * ((nbc + RED_NB - 1) / RED_NB);
   tbegin(ctx, K_SPHERE_REDUCE, &ev);
-  hipLaunchKernelGGL(k_sphere_reduce, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, partial, NB,
-                     nbc, PM, nparts, sp->nsites, (const int *)sp->d_site_np.p, (const int *)sp->d_proj_off.p,
+  hipLaunchKernelGGL(k_sphere_reduce<T>, dim3((unsigned)nblk), dim3(256), 0, ctx->stream, partial, NB, nbc, PM, nparts,
+                     sp->nsites, (const int *)sp->d_site_np.p, (const int *)sp->d_proj_off.p,
                      (const int *)sp->d_proj_m.p, ptot, out);
   tend(ctx, K_SPHERE_REDUCE, ev);
   PP_CHECK_HIP(hipGetLastError());
   return PP_OK;
 }
 
-// Sphere-sum parts per site of a plan (the tuning value, else about eight
-// four-wave work-groups per CU).
+// Sphere-sum parts per site of a plan: the tuning value, else enough for
+// about 2048 work-groups (eight per CU), of at least 64 points each (one
+// group of 16 per wavefront): a cell of 8 sites of 270 points runs 32
+// work-groups of one group per wavefront instead of 8 of four.
 int sphere_parts_of(pp_ctx *ctx, pp_sphere *sp) {
-  int nparts = ctx->tune_sphere_parts;
-  if (nparts <= 0) {
-    nparts = (2048 + sp->nsites - 1) / std::max(1, sp->nsites);
-    long avg = sp->npts / std::max(1, sp->nsites);
-    int maxp = (int)std::max<long>(1, avg / 256);
-    if (nparts > maxp)
-      nparts = maxp;
-    if (nparts < 1)
-      nparts = 1;
-  }
-  return nparts;
+  if (ctx->tune_sphere_parts > 0)
+    return ctx->tune_sphere_parts;
+  const int ns = std::max(1, sp->nsites);
+  const long most = std::max<long>(1, sp->npts / ns / 64);
+  return (int)std::min<long>((2048 + ns - 1) / ns, most);
 }
-// Projector slots per site the sum kernels hold for a plan (8, 18, 32, 64)
-// and whether every site has exactly that many.
-int sphere_pm_of(pp_sphere *sp, bool *full) {
-  const int PM = sp->pmax <= 8 ? 8 : sp->pmax <= 18 ? 18 : sp->pmax <= 32 ? 32 : 64;
-  if (full)
-    *full = sp->pmin == PM;
-  return PM;
-}
+// Widest table row of a plan: the sum kernel that serves it.
+int sphere_pm_of(pp_sphere *sp) { return table_stride(sp->pmax, sp->precision != PP_FP64); }
 // The plan's part of a work item.
 void sphere_item_fields(pp_ctx *ctx, pp_sphere *sp, ChunkItem &it) {
   it.site_pt = (const PP_G int *)sp->d_site_pt.p;
@@ -887,57 +1019,45 @@ void sphere_item_fields(pp_ctx *ctx, pp_sphere *sp, ChunkItem &it) {
 }
 
 // Sphere sums and their reduction for a batch of work items: one launch
-// each.  PM and full as sphere_pm_of for every item's plan; maxblk bounds
-// nsites * nparts and maxred nsites * nbc * PM over the items.
+// each.  PM: the largest sphere_pm_of of the items' plans; maxblk and
+// maxred bound the work-groups of the sums (nsites * nparts) and of the
+// reduction (nsites * band groups of RED_NB) over the items.
 template <typename T>
-int sphere_sums_items(pp_ctx *ctx, const ChunkItem *items, int nitems, int NB, int PM, bool full, long maxblk,
-                      long maxred) {
+int sphere_sums_items(pp_ctx *ctx, const ChunkItem *items, int nitems, int NB, int PM, long maxblk, long maxred) {
   if (nitems == 0 || maxblk == 0)
     return PP_OK;
   hipEvent_t ev;
   tbegin(ctx, K_SPHERE_SUM, &ev);
   dim3 grd((unsigned)maxblk, (unsigned)nitems);
-  const bool u8 = ctx->tune_sphere_unroll == 8;
-#define PP_SI(P, F, U)                                                                                           \
-  hipLaunchKernelGGL((k_sphere_sum_items<T, P, F, U>), grd, dim3(256), 0, ctx->stream, items, NB, ctx->tune_sphere_nt)
-#define PP_SIP(P)                                                                                                \
-  do {                                                                                                           \
-    if (full) {                                                                                                  \
-      if (u8)                                                                                                    \
-        PP_SI(P, true, 8);                                                                                       \
-      else                                                                                                       \
-        PP_SI(P, true, 4);                                                                                       \
-    } else if (u8)                                                                                               \
-      PP_SI(P, false, 8);                                                                                        \
-    else                                                                                                         \
-      PP_SI(P, false, 4);                                                                                        \
-  } while (0)
-  switch (PM) {
-  case 8:
-    PP_SIP(8);
+  const bool u8 = sizeof(T) == 4 || ctx->tune_sphere_unroll == 8;
+#define PP_SI(P)                                                                                                   \
+  case P:                                                                                                          \
+    if (u8)                                                                                                        \
+      hipLaunchKernelGGL((k_sphere_sum_items<T, P, 8>), grd, dim3(256), 0, ctx->stream, items, NB,                 \
+                         ctx->tune_sphere_nt);                                                                     \
+    else                                                                                                           \
+      hipLaunchKernelGGL((k_sphere_sum_items<T, P, 4>), grd, dim3(256), 0, ctx->stream, items, NB,                 \
+                         ctx->tune_sphere_nt);                                                                     \
     break;
-  case 18:
-    PP_SIP(18);
-    break;
-  case 32:
-    PP_SIP(32);
-    break;
-  default:
-    PP_SIP(64);
+  if constexpr (sizeof(T) == 4) {
+    switch (PM) { PP_STRIDES_F32(PP_SI) }
+  } else {
+    switch (PM) { PP_STRIDES_F64(PP_SI) }
   }
-#undef PP_SIP
 #undef PP_SI
   tend(ctx, K_SPHERE_SUM, ev);
   PP_CHECK_HIP(hipGetLastError());
   tbegin(ctx, K_SPHERE_REDUCE, &ev);
-  hipLaunchKernelGGL(k_sphere_reduce_items, dim3((unsigned)((maxred + 255) / 256), (unsigned)nitems), dim3(256), 0,
-                     ctx->stream, items, NB, PM);
+  hipLaunchKernelGGL(k_sphere_reduce_items<T>, dim3((unsigned)maxred, (unsigned)nitems), dim3(256), 0, ctx->stream,
+                     items, NB, PM);
   tend(ctx, K_SPHERE_REDUCE, ev);
   PP_CHECK_HIP(hipGetLastError());
   return PP_OK;
 }
-template int sphere_sums_items<double>(pp_ctx *, const ChunkItem *, int, int, int, bool, long, long);
-template int sphere_sums_items<float>(pp_ctx *, const ChunkItem *, int, int, int, bool, long, long);
+template int sphere_sums_items<double>(pp_ctx *, const ChunkItem *, int, int, int, long, long);
+template int sphere_sums_items<float>(pp_ctx *, const ChunkItem *, int, int, int, long, long);
+// Reduction work-groups of an item.
+long sphere_reduce_blocks(int nsites, int nbc) { return (long)nsites * ((nbc + RED_NB - 1) / RED_NB); }
 
 // phase[pt] = dv / sqrt(V) e^{i k.path} (sphere sums) or, with expand,
 // e^{-i k.path} (the augmentation functions of projector.c:276-330)

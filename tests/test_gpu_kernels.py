@@ -154,6 +154,37 @@ def test_projections_two_species(ctx):
         assert err < tol
 
 
+@pytest.mark.parametrize("ls", [(0,), (0, 1), (0, 0, 1), (0, 1, 2), (0, 0, 1, 1, 2), (0, 1, 2, 3), (0, 0, 1, 1, 2, 2),
+                                (0, 1, 2, 3, 1, 1, 0), (0, 0, 1, 1, 2, 2, 3, 3), (0, 1, 2, 3) * 3, (0, 1, 2, 3) * 4])
+@pytest.mark.parametrize("nb", [3, 67])
+def test_projections_row_widths(ctx, ls, nb):
+    """Sphere sums at every table row width the kernels are compiled for (1
+    to 64 projectors a site, rows padded to the next width), beside a
+    species of 4 projectors in the same plan; the second chunk of 67 bands
+    holds 3 lanes; the part count leaves parts with less than one group of
+    16 points and parts with none.  FP64 sums a site's ~300 terms in FP64;
+    FP32 sums them in FP32 after an FP32 transform (as test_projections_fp32)."""
+    from pawpyseed_amd.core import batched as B
+    wl = synthetic.tiny_config(encut=120.0, fftg=(20, 18, 24), nband=nb, kpts=[[0.25, -0.25, 0.1]])
+    sp = synthetic.make_species(list(ls), [1.5 + 0.2 * i for i in range(len(ls))], 1.15)
+    species, labels = [wl.species, sp], (np.arange(len(wl.frac_S)) % 2).astype(np.int32)
+    Gs, Cs = wl.ensure_gvecs(), wl.coefficients("S", nband=nb)
+    T = orc.site_tables(wl.lattice, wl.fftg, wl.frac_S, species, labels)
+    want = orc.setup_projections(wl.lattice, wl.fftg, wl.kpts, Gs, Cs, T)
+    Cd, Gd, gofs, nw = device_inputs(Gs, Cs)
+    for precision, tol in (("fp64", 1e-12), ("fp32", 1e-5)):
+        plan = B.SpherePlan(ctx, wl.lattice, wl.fftg, wl.frac_S, labels, species, precision)
+        for parts in (0, 1, 29):
+            ctx.set_param("sphere_parts", parts)
+            out = torch.full((1, nb, plan.ptot), np.nan, dtype=torch.complex128, device="cuda")
+            torch.cuda.synchronize()
+            B.setup_projections(ctx, plan, wl.kpts, gofs, Gd, Cd, out, precision)
+            err = normwise(out.cpu().numpy(), want)
+            assert err < tol, (precision, parts, err)
+        ctx.set_param("sphere_parts", 0)
+        plan.close()
+
+
 def test_projections_fp64_cfg0(ctx):
     """64-site cell of the 400 eV / 60^3 workload, Gamma, 16 bands."""
     wl = synthetic.config0()
