@@ -158,7 +158,7 @@ struct pp_ctx {
   hipEvent_t gemm_done[2] = {nullptr, nullptr};  // GEMM of a partials slot finished
   hipEvent_t red_done[2] = {nullptr, nullptr};   // reduction of a partials slot finished
   hipEvent_t split_done[2] = {nullptr, nullptr}; // operand split into a plane buffer finished
-  pp::DevBuf aug_ws;    // gathered / dO-applied projections
+  pp::DevBuf aug_ws;    // dO-applied projections
   // Index tables and dO coefficients of the last augmentation call, on the
   // device and (as the content key) on the host; uploads of changed tables
   // go through a pinned staging buffer.
@@ -275,6 +275,17 @@ struct TuneCand {
 int autotune_core(pp_ctx *ctx, const std::vector<TuneCand> &cands, const std::function<int()> &run, int repeats,
                   char *report, int report_len);
 
+// The batches of one launch of the FP64 GEMM: operand indices and K of each.
+struct GemmBatch {
+  static constexpr int MAX = 16;
+  int n = 0;
+  int a[MAX], b[MAX], k[MAX];
+};
+// zgemm_nt in FP64, with an optional device column map acol of A (FP64
+// operands): conj(A[.][acol[k]]) in the place of conj(A[.][k]).
+int zgemm64_nt(pp_ctx *ctx, int M, int N, int K, int atype, const void *A, long lda, long sA, const int *acol,
+               int btype, const void *B, long ldb, long sB, cplx<double> *C, long ldc, long sC, int nbatch,
+               const int *amap, const int *bmap, const int *klen, bool accumulate);
 // Complex GEMM out[b][m][n] (+)= sum_k conj(A[b][m][k]) B[b][n][k] (pp_gemm.hip).
 // type codes: 0 = c128, 1 = c64.  Batch strides in elements; amap/bmap
 // optional per-batch index remaps (host arrays of length nbatch).

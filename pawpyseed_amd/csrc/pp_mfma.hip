@@ -81,13 +81,19 @@ __device__ __forceinline__ void load8(const float *__restrict__ P, long ld, int 
 
 // FOLD: FP32 sums folded into FP64 every 512 complex terms, FP64 partial
 // sums out; otherwise a chunk's FP32 sums are its (FP32) partial sums.
+//
+// The four k indices of an MFMA are four consecutive complex terms and a
+// lane holds its term's whole complex value: Re takes (ar, br) and (ai, bi),
+// Im (ar, bi) and (-ai, br), one 8-byte LDS read per operand value for all
+// four products (with K taken as the 2K interleaved reals, Im needed the
+// neighbour's value as well: 12 4-byte reads where these are 4 of 8).
 template <bool VEC, bool FOLD>
 __global__ __launch_bounds__(256) void k_cgemm_f32(int M, int N, int kchunk, int K, int nsplit,
                                                    const float *__restrict__ A, long lda,
                                                    const float *__restrict__ B, long ldb, void *__restrict__ Cv,
                                                    long ldc, long sSplit) {
-  __shared__ float As[64][36];
-  __shared__ float Bs[64][36];
+  __shared__ __align__(16) cplx<float> As[64][18];  // 18: 16 rows x 2 terms of a read fall on distinct banks
+  __shared__ __align__(16) cplx<float> Bs[64][18];
   const int tilesN = (N + 63) / 64;
   int split, tile;
   if (!gemm_block(((M + 63) / 64) * tilesN, nsplit, split, tile))
@@ -124,9 +130,11 @@ __global__ __launch_bounds__(256) void k_cgemm_f32(int M, int N, int kchunk, int
   }
   for (int kb = k0; kb < k1; kb += 16) {
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-      As[lrow][part * 8 + c] = va[c];
-      Bs[lrow][part * 8 + c] = vb[c];
+    for (int c = 0; c < 4; c += 2) {
+      *reinterpret_cast<floatx4 *>(&As[lrow][part * 4 + c]) =
+          floatx4{va[2 * c], va[2 * c + 1], va[2 * c + 2], va[2 * c + 3]};
+      *reinterpret_cast<floatx4 *>(&Bs[lrow][part * 4 + c]) =
+          floatx4{vb[2 * c], vb[2 * c + 1], vb[2 * c + 2], vb[2 * c + 3]};
     }
     __syncthreads();
     if (kb + 16 < k1) {
@@ -134,25 +142,28 @@ __global__ __launch_bounds__(256) void k_cgemm_f32(int M, int N, int kchunk, int
       load8<VEC>(B, ldb, tn * 64 + lrow, N, kb + 16 + part * 4, k1, vb);
     }
     const int sub = lane & 15, kq = lane >> 4;
-    // B'' = (b_im, -b_re): the neighbour k ^ 1 (k even for re, odd for im)
-    // with its sign bit flipped for odd k -- one LDS read and no branch
-    // (a conditional choice of the two reads compiles to a divergent branch)
-    const unsigned sgn = (unsigned)(kq & 1) << 31;
 #pragma unroll
-    for (int kk = 0; kk < 32; kk += 4) {
-      const int kr = kk + kq;
-      const float a0 = As[wm * 32 + sub][kr];
-      const float a1 = As[wm * 32 + 16 + sub][kr];
+    for (int kk = 0; kk < 16; kk += 4) {
+      cplx<float> a[2], b[2];
 #pragma unroll
-      for (int nj = 0; nj < 2; nj++) {
-        const int col = wn * 32 + nj * 16 + sub;
-        const float b = Bs[col][kr];
-        const float b2 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, Bs[col][kr ^ 1]) ^ sgn);
-        cr[0][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b, cr[0][nj], 0, 0, 0);
-        ci[0][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b2, ci[0][nj], 0, 0, 0);
-        cr[1][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b, cr[1][nj], 0, 0, 0);
-        ci[1][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b2, ci[1][nj], 0, 0, 0);
+      for (int i = 0; i < 2; i++) {
+        a[i] = As[wm * 32 + i * 16 + sub][kk + kq];
+        b[i] = Bs[wn * 32 + i * 16 + sub][kk + kq];
       }
+#pragma unroll
+      for (int mi = 0; mi < 2; mi++)
+#pragma unroll
+        for (int nj = 0; nj < 2; nj++) {
+          cr[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mi].x, b[nj].x, cr[mi][nj], 0, 0, 0);
+          ci[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mi].x, b[nj].y, ci[mi][nj], 0, 0, 0);
+        }
+#pragma unroll
+      for (int mi = 0; mi < 2; mi++)
+#pragma unroll
+        for (int nj = 0; nj < 2; nj++) {
+          cr[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mi].y, b[nj].y, cr[mi][nj], 0, 0, 0);
+          ci[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(-a[mi].y, b[nj].x, ci[mi][nj], 0, 0, 0);
+        }
     }
     __syncthreads();
     // bound the FP32 accumulation length: fold into FP64 every 512 terms
@@ -568,9 +579,9 @@ __global__ __launch_bounds__(128 * TMW) __attribute__((amdgpu_waves_per_eu(WPE, 
   }
 }
 
-int splitk_count(int precision, int M, int N, int K, int tune);
+int splitk_count(int precision, int M, int N, int K, int tune, int nbatch, bool c128);
 int launch_splitk_reduce(hipStream_t st, int M, int N, int nsplit, const void *P, bool fp32_partials,
-                         cplx<double> *C, long ldc, bool accumulate);
+                         cplx<double> *C, long ldc, bool accumulate, int nbatch, long sP, long sC);
 
 // K chunk (complex terms) of an FP32 GEMM split nsplit ways: a multiple
 // of the kernel's k-step; nsplit is reduced to the chunks needed.
@@ -740,7 +751,7 @@ int gemm_fp32_mfma(pp_ctx *ctx, int precision, int M, int N, int K, const void *
   if (planes) {
     plane_layout(precision, M, N, K, cvt, ldp, nt, nsplit, wsb);
   } else {
-    nsplit = splitk_count(precision, M, N, K, ctx->tune_splitk);
+    nsplit = splitk_count(precision, M, N, K, ctx->tune_splitk, 1, false);
     kchunk = cgemm_chunk(precision, K, nsplit);
   }
   const bool fp32p = planes || fp32_partials_for(precision, kchunk);
@@ -775,7 +786,7 @@ int gemm_fp32_mfma(pp_ctx *ctx, int precision, int M, int N, int K, const void *
     ctx->stream = ctx->aux;
   }
   tbegin(ctx, K_GEMM_REDUCE, &ev);
-  st = launch_splitk_reduce(ctx->stream, M, N, nsplit, P, fp32p, C, ldc, accumulate);
+  st = launch_splitk_reduce(ctx->stream, M, N, nsplit, P, fp32p, C, ldc, accumulate, 1, 0, 0);
   tend(ctx, K_GEMM_REDUCE, ev);
   ctx->stream = main;
   PP_TRY(st);
@@ -871,7 +882,7 @@ int plane_gemm_pipeline(pp_ctx *ctx, int precision, int M, int N, int K, const v
     PP_CHECK_HIP(hipStreamWaitEvent(aux, ctx->gemm_done[slot], 0));
     ctx->stream = aux;
     tbegin(ctx, K_GEMM_REDUCE, &ev);
-    st = launch_splitk_reduce(aux, M, N, nsplit, parts[slot], true, C + (size_t)b * sC, ldc, accumulate);
+    st = launch_splitk_reduce(aux, M, N, nsplit, parts[slot], true, C + (size_t)b * sC, ldc, accumulate, 1, 0, 0);
     tend(ctx, K_GEMM_REDUCE, ev);
     ctx->stream = main;
     PP_TRY(st);

@@ -14,21 +14,26 @@
 // partial sums there; the reduction reads only what the same call wrote.
 // Calls that overlap in time on one GPU (two streams, two threads) race on
 // the array and must be serialised by the caller.
+#include <algorithm>
 #include <mutex>
 
 #include "pp_internal.h"
 
 namespace pp {
 
-int splitk_count(int precision, int M, int N, int K, int tune);
+int splitk_count(int precision, int M, int N, int K, int tune, int nbatch, bool c128);
 int cgemm_chunk(int precision, int K, int &nsplit);
 int launch_cgemm32(hipStream_t st, int precision, int M, int N, int K, const void *A, long lda, const void *B,
                    long ldb, void *P, long ldp, long sSplit, int nsplit, int kchunk);
 bool fp32_partials_for(int precision, int kchunk);
-int launch_zgemm64(hipStream_t st, bool valu, int M, int N, int K, int atype, const void *A, long lda, int btype,
-                   const void *B, long ldb, cplx<double> *dst, long dld, long sSplit, int nsplit, int kchunk);
+int launch_zgemm64(hipStream_t st, int M, int N, const GemmBatch &gb, int atype, const void *A, long lda, long sA,
+                   const int *acol, int btype, const void *B, long ldb, long sB, cplx<double> *dst, long dld,
+                   long sSplit, long sBatch, int nsplit, int kchunk, bool accumulate);
+void zgemm64_split(int M, int N, const GemmBatch &gb, int tune, bool c128, int &nsplit, int &kchunk);
+int launch_zgemm64_valu(hipStream_t st, int M, int N, int K, int atype, const void *A, long lda, int btype,
+                        const void *B, long ldb, cplx<double> *dst, long dld, long sSplit, int nsplit, int kchunk);
 int launch_splitk_reduce(hipStream_t st, int M, int N, int nsplit, const void *P, bool fp32_partials,
-                         cplx<double> *C, long ldc, bool accumulate);
+                         cplx<double> *C, long ldc, bool accumulate, int nbatch, long sP, long sC);
 
 static constexpr size_t kScratchBytes = size_t(64) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -83,6 +88,34 @@ int pp_overlap_gemm_noalloc(pp_ctx *ctx, int nwk, int nspin, int flip, const int
   PP_TRY(scratch_ptr(ctx->device, &P));
   const int max_split64 = (int)(kScratchBytes / plane);  // FP64 partial planes that fit
   hipStream_t st = ctx->stream;
+  if (precision == PP_FP64 && !ctx->tune_gemm_f64_valu) {
+    // the k-points of one launch and their K chunks as pp_overlap_gemm takes
+    // them where the partials fit the array; fewer of either where not
+    for (int k0 = 0; k0 < nkt;) {
+      GemmBatch gb;
+      gb.n = std::min({nkt - k0, (int)GemmBatch::MAX, max_split64});
+      for (int i = 0; i < gb.n; i++) {
+        const int k = k0 + i;
+        gb.a[i] = (flip && nspin == 2) ? (k < nwk ? k + nwk : k - nwk) : k;
+        gb.b[i] = k;
+        gb.k[i] = nw[k];
+      }
+      int nsplit, kchunk;
+      zgemm64_split(nbR, nbS, gb, ctx->tune_splitk, false, nsplit, kchunk);
+      if (nsplit > max_split64 / gb.n)
+        zgemm64_split(nbR, nbS, gb, max_split64 / gb.n, false, nsplit, kchunk);
+      const long mn = (long)nbR * nbS;
+      cplx<double> *C = (cplx<double> *)out_dev + k0 * mn;
+      const bool direct = nsplit == 1;
+      PP_TRY(launch_zgemm64(st, nbR, nbS, gb, 1, CR_dev, ldR, (long)nbR * ldR, nullptr, 1, CS_dev, ldS,
+                            (long)nbS * ldS, direct ? C : P, (long)nbS, mn, direct ? mn : mn * nsplit, nsplit, kchunk,
+                            false));
+      if (!direct)
+        PP_TRY(launch_splitk_reduce(st, nbR, nbS, nsplit, P, false, C, nbS, false, gb.n, mn * nsplit, mn));
+      k0 += gb.n;
+    }
+    return PP_OK;
+  }
   for (int k = 0; k < nkt; k++) {
     const int kR = (flip && nspin == 2) ? (k < nwk ? k + nwk : k - nwk) : k;
     const void *A = (const char *)CR_dev + (size_t)kR * nbR * ldR * sizeof(cplx<float>);
@@ -90,7 +123,7 @@ int pp_overlap_gemm_noalloc(pp_ctx *ctx, int nwk, int nspin, int flip, const int
     cplx<double> *C = (cplx<double> *)out_dev + (size_t)k * nbR * nbS;
     const int K = nw[k];
     // the split policy of pp_overlap_gemm where its partials fit the array
-    int nsplit = splitk_count(precision, nbR, nbS, K, ctx->tune_splitk);
+    int nsplit = splitk_count(precision, nbR, nbS, K, ctx->tune_splitk, 1, false);
     int kchunk;
     bool fp32p = false;
     if (precision == PP_FP32) {
@@ -109,12 +142,12 @@ int pp_overlap_gemm_noalloc(pp_ctx *ctx, int nwk, int nspin, int flip, const int
       kchunk = (K + nsplit - 1) / nsplit;
       kchunk = std::max(16, (kchunk + 15) / 16 * 16);
       nsplit = std::max(1, (K + kchunk - 1) / kchunk);
-      PP_TRY(launch_zgemm64(st, ctx->tune_gemm_f64_valu != 0, nbR, nbS, K, 1, A, ldR, 1, B, ldS, P, (long)nbS,
-                            (long)nbR * nbS, nsplit, kchunk));
+      PP_TRY(launch_zgemm64_valu(st, nbR, nbS, K, 1, A, ldR, 1, B, ldS, P, (long)nbS, (long)nbR * nbS, nsplit,
+                                 kchunk));
     }
     // the next k-point's GEMM overwrites the partials only after this
     // reduction has read them (one stream, in order)
-    PP_TRY(launch_splitk_reduce(st, nbR, nbS, nsplit, P, fp32p, C, nbS, false));
+    PP_TRY(launch_splitk_reduce(st, nbR, nbS, nsplit, P, fp32p, C, nbS, false, 1, 0, 0));
   }
   return PP_OK;
 }

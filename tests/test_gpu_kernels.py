@@ -264,6 +264,32 @@ def test_overlap_mixed(ctx, precision, tol):
     assert err < tol
 
 
+@pytest.mark.parametrize("nbR,nbS,nk,splitk", [(1, 1, 1, 0), (16, 17, 2, 0), (33, 48, 3, 5), (64, 65, 17, 0), (81, 127, 2, 3),
+                                               (130, 20, 18, 1)])
+def test_overlap_fp64_batched_edges(ctx, nbR, nbS, nk, splitk):
+    """The FP64 GEMM runs up to 16 k-points in a launch and only the 16x16
+    tiles that hold outputs: band counts around tile edges, k-point counts
+    around a launch's, uneven plane-wave counts (one k-point empty, counts
+    off the 16-term k-step), one chunk and several, against numpy in FP64.
+    The sums' order differs: 1e-13 of the 2 nw that |a|^2 |b|^2 sum to."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(nbR + nk)
+    nw = rng.integers(900, 2001, nk).astype(np.int32)
+    nw[nk // 2] = 0 if nk > 1 else 37
+    CR, CS = ((rng.standard_normal((nk, nb, 2048)) + 1j * rng.standard_normal((nk, nb, 2048))).astype(np.complex64)
+              for nb in (nbR, nbS))
+    out = torch.full((nk, nbR, nbS), np.nan, dtype=torch.complex128, device="cuda")
+    R, S = torch.from_numpy(CR).cuda(), torch.from_numpy(CS).cuda()
+    torch.cuda.synchronize()
+    ctx.set_param("gemm_splitk", splitk)
+    B.overlap_gemm(ctx, nk, 1, False, nw, R, S, out, "fp64")
+    ctx.set_param("gemm_splitk", 0)
+    got = out.cpu().numpy()
+    for k in range(nk):
+        a, b = CR[k, :, : nw[k]].astype(np.complex128), CS[k, :, : nw[k]].astype(np.complex128)
+        assert np.abs(got[k] - a.conj() @ b.T).max() <= 1e-13 * max(1.0, 2.0 * nw[k])
+
+
 @pytest.mark.parametrize("precision", ["fp32", "fp16x3", "bf16x6"])
 def test_overlap_split_planes_row_scales(ctx, precision):
     """Split-plane overlaps of rows whose magnitudes span eleven decades (and
