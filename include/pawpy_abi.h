@@ -256,16 +256,18 @@ int pp_ctx_set_tuning(pp_ctx *ctx, int fft_bands, int fft_tile, int fft_prune,
  * plan allows -- it writes no real-space grid but measured slower on the
  * 216-atom workload), "fft_xcd" (1: FFT pass work-groups walk
  * XCD-contiguous line ranges), "fft_fixed" (1, default: FFT passes along
- * axes of length 60, 108, 192 or 216 run kernels compiled for that length,
- * with every index and offset a constant; 0: the generic in-place passes;
- * the two agree to rounding), "fft_nt" (FFT passes: 0 cached, 1
+ * axes of a compiled length -- the even ones with factors 2, 3, 5 and 7 up
+ * to 256 and their usual doubles -- run as two register-level DFTs with one
+ * LDS exchange when the chunk holds whole 128-byte band groups; 0: the
+ * staged passes, which the fft_tile, fft_threads, fft_radix, fft_persistent
+ * and fft_pingpong settings are for; the two agree to rounding), "fft_nt" (FFT passes: 0 cached, 1
  * non-temporal stores, 2 non-temporal loads and stores, default 2; 3:
  * cached z pass, streamed stores in the y pass, streamed x pass),
  * "sphere_nt" (1, default: sphere-sum gathers with non-temporal loads),
  * "fft_xmask" (1: the x pass of a setup writes only the grid points some
- * projector sphere holds, the only ones the sphere sums read; 0, default:
- * every point -- the masked stores measured slower on the 216-atom
- * workload although they write 31% fewer bytes), "rs_kernel" (real-space
+ * projector sphere holds, the only ones the sphere sums read; 0: every
+ * point; -1, default: 1 when the x axis has a compiled pass, whose stores
+ * the test costs nothing), "rs_kernel" (real-space
  * augmentation: 0 a site's coefficients in LDS, 1 in registers (up to 32
  * projectors per site), 2, default: tiles of points with their table rows
  * in LDS and the coefficients in registers (up to 18 projectors per site;

@@ -130,7 +130,7 @@ struct SetupState {
   void *phase = nullptr;
   int *gidx = nullptr, *bnd = nullptr, *dlines = nullptr;
   std::vector<int> alias;
-  std::vector<long> zl_off, yl_off;
+  std::vector<long> zl_off, nzl, nyl;
 };
 
 // Where a prepared setup keeps what setup_prepare computes from the call's
@@ -150,11 +150,7 @@ static int setup_prepare(pp_ctx *ctx, pp_sphere *sp, int nk, const double *kfrac
                          int nband, SetupState &S, const PrepBufs &pb) {
   const int *fftg = sphere_fftg(sp);
   PP_TRY(get_fft_plan(ctx, fftg, &S.pl));
-  int NB = ctx->tune_fft_bands > 0 ? ctx->tune_fft_bands : 64;
-  if (NB > 64)
-    NB = 64;
-  if (NB > nband)
-    NB = nband < 1 ? 1 : nband;
+  const int NB = chunk_bands(nband, ctx->tune_fft_bands, 128 / (int)sizeof(cplx<T>));
   S.NB = NB;
   const long npts_grid = (long)fftg[0] * fftg[1] * fftg[2];
   S.ptot = sphere_ptot(sp);
@@ -192,29 +188,18 @@ static int setup_prepare(pp_ctx *ctx, pp_sphere *sp, int nk, const double *kfrac
   // populated lines of the z pass ((x, y) in the sphere's hull) and of the
   // y pass ((x, z) with x in the slab), so no work-group is launched for an
   // empty line
-  S.zl_off.assign(nk + 1, 0);
-  S.yl_off.assign(nk + 1, 0);
+  S.zl_off.assign(nk, 0);
+  S.nzl.assign(nk, 0);
+  S.nyl.assign(nk, 0);
   pb.lines_host[0].clear();
-  const int n0 = fftg[0], n1 = fftg[1], n2 = fftg[2];
   for (int k = 0; k < nk; k++) {
     const int *hb = pb.bounds_host[0].data() + (size_t)k * S.nbnd;
     // no pruning when the grid aliases a G or the G set leaves holes in a
     // z-line's interval (not a cutoff sphere)
     S.alias[k] = hb[S.nbnd - 1] || !bounds_filled(hb, fftg, gofs[k + 1] - gofs[k]);
-    const int *yb = hb + 2 * n0 * n1, *xb = yb + 2 * n0;
     S.zl_off[k] = (long)pb.lines_host[0].size();
     if (!S.alias[k])
-      for (int sx = xb[0]; sx <= xb[1]; sx++) {
-        const int x = (sx + n0) % n0;
-        for (int sy = yb[2 * x]; sy <= yb[2 * x + 1]; sy++)
-          pb.lines_host[0].push_back(x * n1 + (sy + n1) % n1);
-      }
-    S.yl_off[k] = (long)pb.lines_host[0].size();
-    if (!S.alias[k])
-      for (int sx = xb[0]; sx <= xb[1]; sx++)
-        for (int z = 0; z < n2; z++)
-          pb.lines_host[0].push_back(((sx + n0) % n0) * n2 + z);
-    S.zl_off[k + 1] = (long)pb.lines_host[0].size();
+      push_pass_lines(hb, fftg, pb.lines_host[0], S.nzl[k], S.nyl[k]);
   }
   S.dlines = nullptr;
   if (!pb.lines_host[0].empty()) {
@@ -259,12 +244,12 @@ static int setup_launch(pp_ctx *ctx, pp_sphere *sp, int nk, const int *gofs, con
                        fftg[2]};
     if (S.dlines && !S.alias[k] && ctx->tune_fft_prune != 3) {
       bd.zl = S.dlines + S.zl_off[k];
-      bd.nzl = (int)(S.yl_off[k] - S.zl_off[k]);
-      bd.yl = S.dlines + S.yl_off[k];
-      bd.nyl = (int)(S.zl_off[k + 1] - S.yl_off[k]);
+      bd.nzl = (int)S.nzl[k];
+      bd.yl = S.dlines + S.zl_off[k] + 2 * S.nzl[k];
+      bd.nyl = (int)S.nyl[k];
     }
     const bool prune = S.alias[k] == 0 && ctx->tune_fft_prune != 2;
-    if (ctx->tune_fft_xmask && !S.fused)
+    if (!S.fused && fft_masked_stores<T>(ctx, S.pl, NB))
       bd.xm = sphere_xmask(sp, &bd.xmw);
     const cplx<T> *phase_k = (const cplx<T> *)S.phase + (size_t)k * S.npts_sph;
     for (int b0 = 0; b0 < nband && st == PP_OK; b0 += NB, c++) {
@@ -311,7 +296,7 @@ static int aug_freqs_batched(pp_ctx *ctx, pp_sphere *sp, int nk, const double *k
   const int *fftg = sphere_fftg(sp);
   FftPlan *pl = nullptr;
   PP_TRY(get_fft_plan(ctx, fftg, &pl));
-  const int NB = std::min(64, std::max(1, nband));
+  const int NB = chunk_bands(nband, 0, 128 / (int)sizeof(cplx<T>));
   const long npts_grid = (long)fftg[0] * fftg[1] * fftg[2];
   const long npts_sph = std::max<long>(1, sphere_npts(sp));
   PP_TRY(ctx->grid.ensure(sizeof(cplx<T>) * (size_t)npts_grid * NB));
@@ -525,7 +510,7 @@ int pp_ctx_set_param(pp_ctx *ctx, const char *name, int value) {
   else if (n == "fft_radix")
     ctx->tune_fft_radix = value != 0 ? 1 : 0;
   else if (n == "fft_xmask")
-    ctx->tune_fft_xmask = value != 0 ? 1 : 0;
+    ctx->tune_fft_xmask = value < 0 ? -1 : value != 0;
   else if (n == "fft_xcd")
     ctx->tune_fft_xcd = value != 0 ? 1 : 0;
   else if (n == "fft_fixed")

@@ -263,8 +263,8 @@ extern "C" int pp_fft3d_batched(pp_ctx *ctx, const double *lattice, const int *f
   FftPlan *pl = nullptr;
   PP_TRY(get_fft_plan(ctx, fftg, &pl));
   const long npts = (long)fftg[0] * fftg[1] * fftg[2];
-  int NB = nband;
   bool f64 = precision == PP_FP64;
+  const int NB = chunk_bands(nband, 0, f64 ? 8 : 16);
   size_t csz = f64 ? sizeof(cplx<double>) : sizeof(cplx<float>);
   PP_TRY(ctx->grid.ensure(csz * (size_t)npts * NB));
   PP_TRY(ctx->gidx.ensure(sizeof(int) * (size_t)std::max(1, nw)));

@@ -13,7 +13,9 @@
 // Stockham transform (radices 4,2,3,5 and any other small prime) there,
 // and writes the line back in place.
 #include <cmath>
+#include <initializer_list>
 
+#include "pp_fft2.h"
 #include "pp_internal.h"
 #include "pp_stages.h"
 
@@ -76,6 +78,17 @@ static void push_stage_twiddles(std::vector<double> &tw, int p, int R) {
   }
 }
 
+const Fft2Entry *fft2_table_a(), *fft2_table_b(), *fft2_table_c(), *fft2_table_d(), *fft2_table_e(), *fft2_table_f(),
+    *fft2_table_g(), *fft2_table_h();
+const Fft2Entry *fft2_entry(int n) {
+  for (const Fft2Entry *t : {fft2_table_a(), fft2_table_b(), fft2_table_c(), fft2_table_d(), fft2_table_e(),
+                             fft2_table_f(), fft2_table_g(), fft2_table_h()})
+    for (; t->n; t++)
+      if (t->n == n)
+        return t;
+  return nullptr;
+}
+
 int get_fft_plan(pp_ctx *ctx, const int *fftg, FftPlan **out) {
   long long key = ((long long)fftg[0] << 40) | ((long long)fftg[1] << 20) | fftg[2];
   auto it = ctx->fft_plans.find(key);
@@ -119,6 +132,16 @@ int get_fft_plan(pp_ctx *ctx, const int *fftg, FftPlan **out) {
       }
     }
     ap.twlen = (int)(tw.size() / 2) - pl->twbase[a];
+    // the [k1][j2] twiddles of the two-DFT pass, past the staged ones
+    ap.tw2off = ap.twlen;
+    if (const Fft2Entry *fe = fft2_entry(fftg[a]))
+      for (int k1 = 0; k1 < fe->r1; k1++)
+        for (int j2 = 0; j2 < fe->r2; j2++) {
+          const long double ang =
+              2.0L * 3.14159265358979323846264338327950288L * (long double)(k1 * j2) / (long double)fftg[a];
+          tw.push_back((double)cosl(ang));
+          tw.push_back((double)sinl(ang));
+        }
   }
   size_t ntw = tw.size() / 2;
   std::vector<float> tw32(tw.size());
@@ -261,7 +284,7 @@ __device__ void stage_generic(const cplx<T> *__restrict__ in, cplx<T> *__restric
 template <int AXIS>
 __device__ __forceinline__ int pass_line(const SphereBounds &bd, int l) {
   const int *ll = AXIS == 2 ? bd.zl : AXIS == 1 ? bd.yl : nullptr;
-  return ll ? ll[l] : l;
+  return ll ? ll[2 * l] : l;
 }
 
 // One pass of 1D transforms along an axis.  Work-group: one line (fixed
@@ -357,16 +380,13 @@ __global__ __launch_bounds__(256) void k_fft_pass(cplx<T> *__restrict__ g, AxisP
 // also read with non-temporal loads (each pass touches its data once).
 // The work of one work-group of the in-place pass: tile blk (line
 // blk / nslices, band slice blk % nslices) of the chunk g.
-// N > 0: the axis length and its stages are compile-time constants
-// (stages_fixed); the host launches that form only when its plan has the
-// same stages.
-template <typename T, int NBW, int AXIS, int MAXB, int NT, bool COMP, int N = 0>
+template <typename T, int NBW, int AXIS, int MAXB, int NT, bool COMP>
 __device__ __forceinline__ void fft_pass_ip_tile(cplx<T> *__restrict__ g, const AxisPlan &pl,
                                                  const cplx<T> *__restrict__ tw, long es, long s1, long s2, int n2,
                                                  int nslices, const SphereBounds &bd, int blk, int streaming) {
   extern __shared__ unsigned char smem_raw[];
   cplx<T> *buf = reinterpret_cast<cplx<T> *>(smem_raw);
-  const int n = N > 0 ? N : pl.n;
+  const int n = pl.n;
   const int slice = blk % nslices;
   const int line = pass_line<AXIS>(bd, blk / nslices);
   const int l1 = line / n2, l2 = line % n2;
@@ -395,69 +415,9 @@ __device__ __forceinline__ void fft_pass_ip_tile(cplx<T> *__restrict__ g, const 
   // the line's loads are issued in batches of FFT_LB per thread before any
   // is written to LDS, so that many are in flight at once (a load-then-store
   // loop waits for each load in turn); FP32 lines move two bands (16 bytes)
-  // per access.  Compile-time lengths: a thread's elements are EST apart on
-  // the axis, so their addresses step by a uniform stride from one base.
-  constexpr int PK = (sizeof(T) == 4 && NBW % 2 == 0) ? 2 : 1;  // complex values per access
-  constexpr int EST = PK * NT / NBW;
-  constexpr bool FXLS = N > 0 && (PK * NT) % NBW == 0;
-  constexpr int FX_MW = N > 0 ? (N + 31) / 32 : 1;  // coverage words of an x line
-  unsigned mw[FX_MW];
-  // compile-time lengths: the first 2 NT twiddles (all of them for the
-  // compiled lengths) are read into registers ahead of the line's loads and
-  // written to LDS after them, so that the two wait on one memory latency
-  // rather than one after the other
-  cplx<T> twv[2];
-  if constexpr (FXLS) {
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-      const int i = threadIdx.x + r * NT;
-      twv[r] = i < pl.twlen ? tw[i] : mk<T>(0, 0);
-    }
-    for (int i = threadIdx.x + 2 * NT; i < pl.twlen; i += NT)
-      twl[i] = tw[i];
-  } else
-    stage_twiddles<T, NT>(twl, tw, pl.twlen);
-  if constexpr (FXLS) {
-    constexpr int TOTA = N * NBW / PK, EPT = (TOTA + NT - 1) / NT;
-    const int t = threadIdx.x, e0 = PK * t / NBW, bb = PK * t % NBW;
-    const cplx<T> *p = g + base + (long)e0 * es + bb;
-    const long step = (long)EST * es;
-    cplx<T> va[EPT][PK];
-#pragma unroll
-    for (int u = 0; u < EPT; u++) {
-#pragma unroll
-      for (int c = 0; c < PK; c++)
-        va[u][c] = mk<T>(0, 0);
-      const int e = e0 + u * EST;
-      const int se = e < N - N / 2 ? e : e - N;
-      if ((TOTA % NT == 0 || t + u * NT < TOTA) && se >= lo && se <= hi) {
-        if constexpr (PK == 2)
-          load2(reinterpret_cast<const cplx<float> *>(p + u * step), streaming > 1, va[u][0], va[u][1]);
-        else
-          va[u][0] = streaming > 1 ? load_nt(p + u * step) : p[u * step];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-      if (threadIdx.x + r * NT < pl.twlen)
-        twl[threadIdx.x + r * NT] = twv[r];
-#pragma unroll
-    for (int u = 0; u < EPT; u++)
-      if (TOTA % NT == 0 || t + u * NT < TOTA) {
-#pragma unroll
-        for (int c = 0; c < PK; c++)
-          buf[PK * (t + u * NT) + c] = va[u][c];
-      }
-    // the x line's coverage words, read here so that their loads complete
-    // during the stages and the masked stores below test registers (a load
-    // of the word beside each store waited for it store by store)
-    if constexpr (AXIS == 0) {
-      const unsigned *xm0 = bd.xm ? bd.xm + (long)line * bd.xmw : nullptr;
-#pragma unroll
-      for (int q = 0; q < FX_MW; q++)
-        mw[q] = (xm0 && q < bd.xmw) ? xm0[q] : ~0u;
-    }
-  } else if constexpr (sizeof(T) == 4 && NBW % 2 == 0) {
+  // per access.
+  stage_twiddles<T, NT>(twl, tw, pl.twlen);
+  if constexpr (sizeof(T) == 4 && NBW % 2 == 0) {
     const int tot2 = tot / 2;
     for (int t0 = threadIdx.x; t0 < tot2; t0 += NT * FFT_LB) {
       cplx<T> va[FFT_LB], vb[FFT_LB];
@@ -499,46 +459,8 @@ __device__ __forceinline__ void fft_pass_ip_tile(cplx<T> *__restrict__ g, const 
         buf[t0 + u * NT] = v[u];
   }
   __syncthreads();
-  if constexpr (N > 0)
-    stages_fixed<T, NBW, N, NT>(buf, twl);
-  else
-    stages_ip<T, NBW, MAXB, NT, COMP>(buf, twl, pl, n);
+  stages_ip<T, NBW, MAXB, NT, COMP>(buf, twl, pl, n);
   const unsigned *xm = (AXIS == 0 && bd.xm) ? bd.xm + (long)line * bd.xmw : nullptr;
-  if constexpr (FXLS) {
-    constexpr int TOTA = N * NBW / PK, EPT = (TOTA + NT - 1) / NT;
-    const int t = threadIdx.x, e0 = PK * t / NBW, bb = PK * t % NBW;
-    cplx<T> *p = g + base + (long)e0 * es + bb;
-    const long step = (long)EST * es;
-    cplx<T> va[EPT][PK];
-#pragma unroll
-    for (int u = 0; u < EPT; u++)
-      if (TOTA % NT == 0 || t + u * NT < TOTA) {
-#pragma unroll
-        for (int c = 0; c < PK; c++)
-          va[u][c] = buf[PK * (t + u * NT) + c];
-      }
-#pragma unroll
-    for (int u = 0; u < EPT; u++) {
-      const int e = e0 + u * EST;
-      if (!(TOTA % NT == 0 || t + u * NT < TOTA))
-        continue;
-      if constexpr (AXIS == 0) {
-        unsigned w = mw[0];
-#pragma unroll
-        for (int q = 1; q < FX_MW; q++)
-          w = (e >> 5) == q ? mw[q] : w;
-        if (!((w >> (e & 31)) & 1u))
-          continue;  // no projector sphere reads this point
-      }
-      if constexpr (PK == 2)
-        store2(reinterpret_cast<cplx<float> *>(p + u * step), streaming != 0, va[u][0], va[u][1]);
-      else if (streaming)
-        store_nt(p + u * step, va[u][0]);
-      else
-        p[u * step] = va[u][0];
-    }
-    return;
-  }
   if constexpr (sizeof(T) == 4 && NBW % 2 == 0) {
     const int tot2 = tot / 2;
     for (int t0 = threadIdx.x; t0 < tot2; t0 += NT * FFT_LB) {
@@ -595,50 +517,22 @@ __global__ __launch_bounds__(NT, (FftWaves<T, MAXB, COMP>::value)) void k_fft_pa
   fft_pass_ip_tile<T, NBW, AXIS, MAXB, NT, COMP>(g, pl, tw, es, s1, s2, n2, nslices, bd, blk, streaming);
 }
 
-// The in-place pass for an axis of compile-time length N (see
-// fft_pass_ip_tile); FP32 kernels at 8 wavefronts per SIMD as
-// k_fft_pass_ip's.
-template <typename T, int NBW, int AXIS, int N, int NT>
-__global__ __launch_bounds__(NT, (PassWaves<T, 4, N, NBW>::value)) void k_fft_pass_fx(
-    cplx<T> *__restrict__ g, AxisPlan pl, const cplx<T> *__restrict__ tw, long es, long s1, long s2, int n2,
-    int nslices, SphereBounds bd, int xcd_per, int nblk, int streaming) {
-  const int blk = xcd_per > 0 ? (int)(blockIdx.x % 8) * xcd_per + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-  if (blk >= nblk)
-    return;
-  fft_pass_ip_tile<T, NBW, AXIS, 4, NT, false, N>(g, pl, tw, es, s1, s2, n2, nslices, bd, blk, streaming);
-}
-
 // The same pass over the chunks of a batch of work items (one per
 // blockIdx.y): each item brings its own chunk buffer and the plane-wave
 // bounds and line lists of its k-point; tiles past the item's lines exit.
 // (7 rather than 8 waves per SIMD where the single-chunk pass takes 8: the
 // descriptor's pointers and counts cost a few registers, and 64 would spill)
-template <typename T, int NBW, int AXIS, int MAXB, int NT, int N = 0>
-__global__ __launch_bounds__(NT, (PassWaves<T, MAXB, N, NBW>::value == 8 ? 7 : PassWaves<T, MAXB, N, NBW>::value))
-void k_fft_pass_ip_items(
+template <typename T, int NBW, int AXIS, int MAXB, int NT>
+__global__ __launch_bounds__(NT, (FftWaves<T, MAXB, false>::value == 8 ? 7 : 1)) void k_fft_pass_ip_items(
     const ChunkItem *__restrict__ items, AxisPlan pl, const cplx<T> *__restrict__ tw, long es, long s1, long s2,
     int n2, int nslices, int streaming) {
   const ChunkItem *it = items + blockIdx.y;
-  SphereBounds bd;
-  bd.zb = (const int *)it->zb;
-  bd.yb = (const int *)it->yb;
-  bd.xb = (const int *)it->xb;
-  bd.n0 = it->n0;
-  bd.n1 = it->n1;
-  bd.n2 = it->n2;
-  bd.zl = AXIS == 2 ? (const int *)it->zl : nullptr;
-  bd.nzl = AXIS == 2 ? it->nzl : 0;
-  bd.yl = AXIS == 1 ? (const int *)it->yl : nullptr;
-  bd.nyl = AXIS == 1 ? it->nyl : 0;
-  bd.xm = AXIS == 0 ? (const unsigned *)it->xm : nullptr;
-  bd.xmw = AXIS == 0 ? it->xmw : 0;
-  const long nlin = AXIS == 2 ? (bd.zl ? bd.nzl : (long)bd.n0 * bd.n1)
-                              : AXIS == 1 ? (bd.yl ? bd.nyl : (long)bd.n0 * bd.n2) : (long)bd.n1 * bd.n2;
+  const SphereBounds bd = item_bounds(it, AXIS);
   const int blk = (int)blockIdx.x;
-  if (blk >= nlin * nslices)
+  if (blk >= pass_lines(bd, AXIS) * nslices)
     return;
-  fft_pass_ip_tile<T, NBW, AXIS, MAXB, NT, false, N>((cplx<T> *)it->grid, pl, tw, es, s1, s2, n2, nslices, bd, blk,
-                                                     streaming);
+  fft_pass_ip_tile<T, NBW, AXIS, MAXB, NT, false>((cplx<T> *)it->grid, pl, tw, es, s1, s2, n2, nslices, bd, blk,
+                                                  streaming);
 }
 
 // Line bounds of a pass (see k_fft_pass); false when the line is skipped.
@@ -843,29 +737,34 @@ int compute_gidx(pp_ctx *ctx, const int *fftg, int nw, const int *G_dev, int *gi
   return PP_OK;
 }
 
-// Axis lengths with a compile-time pass (k_fft_pass_fx): the grids of the
-// 64-atom (60), 216-atom (108), 512-atom (192) cells and the doubled
-// 216-atom grid (216).
-#define PP_FIXED_LENGTHS(X) X(60) X(108) X(192) X(216)
-static bool fixed_length(int n) {
-#define PP_FX_IS(NN) n == NN ||
-  return PP_FIXED_LENGTHS(PP_FX_IS) false;
-#undef PP_FX_IS
+// The two-DFT pass of an axis, where the length has one, the chunk holds
+// whole band groups and the staged forms are not asked for.
+static const Fft2Entry *fft2_pass(pp_ctx *ctx, const AxisPlan &ap, int NB, int bands) {
+  if (!ctx->tune_fft_fixed || ctx->tune_fft_pingpong || ctx->tune_fft_persistent || ctx->tune_fft_radix || NB % bands)
+    return nullptr;
+  return fft2_entry(ap.n);
 }
-// The compile-time pass serves an axis when its length has one and the
-// host plan's stages and twiddle offsets are the ones it was compiled with.
-// Its results agree with the generic pass's to rounding (the compiler is
-// free to contract the complex products differently in the two).
-static bool fixed_plan_matches(const AxisPlan &ap) {
-  if (!fixed_length(ap.n))
-    return false;
-  const FftFactors f = fft_factors(ap.n);
-  if (f.nst != ap.nst)
-    return false;
-  for (int s = 0; s < f.nst; s++)
-    if (f.r[s] != ap.radix[s] || f.p[s] != ap.pprev[s] || f.twoff[s] != ap.twoff[s])
-      return false;
-  return true;
+// Whether the x pass of a setup stores covered points only: fft_xmask, or by
+// itself with the two-DFT pass, whose stores the test costs nothing (216
+// atoms: x pass 210 -> 181 us per chunk, 64 atoms FP64 89 -> 56); the staged
+// passes are bound by their instructions and lose (setup 20.6 -> 21.5 ms).
+template <typename T> bool fft_masked_stores(pp_ctx *ctx, FftPlan *pl, int NB) {
+  if (ctx->tune_fft_xmask >= 0)
+    return ctx->tune_fft_xmask != 0;
+  return fft2_pass(ctx, pl->ax[0], NB, fft2_bands<T>()) != nullptr;
+}
+template bool fft_masked_stores<double>(pp_ctx *, FftPlan *, int);
+template bool fft_masked_stores<float>(pp_ctx *, FftPlan *, int);
+// Streaming access of a pass: fft_nt 0..2 for every pass; 3 keeps the z
+// pass's stores cacheable (the y pass reads them next), streams the y
+// pass's stores and both directions of the x pass.
+static int nt_mode_of(pp_ctx *ctx, int axis) {
+  return ctx->tune_fft_nt < 3 ? ctx->tune_fft_nt : (axis == 2 ? 0 : axis == 1 ? 1 : 2);
+}
+template <typename T>
+static Fft2Args<T> fft2_args(pp_ctx *ctx, const AxisPlan &ap, const cplx<T> *tw, int axis, long es, long s1, long s2,
+                             int n2, int NB, long nlines) {
+  return {tw + ap.tw2off, es, s1, s2, axis, n2, NB / fft2_bands<T>(), nt_mode_of(ctx, axis), nlines};
 }
 
 template <typename T, int NBW, int AXIS>
@@ -895,10 +794,7 @@ static int launch_pass(pp_ctx *ctx, cplx<T> *grid, const AxisPlan &ap, const cpl
   for (int s = 0; comp && s < ap.nstc; s++)
     if (!dft_supported(ap.radixc[s]) || ((ap.n / ap.radixc[s]) * NBW + 255) / 256 > 2)
       comp = false;
-  // streaming access: fft_nt 0..2 for every pass; 3 keeps the z pass's
-  // stores cacheable (the y pass reads them next), streams the y pass's
-  // stores and both directions of the x pass
-  const int nt_mode = ctx->tune_fft_nt < 3 ? ctx->tune_fft_nt : (AXIS == 2 ? 0 : AXIS == 1 ? 1 : 2);
+  const int nt_mode = nt_mode_of(ctx, AXIS);
   // XCD-contiguous line ranges (fft_xcd = 1)
   const int xcd_per = ctx->tune_fft_xcd ? (int)((nblk + 7) / 8) : 0;
   const long nlaunch = xcd_per ? 8L * xcd_per : nblk;
@@ -940,21 +836,6 @@ static int launch_pass(pp_ctx *ctx, cplx<T> *grid, const AxisPlan &ap, const cpl
         PP_PL(8, 16);
 #undef PP_PL
       launched = true;
-    }
-    // the compile-time pass for the default tile width (16 FP32, 8 FP64 bands)
-    // and twice it
-    if constexpr (NBW == (sizeof(T) == 4 ? 16 : 8) || NBW == (sizeof(T) == 4 ? 32 : 16)) {
-      if (!launched && ip && nt == 256 && ctx->tune_fft_fixed && fixed_plan_matches(ap)) {
-        size_t lds = ((size_t)ap.n * NBW + ap.twlen) * sizeof(cplx<T>);
-#define PP_FX(NN)                                                                                               \
-  case NN:                                                                                                      \
-    hipLaunchKernelGGL((k_fft_pass_fx<T, NBW, AXIS, NN, 256>), dim3((unsigned)nlaunch), dim3(256), lds,         \
-                       ctx->stream, grid, ap, tw, es, s1, s2, n2, nslices, bd, xcd_per, (int)nblk, nt_mode);    \
-    launched = true;                                                                                            \
-    break;
-        switch (ap.n) { PP_FIXED_LENGTHS(PP_FX) default: break; }
-#undef PP_FX
-      }
     }
     if (!launched && ip) {
       size_t lds = ((size_t)ap.n * NBW + ap.twlen) * sizeof(cplx<T>);
@@ -998,6 +879,21 @@ static int launch_pass(pp_ctx *ctx, cplx<T> *grid, const AxisPlan &ap, const cpl
 template <typename T, int AXIS>
 static int run_pass(pp_ctx *ctx, cplx<T> *grid, const AxisPlan &ap, const cplx<T> *tw, long es, long s1, long s2,
                     int n1, int n2, int NB, int cls, const SphereBounds &bd) {
+  if (const Fft2Entry *fe = fft2_pass(ctx, ap, NB, fft2_bands<T>())) {
+    const long nlines = pass_lines(bd, AXIS);
+    if (nlines == 0)
+      return PP_OK;
+    const Fft2Args<T> a = fft2_args<T>(ctx, ap, tw, AXIS, es, s1, s2, n2, NB, nlines);
+    hipEvent_t ev;
+    tbegin(ctx, cls, &ev);
+    if constexpr (sizeof(T) == 4)
+      fe->f32(ctx->stream, grid, a, bd, ctx->tune_fft_xcd != 0);
+    else
+      fe->f64(ctx->stream, grid, a, bd, ctx->tune_fft_xcd != 0);
+    tend(ctx, cls, ev);
+    PP_CHECK_HIP(hipGetLastError());
+    return PP_OK;
+  }
   const size_t ldsmax = 64 * 1024;
   int nbw = ctx->tune_fft_tile > 0 ? ctx->tune_fft_tile : (sizeof(T) == 4 ? 16 : 8);
   while (nbw > 1 && (NB % nbw != 0 || (size_t)2 * ap.n * nbw * sizeof(cplx<T>) > ldsmax))
@@ -1051,24 +947,12 @@ static int launch_pass_items(pp_ctx *ctx, const ChunkItem *items, int nitems, lo
     }
     if (!ip || maxb > 8)
       return PP_ERR_UNSUPPORTED;
-    const int nt_mode = ctx->tune_fft_nt < 3 ? ctx->tune_fft_nt : (AXIS == 2 ? 0 : AXIS == 1 ? 1 : 2);
+    const int nt_mode = nt_mode_of(ctx, AXIS);
     const size_t lds = ((size_t)ap.n * NBW + ap.twlen) * sizeof(cplx<T>);
     dim3 grd((unsigned)nblk, (unsigned)nitems);
     hipEvent_t ev;
     tbegin(ctx, cls, &ev);
     bool done = false;
-    if constexpr (NBW == (sizeof(T) == 4 ? 16 : 8) || NBW == (sizeof(T) == 4 ? 32 : 16)) {
-      if (nt == 256 && ctx->tune_fft_fixed && fixed_plan_matches(ap)) {
-#define PP_FXI(NN)                                                                                              \
-  case NN:                                                                                                      \
-    hipLaunchKernelGGL((k_fft_pass_ip_items<T, NBW, AXIS, 4, 256, NN>), grd, dim3(256), lds, ctx->stream, items, ap, \
-                       tw, es, s1, s2, n2, nslices, nt_mode);                                                   \
-    done = true;                                                                                                \
-    break;
-        switch (ap.n) { PP_FIXED_LENGTHS(PP_FXI) default: break; }
-#undef PP_FXI
-      }
-    }
 #define PP_IPI(MB, NT)                                                                                           \
   hipLaunchKernelGGL((k_fft_pass_ip_items<T, NBW, AXIS, MB, NT>), grd, dim3(NT), lds, ctx->stream, items, ap, tw, es, \
                      s1, s2, n2, nslices, nt_mode)
@@ -1101,6 +985,20 @@ static int launch_pass_items(pp_ctx *ctx, const ChunkItem *items, int nitems, lo
 template <typename T, int AXIS>
 static int run_pass_items(pp_ctx *ctx, const ChunkItem *items, int nitems, long maxlines, const AxisPlan &ap,
                           const cplx<T> *tw, long es, long s1, long s2, int n2, int NB, int cls) {
+  if (const Fft2Entry *fe = fft2_pass(ctx, ap, NB, fft2_bands<T>())) {
+    if (maxlines == 0 || nitems == 0)
+      return PP_OK;
+    const Fft2Args<T> a = fft2_args<T>(ctx, ap, tw, AXIS, es, s1, s2, n2, NB, maxlines);
+    hipEvent_t ev;
+    tbegin(ctx, cls, &ev);
+    if constexpr (sizeof(T) == 4)
+      fe->items32(ctx->stream, items, nitems, a);
+    else
+      fe->items64(ctx->stream, items, nitems, a);
+    tend(ctx, cls, ev);
+    PP_CHECK_HIP(hipGetLastError());
+    return PP_OK;
+  }
   const size_t ldsmax = 64 * 1024;
   int nbw = ctx->tune_fft_tile > 0 ? ctx->tune_fft_tile : (sizeof(T) == 4 ? 16 : 8);
   while (nbw > 1 && (NB % nbw != 0 || (size_t)2 * ap.n * nbw * sizeof(cplx<T>) > ldsmax))
@@ -1124,6 +1022,8 @@ template <typename T> bool fft_items_supported(pp_ctx *ctx, FftPlan *pl, int NB)
   int nbw = ctx->tune_fft_tile > 0 ? ctx->tune_fft_tile : (sizeof(T) == 4 ? 16 : 8);
   for (int a = 0; a < 3; a++) {
     const AxisPlan &ap = pl->ax[a];
+    if (fft2_pass(ctx, ap, NB, fft2_bands<T>()))
+      continue;
     int w = nbw;
     while (w > 1 && (NB % w != 0 || (size_t)2 * ap.n * w * sizeof(cplx<T>) > 64 * 1024))
       w >>= 1;
@@ -1205,6 +1105,32 @@ int sphere_bounds(pp_ctx *ctx, const int *fftg, int nw, const int *G_dev, int *b
   hipLaunchKernelGGL(k_bounds_rows, dim3(1), dim3(256), 0, ctx->stream, fftg[0], fftg[1], bnd_dev);
   PP_CHECK_HIP(hipGetLastError());
   return PP_OK;
+}
+
+void push_pass_lines(const int *hb, const int *fftg, std::vector<int> &out, long &nzl, long &nyl) {
+  const int n0 = fftg[0], n1 = fftg[1], n2 = fftg[2];
+  const int *yb = hb + 2 * n0 * n1, *xb = yb + 2 * n0;
+  auto push = [&](int line, int lo, int hi) {
+    out.push_back(line);
+    out.push_back((int)(((unsigned)lo << 16) | ((unsigned)hi & 0xffffu)));
+  };
+  const size_t z0 = out.size();
+  for (int sx = xb[0]; sx <= xb[1]; sx++) {
+    const int x = (sx + n0) % n0;
+    for (int sy = yb[2 * x]; sy <= yb[2 * x + 1]; sy++) {
+      const int l = x * n1 + (sy + n1) % n1;
+      const bool any = hb[2 * l] <= hb[2 * l + 1];  // a line of the hull may hold no G
+      push(l, any ? hb[2 * l] : 1, any ? hb[2 * l + 1] : 0);
+    }
+  }
+  nzl = (long)(out.size() - z0) / 2;
+  for (int sx = xb[0]; sx <= xb[1]; sx++) {
+    const int x = (sx + n0) % n0;
+    const bool any = yb[2 * x] <= yb[2 * x + 1];
+    for (int z = 0; z < n2; z++)
+      push(x * n2 + z, any ? yb[2 * x] : 1, any ? yb[2 * x + 1] : 0);
+  }
+  nyl = (long)(out.size() - z0) / 2 - nzl;
 }
 
 bool bounds_filled(const int *hb, const int *fftg, long nw) {

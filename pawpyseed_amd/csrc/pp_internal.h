@@ -1,5 +1,6 @@
 // Internal host-side interfaces shared by the library's translation units.
 #pragma once
+#include <algorithm>
 #include <functional>
 #include <map>
 #include <string>
@@ -51,6 +52,7 @@ struct AxisPlan {
   int twoff[12];
   unsigned pmag[12];  // ceil(2^32 / pprev): j / pprev == umulhi(j, pmag) for j < 2^16 (pprev > 1)
   int twlen = 0;      // twiddle + root entries of this axis (both factorizations)
+  int tw2off = 0;     // the two-DFT pass's twiddles, past those
   // second factorization with composite radices (6, 8, 9, 12, 16): fewer
   // stages for the in-place passes; nstc = 0 when there is none
   int nstc = 0;
@@ -63,8 +65,8 @@ struct AxisPlan {
 struct SphereBounds {
   const int *zb, *yb, *xb;
   int n0, n1, n2;
-  // populated lines of the z and y passes (packed l1 * n2 + l2 of the
-  // pass), nullptr = every line
+  // populated lines of the z and y passes, two ints a line (push_pass_lines),
+  // nullptr = every line
   const int *zl = nullptr, *yl = nullptr;
   int nzl = 0, nyl = 0;
   // x pass: points of x-line y * n2 + z that some projector sphere holds,
@@ -135,9 +137,9 @@ struct pp_ctx {
   int tune_fft_radix = 0;       // 0: radices 2-5, 1: composite radices where they fit
   int tune_sphere_nt = 1;       // 1: sphere-sum gathers with non-temporal loads
   int tune_fft_nt = 2;          // FFT passes: 1 non-temporal stores, 2 non-temporal loads and stores
-  int tune_fft_xmask = 0;        // 1: the x pass writes only points a projector sphere holds
+  int tune_fft_xmask = -1;      // 1: the x pass writes only points a projector sphere holds; -1: by the pass
   int tune_fft_xcd = 0;         // 1: FFT pass work-groups in XCD-contiguous line ranges
-  int tune_fft_fixed = 1;       // 1: compile-time passes for the axis lengths that have one
+  int tune_fft_fixed = 1;       // 1: two-DFT passes for the axis lengths that have one
   int tune_fused = 0;           // 1: x pass fused with the sphere sums where the plan allows
   int tune_rs_kernel = 2;       // real-space augmentation: 0 LDS coefficients, 1 registers, 2 tiled
   int tune_rs_unroll = 4;       // real-space augmentation: points of a wavefront in flight (1, 2, 4)
@@ -209,6 +211,19 @@ int get_fft_plan(pp_ctx *ctx, const int *fftg, FftPlan **out);
 // Fill a device buffer with zeros (a kernel; no memset node).
 int zero_async(pp_ctx *ctx, void *p, size_t bytes);
 
+// Bands of a chunk for nband bands of 2 sizeof(T) bytes: as few chunks of at
+// most 64 as hold them, even ones, in whole 128-byte band groups (the
+// columns past the bands are transformed as they are and read by nobody):
+// 70 bands run as 48 + 22 rather than 64 + 6, 45 as one chunk of 48 whose
+// passes take whole groups (45 fell to the one-band tiles).  Less than half
+// a group stays as it is.  tune > 0 forces the width.
+inline int chunk_bands(int nband, int tune, int group) {
+  if (tune > 0)
+    return std::max(1, std::min(std::min(tune, 64), nband));
+  const int nch = std::max(1, (nband + 63) / 64), per = (std::max(1, nband) + nch - 1) / nch;
+  return 2 * per < group ? per : (per + group - 1) / group * group;
+}
+
 // Band-fastest grid chunk pipeline pieces (pp_fft.hip).
 int compute_gidx(pp_ctx *ctx, const int *fftg, int nw, const int *G_dev, int *gidx_dev);
 // Scatter and backward FFT of a band chunk; with last_pass false the x
@@ -219,6 +234,7 @@ int fft_chunk(pp_ctx *ctx, FftPlan *pl, cplx<T> *grid, int NB, int nw, const int
 // twiddle / root table of one axis in the precision of T
 template <typename T> const cplx<T> *fft_twiddles(FftPlan *pl, int axis);
 template <typename T> int fft_passes(pp_ctx *ctx, FftPlan *pl, cplx<T> *grid, int NB);
+template <typename T> bool fft_masked_stores(pp_ctx *ctx, FftPlan *pl, int NB);
 template <typename T>
 int gather_conj(pp_ctx *ctx, const cplx<T> *grid, int NB, int nbc, const int *gidx, int nw, double scl,
                 cplx<double> *out, long ldo);
@@ -230,6 +246,11 @@ int sphere_bounds(pp_ctx *ctx, const int *fftg, int nw, const int *G_dev, int *b
 bool bounds_filled(const int *hb, const int *fftg, long nw);
 int grid_to_bandmajor(pp_ctx *ctx, int precision, const void *grid, int NB, int nbc, long npts,
                       double scl, void *out);
+// Appends the populated lines of the z pass ((x, y) in the sphere's hull)
+// and of the y pass ((x, z) with x in the slab) under the host bounds hb to
+// out, each as the packed line (l1 * n2 + l2 of the pass) and its input
+// interval (lo << 16 | hi & 0xffff, signed indices; lo > hi: none).
+void push_pass_lines(const int *hb, const int *fftg, std::vector<int> &out, long &nzl, long &nyl);
 double det3(const double *m);
 // Real-space states (pp_realspace.hip): x *= e^{-2 pi i k.r} on the grid
 // fftg; out[b] = scale sum_r conj(R[b * ldr + r]) S[r] (synchronises).

@@ -85,11 +85,12 @@ static int multi_prepare(pp_ctx *ctx, const MultiArgs &a, const MultiBufs &mb, M
   PP_TRY(get_fft_plan(ctx, fftg, &S.pl));
   const int n0 = fftg[0], n1 = fftg[1], n2 = fftg[2];
   const long npts_grid = (long)n0 * n1 * n2;
-  int NB = ctx->tune_fft_bands > 0 ? std::min(64, ctx->tune_fft_bands) : 64;
   int maxnb = 0;
   for (int i = 0; i < a.nstruct * a.nk; i++)
     maxnb = std::max(maxnb, a.nband[i]);
-  NB = std::max(1, std::min(NB, maxnb));
+  // more than one chunk for some item: 64, as the items' counts differ
+  const int NB = maxnb > 64 ? chunk_bands(64, ctx->tune_fft_bands, 1)
+                            : chunk_bands(maxnb, ctx->tune_fft_bands, 128 / (int)sizeof(cplx<T>));
   S.NB = NB;
   if (!fft_items_supported<T>(ctx, S.pl, NB))
     return PP_ERR_UNSUPPORTED;
@@ -113,23 +114,13 @@ static int multi_prepare(pp_ctx *ctx, const MultiArgs &a, const MultiBufs &mb, M
   PP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   std::vector<int> &lh = *mb.lines_host;
   lh.clear();
-  std::vector<long> zl_off(a.nk + 1, 0), yl_off(a.nk + 1, 0);
+  std::vector<long> zl_off(a.nk, 0), nzl(a.nk, 0), nyl(a.nk, 0);
   for (int k = 0; k < a.nk; k++) {
     const int *hb = hb_all.data() + (size_t)k * nbnd;
     if (hb[nbnd - 1] || !bounds_filled(hb, fftg, a.gofs[k + 1] - a.gofs[k]))
       return PP_ERR_UNSUPPORTED;
-    const int *yb = hb + 2 * n0 * n1, *xb = yb + 2 * n0;
     zl_off[k] = (long)lh.size();
-    for (int sx = xb[0]; sx <= xb[1]; sx++) {
-      const int x = (sx + n0) % n0;
-      for (int sy = yb[2 * x]; sy <= yb[2 * x + 1]; sy++)
-        lh.push_back(x * n1 + (sy + n1) % n1);
-    }
-    yl_off[k] = (long)lh.size();
-    for (int sx = xb[0]; sx <= xb[1]; sx++)
-      for (int z = 0; z < n2; z++)
-        lh.push_back(((sx + n0) % n0) * n2 + z);
-    zl_off[k + 1] = (long)lh.size();
+    push_pass_lines(hb, fftg, lh, nzl[k], nyl[k]);
   }
   PP_TRY(mb.lines->ensure(sizeof(int) * std::max<size_t>(1, lh.size())));
   int *dl = (int *)mb.lines->p;
@@ -152,13 +143,13 @@ static int multi_prepare(pp_ctx *ctx, const MultiArgs &a, const MultiBufs &mb, M
     const int *kb = bnd + (size_t)k * nbnd;
     SphereBounds bd = {kb, kb + 2 * n0 * n1, kb + 2 * n0 * n1 + 2 * n0, n0, n1, n2};
     bd.zl = dl + zl_off[k];
-    bd.nzl = (int)(yl_off[k] - zl_off[k]);
-    bd.yl = dl + yl_off[k];
-    bd.nyl = (int)(zl_off[k + 1] - yl_off[k]);
+    bd.nzl = (int)nzl[k];
+    bd.yl = dl + zl_off[k] + 2 * nzl[k];
+    bd.nyl = (int)nyl[k];
     for (int s = 0; s < a.nstruct; s++) {
       const int i = s * a.nk + k;
       SphereBounds bds = bd;
-      if (ctx->tune_fft_xmask)
+      if (fft_masked_stores<T>(ctx, S.pl, NB))
         bds.xm = sphere_xmask(a.plans[s], &bds.xmw);
       const long ptot = sphere_ptot(a.plans[s]);
       for (int b0 = 0; b0 < a.nband[i]; b0 += NB) {

@@ -802,17 +802,9 @@ int rs_bounds(pp_ctx *ctx, const int *fftg, int nw, const int *G_dev, SphereBoun
   if (hb[nbnd - 1] || !bounds_filled(hb, fftg, nw))
     return PP_OK;  // aliasing, or a G set with holes: no pruning
   bd = SphereBounds{bnd, bnd + 2 * n0 * n1, bnd + 2 * n0 * n1 + 2 * n0, n0, n1, n2};
-  const int *yb = hb + 2 * n0 * n1, *xb = yb + 2 * n0;
   ctx->lines_host.clear();
-  for (int sx = xb[0]; sx <= xb[1]; sx++) {
-    const int x = (sx + n0) % n0;
-    for (int sy = yb[2 * x]; sy <= yb[2 * x + 1]; sy++)
-      ctx->lines_host.push_back(x * n1 + (sy + n1) % n1);
-  }
-  const int nzl = (int)ctx->lines_host.size();
-  for (int sx = xb[0]; sx <= xb[1]; sx++)
-    for (int z = 0; z < n2; z++)
-      ctx->lines_host.push_back(((sx + n0) % n0) * n2 + z);
+  long nzl = 0, nyl = 0;
+  push_pass_lines(hb, fftg, ctx->lines_host, nzl, nyl);
   if (!ctx->lines_host.empty()) {
     PP_TRY(ctx->lines.ensure(sizeof(int) * ctx->lines_host.size()));
     // the stream is idle (synchronised above); lines_host stays in the
@@ -820,9 +812,9 @@ int rs_bounds(pp_ctx *ctx, const int *fftg, int nw, const int *G_dev, SphereBoun
     PP_CHECK_HIP(hipMemcpyAsync(ctx->lines.p, ctx->lines_host.data(), sizeof(int) * ctx->lines_host.size(),
                                 hipMemcpyHostToDevice, ctx->stream));
     bd.zl = (const int *)ctx->lines.p;
-    bd.nzl = nzl;
-    bd.yl = (const int *)ctx->lines.p + nzl;
-    bd.nyl = (int)ctx->lines_host.size() - nzl;
+    bd.nzl = (int)nzl;
+    bd.yl = (const int *)ctx->lines.p + 2 * nzl;
+    bd.nyl = (int)nyl;
   }
   prune = true;
   return PP_OK;

@@ -618,6 +618,67 @@ def test_fixed_length_passes(ctx, fftg, precision, tol, wide):
     plan.close()
 
 
+FFT2_LENGTHS = (8, 10, 12, 14, 16, 18, 20, 24, 28, 30, 32, 36, 40, 42, 48, 50, 54, 56, 60, 64, 70, 72, 80, 84, 90, 96, 98,
+                100, 108, 112, 120, 126, 128, 140, 144, 150, 160, 162, 168, 180, 192, 196, 200, 210, 216, 224, 240, 250,
+                252, 256, 270, 280, 288, 300, 320, 324, 360)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_two_dft_pass_lengths(ctx, axis):
+    """Every axis length with a two-DFT pass, on each axis, FP64 and FP32, in
+    chunks of whole band groups, of a rounded-up band count and of fewer
+    bands than half a group (the staged passes): the transform of random
+    coefficients at random G against numpy.  A length-n FP64 (FP32)
+    transform rounds by a few log2(n) times 1.1e-16 (6e-8), normwise."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(axis)
+    for i, n in enumerate(FFT2_LENGTHS):
+        fftg = [10, 12, 14]
+        fftg[axis] = n
+        nb = (64, 16, 13, 3)[i % 4]
+        G = np.unique(rng.integers([-(m // 2 - 1) for m in fftg], [m // 2 for m in fftg], (60, 3)), axis=0).astype(np.int32)
+        C = (rng.standard_normal((nb, len(G))) + 1j * rng.standard_normal((nb, len(G)))).astype(np.complex64)
+        x = np.zeros((nb, *fftg), np.complex128)
+        x[:, G[:, 0], G[:, 1], G[:, 2]] = C
+        want = np.fft.ifftn(x, axes=(1, 2, 3), norm="forward")
+        out = torch.empty((nb, *fftg), dtype=torch.complex128, device="cuda")
+        Gd, Cd = torch.from_numpy(G).cuda(), torch.from_numpy(C).cuda()
+        torch.cuda.synchronize()
+        for precision, tol in (("fp64", 5e-15), ("fp32", 2e-6)):
+            B.fft3d(ctx, np.eye(3), fftg, Gd, Cd, out, precision)
+            err = normwise(out.cpu().numpy(), want)
+            assert err < tol, (fftg, nb, precision, err)
+
+
+@pytest.mark.parametrize("fftg", [(80, 54, 56), (54, 98, 30), (126, 28, 50), (36, 42, 150)])
+@pytest.mark.parametrize("nb", [45, 70])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 3e-6)])
+def test_two_dft_pass_pruned(ctx, fftg, nb, precision, tol):
+    """Pruned two-DFT passes with coverage-masked stores (the default) in
+    rounded-up band chunks, eager and in a work list, against the staged
+    passes storing every point; the bounds as test_two_dft_pass_lengths
+    for three axes."""
+    from pawpyseed_amd.core import batched as B
+    wl = synthetic.tiny_config(encut=150.0, fftg=fftg, nband=nb, kpts=[[0.25, -0.25, 0.1], [0, 0, 0.5]])
+    Gs, Cs = wl.ensure_gvecs(), wl.coefficients("S", nband=nb)
+    Cd, Gd, gofs, nw = device_inputs(Gs, Cs)
+    plan = B.SpherePlan(ctx, wl.lattice, wl.fftg, wl.frac_S, np.zeros(len(wl.frac_S), np.int32), [wl.species], precision)
+    outs = []
+    for fixed, xmask in ((0, 0), (1, -1)):
+        ctx.set_param("fft_fixed", fixed)
+        ctx.set_param("fft_xmask", xmask)
+        out = torch.full((2, nb, plan.ptot), np.nan, dtype=torch.complex128, device="cuda")
+        torch.cuda.synchronize()
+        B.setup_projections(ctx, plan, wl.kpts, gofs, Gd, Cd, out, precision)
+        outs.append(out.cpu().numpy())
+    multi = torch.full((2, nb, plan.ptot), np.nan, dtype=torch.complex128, device="cuda")
+    torch.cuda.synchronize()
+    B.setup_projections_multi(ctx, [plan], wl.kpts, gofs, Gd, [[Cd[0], Cd[1]]], [[multi[0], multi[1]]], precision)
+    assert normwise(outs[1], outs[0]) < tol
+    assert normwise(multi.cpu().numpy(), outs[0]) < tol
+    plan.close()
+
+
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-9), ("fp32", 1e-5)])
 def test_projections_g_set_with_holes(ctx, precision, tol):
     """A plane-wave list that is not a cutoff sphere (a random subset of
