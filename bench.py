@@ -722,9 +722,8 @@ def bench_aedensity(args, torch, B):
     # restricted to the plane-wave sphere as in the projection path (z:
     # coefficients in, populated z-lines out; y: populated rows of the
     # x-slab in, the slab out; x: the slab in, the whole grid out),
-    # augmentation: the table (16 P per sphere point) and a read-modify-write
-    # of the point's NB values, density emit: the chunk in, the density
-    # read and written
+    # augmentation and density in one pass: the chunk in, the density read
+    # and written, the table (8 P per sphere point)
     npts = int(np.prod(fine))
     n0, n1, n2 = fine
     NBc = 64
@@ -745,13 +744,13 @@ def bench_aedensity(args, torch, B):
             by.append(NBc * pb * n2 * (yrow + xs * n1))
             bz.append(NBc * pb * ((len(G) if prune else npts) + rows * n2))
         alg = {"fft_z": float(np.mean(bz)), "fft_y": float(np.mean(by)), "fft_x": float(np.mean(bx)),
-               "rs_augment": rs.npts * (16 * P + 2 * NBc * pb), "rs_emit": npts * (NBc * pb + 16)}
+               "rs_augment": npts * (NBc * pb + 16) + rs.npts * 8 * P}
         kr = {}
         for c, b in alg.items():
             kc = r["kernels"].get(c)
             if not kc:
                 continue
-            ms = kc[0] / nchunks  # per chunk (one launch per augmentation colour)
+            ms = kc[0] / nchunks  # per chunk
             kr[c] = {"bound": "hbm", "achieved": b / (ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                      "alg_bytes_per_chunk": b, "ms_per_chunk": ms, "ms_per_step": kc[0], "launches": kc[1]}
             kr[c]["frac"] = kr[c]["achieved"] / kr[c]["peak"]

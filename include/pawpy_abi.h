@@ -269,11 +269,13 @@ int pp_ctx_set_tuning(pp_ctx *ctx, int fft_bands, int fft_tile, int fft_prune,
  * point; -1, default: 1 when the x axis has a compiled pass, whose stores
  * the test costs nothing), "rs_kernel" (real-space
  * augmentation: 0 a site's coefficients in LDS, 1 in registers (up to 32
- * projectors per site), 2, default: tiles of points with their table rows
+ * projectors per site), 2: tiles of points with their table rows
  * in LDS and the coefficients in registers (up to 18 projectors per site;
- * else 0)), "rs_unroll" (1, 2 or 4,
+ * else 0), 3, default: blocks of 16 points along x on the FP64 matrix cores,
+ * densities included; 2 where a site box reaches past the neighbouring cells
+ * or the blocks' tables do not fit in memory), "rs_unroll" (1, 2 or 4,
  * default 4: sphere points of a wavefront in flight in the real-space
- * augmentation), "rs_prune" (1, default: the real-space FFT passes skip
+ * augmentation of rs_kernel 0 to 2), "rs_prune" (1, default: the real-space FFT passes skip
  * lines outside the plane-wave sphere), "multi_items" (1..64, default 8:
  * work items per launch of pp_setup_projections_multi), "gemm_planes"
  * (two-plane split GEMMs, PP_FP16X3 and PP_BF16X3: 1 one work-group per

@@ -522,7 +522,7 @@ int pp_ctx_set_param(pp_ctx *ctx, const char *name, int value) {
   else if (n == "fused")
     ctx->tune_fused = value != 0 ? 1 : 0;
   else if (n == "rs_kernel")
-    ctx->tune_rs_kernel = value < 0 ? 0 : value > 2 ? 2 : value;
+    ctx->tune_rs_kernel = value < 0 ? 0 : value > 3 ? 3 : value;
   else if (n == "rs_prune")
     ctx->tune_rs_prune = value != 0 ? 1 : 0;
   else if (n == "rs_unroll")

@@ -141,7 +141,7 @@ struct pp_ctx {
   int tune_fft_xcd = 0;         // 1: FFT pass work-groups in XCD-contiguous line ranges
   int tune_fft_fixed = 1;       // 1: two-DFT passes for the axis lengths that have one
   int tune_fused = 0;           // 1: x pass fused with the sphere sums where the plan allows
-  int tune_rs_kernel = 2;       // real-space augmentation: 0 LDS coefficients, 1 registers, 2 tiled
+  int tune_rs_kernel = 3;       // real-space augmentation: 0 LDS, 1 registers, 2 tiled, 3 blocks of x (MFMA)
   int tune_rs_unroll = 4;       // real-space augmentation: points of a wavefront in flight (1, 2, 4)
   int tune_rs_prune = 1;        // real-space FFT passes restricted to the plane-wave sphere's lines
   int tune_multi_items = 8;     // work items per launch of the multi-structure setup
@@ -151,6 +151,7 @@ struct pp_ctx {
   int slot = 0;                 // chunk buffer set in use (0 or 1)
   pp::DevBuf grid, grid2;       // band-fastest FFT chunk, one per slot
   pp::DevBuf partial, partial2; // sphere-sum partials, one per slot
+  pp::DevBuf rs_coef[2];  // real-space tile kernel: the chunk's site coefficients and axis phases, one per slot
   pp::DevBuf gidx;      // wrapped grid index per G
   pp::DevBuf phase;     // per-point Bloch phase of every k
   pp::DevBuf gemm_ws;   // split-K partials

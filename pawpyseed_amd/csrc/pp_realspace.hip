@@ -9,68 +9,37 @@
 // |d| < rmax_s (the last point of the species' wave grid), T the lattice
 // vector that wraps the point into the cell.
 //
-// Plan (pp_rs_plan_create): per site the box points inside its sphere
-// (count, host scan, ordered fill; the order of the reference's i-j-k
-// loops) and a complex table of the partial-wave values per point and
-// projector, independent of k and band.  Sites whose spheres can share a
-// grid point get different colours, so one launch per colour adds the
-// augmentation with plain read-modify-writes (deterministic); when a
-// site's box wraps onto itself the plan uses atomic adds instead.
+// Plan (pp_rs_plan_create): per site the count of box points inside its
+// sphere, in blocks of candidates.  Sites whose spheres can share a
+// grid point get different colours; a site's box may wrap onto itself
+// (atomic).  The augmentation kernel in use builds its own lists and tables,
+// independent of k and band, on its first call: pp_rstile.hip, or for the
+// per-site kernels here the points (ordered fill; the order of the
+// reference's i-j-k loops) and a complex table of the partial-wave values per
+// point and projector.
 //
 // Per band chunk (pp_realspace_batched; two chunks in flight on two
 // streams): scatter + backward FFT into the band-fastest chunk (the
-// projection path's kernels), augmentation added
-// in the chunk with the phase e^{-2 pi i k.(r_unwrapped - R)} / scale so
-// that the emit kernel's common factor scale e^{2 pi i k.r} restores the
-// reference's terms, then either the band-major states (LDS transpose,
-// with or without the Bloch phase, i.e. remove_phase) or the weighted
-// density sum_b w_b |psi_b|^2 (ae_state_density / ae_chg_density,
-// density.c:158-179).
+// projection path's kernels), then the blocks-of-x kernel adds the
+// augmentation and gives the weighted density sum_b w_b |psi_b|^2
+// (ae_state_density / ae_chg_density, density.c:158-179), or the finished
+// states for the band-major copy (LDS transpose).  The per-site kernels,
+// which need no tables padded to blocks and take boxes of any reach, add the
+// augmentation in the chunk, one launch per colour with plain
+// read-modify-writes (atomic adds where a box wraps onto itself), with the
+// phase e^{-2 pi i k.(r_unwrapped - R)} / scale so that the emit kernel's
+// common factor scale e^{2 pi i k.r} restores the reference's terms; the
+// states (with or without the Bloch phase, i.e. remove_phase) or the density
+// follow in a pass of their own.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
 #include <vector>
 
-#include "pp_geom.h"
-#include "pp_internal.h"
+#include "pp_realspace.h"
 
 namespace pp {
-
-struct RsSite {
-  double R[3];
-  double rmax;
-  int c[3], g[3];
-  int nproj, nchan, n;  // projectors, channels, wave-grid points
-  int chan_off;         // first channel of the species in chan_l
-  int proj_off;         // first projection of the site
-  long spl_off;         // species block: x[n], then f, b, c, d (n each) per channel
-};
-
-struct RsLat {
-  double m[9];
-};
-
-struct RsWeights {
-  double w[64];
-};
-
-// candidate c of a site's box -> unwrapped (i, j, k), k fastest (the
-// reference's loop order, density.c:272-276)
-__device__ __forceinline__ void rs_cand(const RsSite &s, int c, int &i, int &j, int &k) {
-  const int w1 = 2 * s.g[1] + 1, w2 = 2 * s.g[2] + 1;
-  k = c % w2 - s.g[2] + s.c[2];
-  j = (c / w2) % w1 - s.g[1] + s.c[1];
-  i = c / (w1 * w2) - s.g[0] + s.c[0];
-}
-
-// unwrapped box vector r - R in cartesian coordinates (density.c:277-281)
-__device__ __forceinline__ double rs_vec(const RsSite &s, const RsLat &L, int f0, int f1, int f2, int i, int j, int k,
-                                         double *v) {
-  double f[3] = {(double)i / f0 - s.R[0], (double)j / f1 - s.R[1], (double)k / f2 - s.R[2]};
-  d_frac_to_cart(f, L.m, v);
-  return sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-}
 
 __global__ __launch_bounds__(256) void k_rs_count(const RsSite *__restrict__ geo, RsLat L, int f0, int f1, int f2,
                                                   int nblk, int *__restrict__ blkcnt) {
@@ -135,40 +104,18 @@ __global__ __launch_bounds__(256) void k_rs_values(const RsSite *__restrict__ ge
   const int4 pt = pts[p0 + q];
   double v[3];
   const double r = rs_vec(g, L, f0, f1, f2, pt.y, pt.z, pt.w, v);
-  double theta = 0.0, phi = 0.0;
-  if (r != 0.0) {
-    theta = acos(v[2] / r);
-    if (r - fabs(v[2]) != 0.0)
-      phi = acos(v[0] / sqrt(v[0] * v[0] + v[1] * v[1]));
-    if (v[1] < 0)
-      phi = 2.0 * M_PI - phi;
-  }
-  const double ct = cos(theta);
-  const int n = g.n;
   const double *x = spl + g.spl_off;
-  int id = 0;
-  double t = 0.0;
-  const bool below = r < x[0], beyond = r > x[n - 1];
-  if (!below && !beyond) {
-    id = (int)(log(r / x[0]) / log(x[1] / x[0]));
-    if (id > n - 2)
-      id = n - 2;
-    t = r - x[id];
-  }
-  const double rdiv = below ? x[0] : r;
+  const RsPoint rp = rs_point(x, g.n, v, r);
   cplx<double> *out = tab + tab_off[s] + (long)q * g.nproj;
   int p = 0;
   for (int ch = 0; ch < g.nchan; ch++) {
     const int l = chan_l[g.chan_off + ch];
-    const double *fc = x + (long)n * (1 + 4 * ch);
-    const double *bc = fc + n, *cc = bc + n, *dc = cc + n;
-    double radial = beyond ? 0.0 : below ? fc[0] : fc[id] + t * (bc[id] + t * (cc[id] + t * dc[id]));
-    radial /= rdiv;
+    const double radial = rs_radial(x, g.n, ch, rp);
     for (int m = -l; m <= l; m++, p++) {
       const double norm = sqrt((2 * l + 1) / (4.0 * M_PI) * d_fact(l - m) / d_fact(l + m));
-      const double a = norm * d_legendre(l, m, ct) * radial;
+      const double a = norm * d_legendre(l, m, rp.ct) * radial;
       double sn, cs;
-      sincos(m * phi, &sn, &cs);
+      sincos(m * rp.phi, &sn, &cs);
       out[p] = mk<double>(a * cs, a * sn);
     }
   }
@@ -529,19 +476,6 @@ __global__ __launch_bounds__(256) void k_rs_add(double *__restrict__ d, const do
 
 using namespace pp;
 
-struct pp_rsplan {
-  pp_ctx *ctx = nullptr;
-  double lattice[9];
-  int fftg[3];
-  int nsites = 0, ptot = 0, pmax = 0;
-  long npts = 0;
-  bool atomic = false;
-  std::vector<int> proj_off, site_pt;
-  std::vector<int> color_off, color_sites, color_maxpts;
-  DevBuf d_geo, d_pts, d_tab, d_tab_off, d_site_pt, d_colors, d_spl, d_chan_l;
-  DevBuf dens2;  // densities of the second stream's chunks
-};
-
 namespace {
 
 double cross_norm(const double *a, const double *b) {
@@ -682,9 +616,8 @@ extern "C" int pp_rs_plan_create(pp_ctx *ctx, pp_rsplan **out, const double *lat
   memcpy(L.m, lattice, sizeof(L.m));
   rp->site_pt.assign(num_sites + 1, 0);
   if (num_sites) {
-    DevBuf cnt, boff;
-    if ((st = cnt.ensure(sizeof(int) * (size_t)num_sites * nblk)) ||
-        (st = boff.ensure(sizeof(long) * (size_t)num_sites * nblk)))
+    DevBuf cnt;
+    if ((st = cnt.ensure(sizeof(int) * (size_t)num_sites * nblk)))
       return st;
     hipLaunchKernelGGL(k_rs_count, dim3(nblk, num_sites), dim3(256), 0, sm, (const RsSite *)rp->d_geo.p, L, fftg[0],
                        fftg[1], fftg[2], nblk, (int *)cnt.p);
@@ -703,33 +636,8 @@ extern "C" int pp_rs_plan_create(pp_ctx *ctx, pp_rsplan **out, const double *lat
       rp->site_pt[s + 1] = (int)acc;
     }
     rp->npts = acc;
-    if ((st = rp->d_pts.ensure(sizeof(int4) * std::max(1L, acc))))
-      return st;
-    PP_CHECK_HIP(hipMemcpyAsync(boff.p, ho.data(), sizeof(long) * ho.size(), hipMemcpyHostToDevice, sm));
-    hipLaunchKernelGGL(k_rs_fill, dim3(nblk, num_sites), dim3(256), 0, sm, (const RsSite *)rp->d_geo.p, L, fftg[0],
-                       fftg[1], fftg[2], nblk, (const long *)boff.p, (int4 *)rp->d_pts.p);
-    PP_CHECK_HIP(hipGetLastError());
-    // value table
-    std::vector<long> toff(num_sites + 1, 0);
-    int maxp = 1;
-    for (int s = 0; s < num_sites; s++) {
-      const int np = rp->site_pt[s + 1] - rp->site_pt[s];
-      toff[s + 1] = toff[s] + (long)np * geo[s].nproj;
-      maxp = std::max(maxp, np);
-    }
-    if ((st = rp->d_tab.ensure(sizeof(cplx<double>) * std::max(1L, toff[num_sites]))) ||
-        (st = rp->d_tab_off.ensure(sizeof(long) * (num_sites + 1))) ||
-        (st = rp->d_site_pt.ensure(sizeof(int) * (num_sites + 1))))
-      return st;
-    PP_CHECK_HIP(
-        hipMemcpyAsync(rp->d_tab_off.p, toff.data(), sizeof(long) * toff.size(), hipMemcpyHostToDevice, sm));
-    PP_CHECK_HIP(hipMemcpyAsync(rp->d_site_pt.p, rp->site_pt.data(), sizeof(int) * rp->site_pt.size(),
-                                hipMemcpyHostToDevice, sm));
-    hipLaunchKernelGGL(k_rs_values, dim3((maxp + 255) / 256, num_sites), dim3(256), 0, sm,
-                       (const RsSite *)rp->d_geo.p, L, fftg[0], fftg[1], fftg[2], (const int *)rp->d_site_pt.p,
-                       (const int4 *)rp->d_pts.p, (const long *)rp->d_tab_off.p, (const double *)rp->d_spl.p,
-                       (const int *)rp->d_chan_l.p, (cplx<double> *)rp->d_tab.p);
-    PP_CHECK_HIP(hipGetLastError());
+    rp->blkoff = ho;
+    rp->nblk = nblk;
     // colours (one launch per colour; a single "colour" with atomics when
     // a box wraps onto itself)
     std::vector<int> colour;
@@ -757,7 +665,56 @@ extern "C" int pp_rs_plan_create(pp_ctx *ctx, pp_rsplan **out, const double *lat
                                 hipMemcpyHostToDevice, sm));
     PP_CHECK_HIP(hipStreamSynchronize(sm));  // host staging buffers end here
   }
+  // x-line blocks as an int counts them, and the kernel's grid
+  const long nxb = (fftg[0] + 15) / 16;
+  rp->tile_ok = num_sites > 0 && rp->ptot > 0 && nxb * fftg[1] * fftg[2] < (1L << 31);
+  for (const RsSite &g : geo)
+    for (int q = 0; q < 3; q++)
+      if (g.c[q] - g.g[q] < -fftg[q] || g.c[q] + g.g[q] >= 2 * fftg[q])
+        rp->tile_ok = false;
+  rp->geo = std::move(geo);
   *out = hold.release();
+  return PP_OK;
+}
+
+// The per-site kernels' points (box order) and complex value table.
+static int rs_sites_ensure(pp_ctx *ctx, pp_rsplan *rp) {
+  std::lock_guard<std::mutex> lk(rp->build_mu);
+  if (rp->sites_built || rp->nsites == 0)
+    return PP_OK;
+  const int ns = rp->nsites, *fftg = rp->fftg;
+  hipStream_t sm = ctx->stream;
+  RsLat L;
+  memcpy(L.m, rp->lattice, sizeof(L.m));
+  int st = PP_OK;
+  DevBuf boff;
+  if ((st = boff.ensure(sizeof(long) * rp->blkoff.size())) ||
+      (st = rp->d_pts.ensure(sizeof(int4) * std::max(1L, rp->npts))))
+    return st;
+  PP_CHECK_HIP(hipMemcpyAsync(boff.p, rp->blkoff.data(), sizeof(long) * rp->blkoff.size(), hipMemcpyHostToDevice, sm));
+  hipLaunchKernelGGL(k_rs_fill, dim3(rp->nblk, ns), dim3(256), 0, sm, (const RsSite *)rp->d_geo.p, L, fftg[0], fftg[1],
+                     fftg[2], rp->nblk, (const long *)boff.p, (int4 *)rp->d_pts.p);
+  PP_CHECK_HIP(hipGetLastError());
+  std::vector<long> toff(ns + 1, 0);
+  int maxp = 1;
+  for (int s = 0; s < ns; s++) {
+    const int np = rp->site_pt[s + 1] - rp->site_pt[s];
+    toff[s + 1] = toff[s] + (long)np * rp->geo[s].nproj;
+    maxp = std::max(maxp, np);
+  }
+  if ((st = rp->d_tab.ensure(sizeof(cplx<double>) * std::max(1L, toff[ns]))) ||
+      (st = rp->d_tab_off.ensure(sizeof(long) * (ns + 1))) || (st = rp->d_site_pt.ensure(sizeof(int) * (ns + 1))))
+    return st;
+  PP_CHECK_HIP(hipMemcpyAsync(rp->d_tab_off.p, toff.data(), sizeof(long) * toff.size(), hipMemcpyHostToDevice, sm));
+  PP_CHECK_HIP(hipMemcpyAsync(rp->d_site_pt.p, rp->site_pt.data(), sizeof(int) * rp->site_pt.size(),
+                              hipMemcpyHostToDevice, sm));
+  hipLaunchKernelGGL(k_rs_values, dim3((maxp + 255) / 256, ns), dim3(256), 0, sm, (const RsSite *)rp->d_geo.p, L,
+                     fftg[0], fftg[1], fftg[2], (const int *)rp->d_site_pt.p, (const int4 *)rp->d_pts.p,
+                     (const long *)rp->d_tab_off.p, (const double *)rp->d_spl.p, (const int *)rp->d_chan_l.p,
+                     (cplx<double> *)rp->d_tab.p);
+  PP_CHECK_HIP(hipGetLastError());
+  PP_CHECK_HIP(hipStreamSynchronize(sm));  // host staging buffers end here
+  rp->sites_built = true;
   return PP_OK;
 }
 
@@ -778,6 +735,14 @@ extern "C" int pp_rs_plan_info(pp_rsplan *rp, int *total_projs, long *total_poin
     memcpy(proj_off, rp->proj_off.data(), sizeof(int) * rp->proj_off.size());
   return PP_OK;
 }
+
+namespace pp {
+// the tile kernel (pp_rstile.hip)
+int rs_tile_ensure(pp_ctx *ctx, pp_rsplan *rp, bool *use);
+template <typename T>
+int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, const cplx<double> *proj, long ldp,
+                int remove_phase, bool states, const double *wts, double *dens, cplx<T> *grid);
+}  // namespace pp
 
 namespace {
 
@@ -824,13 +789,24 @@ template <typename T>
 int rs_chunk(pp_ctx *ctx, pp_rsplan *rp, FftPlan *pl, const double *kf, int nw, const int *gidx,
              const cplx<float> *C, long ldc, int nbc, const cplx<double> *proj, long ldp, int remove_phase,
              cplx<double> *states, long ldo, const double *wts, double *dens, const SphereBounds *bd,
-             cplx<T> *grid) {
-  const int NB = nbc;
+             cplx<T> *grid, int NB, bool tiles) {
   const long npts = (long)rp->fftg[0] * rp->fftg[1] * rp->fftg[2];
   PP_TRY(fft_chunk<T>(ctx, pl, grid, NB, nw, gidx, C, ldc, nbc, bd));
-  const double scl = 1.0 / sqrt(det3(rp->lattice));
+  double scl = 1.0 / sqrt(det3(rp->lattice));
   hipEvent_t ev;
-  if (rp->nsites && rp->ptot) {
+  int phase_on = remove_phase ? 0 : 1;
+  if (tiles) {
+    // augmentation and density (or the finished states, scale and phase
+    // included) in one pass over the chunk
+    tbegin(ctx, K_RS_AUG, &ev);
+    const int st = rs_tile_run<T>(ctx, rp, kf, nbc, NB, proj, ldp, remove_phase, states != nullptr, wts, dens, grid);
+    tend(ctx, K_RS_AUG, ev);
+    PP_TRY(st);
+    if (!states)
+      return PP_OK;
+    scl = 1.0;
+    phase_on = 0;
+  } else if (rp->nsites && rp->ptot) {
     tbegin(ctx, K_RS_AUG, &ev);
     const int ppb = 64;
     const size_t lds = sizeof(cplx<double>) * 64 * (size_t)std::max(1, rp->pmax);
@@ -844,7 +820,7 @@ int rs_chunk(pp_ctx *ctx, pp_rsplan *rp, FftPlan *pl, const double *kf, int nw, 
                      (const RsSite *)rp->d_geo.p, sites, (const int *)rp->d_site_pt.p, (const int4 *)rp->d_pts.p,   \
                      (const long *)rp->d_tab_off.p, (const cplx<double> *)rp->d_tab.p, proj, ldp, kf[0], kf[1],      \
                      kf[2], 1.0 / scl, rp->fftg[0], rp->fftg[1], rp->fftg[2], ppb)
-      if (rp->pmax <= 18 && ctx->tune_rs_kernel == 2 && !rp->atomic) {
+      if (rp->pmax <= 18 && ctx->tune_rs_kernel >= 2 && !rp->atomic) {
         const size_t tl = (sizeof(cplx<double>) * ((size_t)ppb * rp->pmax + ppb) + sizeof(int) * ppb);
         const int u = ctx->tune_rs_unroll;
         if (u >= 4)
@@ -900,11 +876,11 @@ int rs_chunk(pp_ctx *ctx, pp_rsplan *rp, FftPlan *pl, const double *kf, int nw, 
   tbegin(ctx, K_RS_EMIT, &ev);
   if (states) {
     hipLaunchKernelGGL(k_rs_state<T>, dim3((unsigned)((npts + RS_TP - 1) / RS_TP)), dim3(256), 0, ctx->stream, grid,
-                       NB, nbc, npts, scl, rp->fftg[0], rp->fftg[1], rp->fftg[2], kf[0], kf[1], kf[2],
-                       remove_phase ? 0 : 1, states, ldo);
+                       NB, nbc, npts, scl, rp->fftg[0], rp->fftg[1], rp->fftg[2], kf[0], kf[1], kf[2], phase_on,
+                       states, ldo);
     PP_CHECK_HIP(hipGetLastError());
   }
-  if (dens) {
+  if (dens && !tiles) {
     RsWeights W;
     for (int b = 0; b < 64; b++)
       W.w[b] = b < nbc ? wts[b] : 0.0;
@@ -940,8 +916,14 @@ extern "C" int pp_realspace_batched(pp_ctx *ctx, pp_rsplan *rp, const double *kf
   FftPlan *pl = nullptr;
   PP_TRY(get_fft_plan(ctx, rp->fftg, &pl));
   const bool f64 = precision == PP_FP64;
-  const int nbmax = std::min(64, nband);
+  const int group = f64 ? 8 : 16;
+  const int nbmax = chunk_bands(nband, 0, group);
   const size_t csz = f64 ? sizeof(cplx<double>) : sizeof(cplx<float>);
+  bool tiles = ctx->tune_rs_kernel == 3;
+  if (tiles)
+    PP_TRY(rs_tile_ensure(ctx, rp, &tiles));
+  if (!tiles && rp->ptot)
+    PP_TRY(rs_sites_ensure(ctx, rp));
   PP_TRY(ctx->grid.ensure(csz * (size_t)npts * nbmax));
   PP_TRY(ctx->gidx.ensure(sizeof(int) * (size_t)std::max(1, nw)));
   PP_TRY(compute_gidx(ctx, rp->fftg, nw, G_dev, (int *)ctx->gidx.p));
@@ -950,9 +932,9 @@ extern "C" int pp_realspace_batched(pp_ctx *ctx, pp_rsplan *rp, const double *kf
   PP_TRY(rs_bounds(ctx, rp->fftg, nw, G_dev, bd, prune));
   // chunks to run (a density-only call skips chunks whose weights are all 0)
   std::vector<int> starts;
-  for (int b0 = 0; b0 < nband; b0 += 64) {
+  for (int b0 = 0; b0 < nband; b0 += nbmax) {
     bool any = !density_dev || states_dev;
-    for (int b = 0; b < std::min(64, nband - b0) && !any; b++)
+    for (int b = 0; b < std::min(nbmax, nband - b0) && !any; b++)
       any = weights[b0 + b] != 0.0;
     if (any)
       starts.push_back(b0);
@@ -985,7 +967,8 @@ extern "C" int pp_realspace_batched(pp_ctx *ctx, pp_rsplan *rp, const double *kf
   int st = PP_OK;
   for (size_t c = 0; c < starts.size() && st == PP_OK; c++) {
     const int b0 = starts[c];
-    const int nbc = std::min(64, nband - b0);
+    const int nbc = std::min(nbmax, nband - b0);
+    const int NB = nbmax % group ? nbc : (nbc + group - 1) / group * group;
     const int sl = two ? (int)(c & 1) : 0;
     ctx->stream = streams[sl];
     ctx->slot = sl;
@@ -997,10 +980,10 @@ extern "C" int pp_realspace_batched(pp_ctx *ctx, pp_rsplan *rp, const double *kf
     const double *W = density_dev ? weights + b0 : nullptr;
     if (f64)
       st = rs_chunk<double>(ctx, rp, pl, kfrac, nw, (const int *)ctx->gidx.p, C, ldc, nbc, P, ldp, remove_phase, S,
-                            ldo, W, dens, prune ? &bd : nullptr, (cplx<double> *)grid);
+                            ldo, W, dens, prune ? &bd : nullptr, (cplx<double> *)grid, NB, tiles);
     else
       st = rs_chunk<float>(ctx, rp, pl, kfrac, nw, (const int *)ctx->gidx.p, C, ldc, nbc, P, ldp, remove_phase, S,
-                           ldo, W, dens, prune ? &bd : nullptr, (cplx<float> *)grid);
+                           ldo, W, dens, prune ? &bd : nullptr, (cplx<float> *)grid, NB, tiles);
   }
   ctx->stream = streams[0];
   ctx->slot = 0;

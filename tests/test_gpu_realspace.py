@@ -283,6 +283,51 @@ def test_augmentation_variants_agree(ctx, kernel, unroll):
     plan.close()
 
 
+@pytest.mark.parametrize("name,nband", [("cubic", 1), ("cubic", 17), ("cubic", 33), ("skewed", 64), ("skewed", 70),
+                                        ("wrapping", 13)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_blocks_of_x_agree_with_the_site_kernels(ctx, name, nband, precision):
+    """The blocks-of-x augmentation (rs_kernel 3) against the per-site
+    kernels: grids that end inside a block, partial band groups, one and two
+    groups per step, several chunks, spheres on faces and boxes that wrap;
+    states with and without their phase and the density, zero weights among
+    the bands.  Both add the same FP64 terms to the same transform in another
+    order, a few roundings of 1.1e-16; an FP32 chunk rounds the sum once more
+    (6e-8 of its value, and as much where sites share points)."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(23)
+    lat, fftg, k, G, C, species, labels, coords = _case(name, nband, rng)
+    plan = B.RealspacePlan(ctx, lat, fftg, coords, labels, species)
+    proj = torch.from_numpy(rng.normal(size=(nband, plan.ptot)) + 1j * rng.normal(size=(nband, plan.ptot))).cuda()
+    Ch = np.zeros((nband, -(-len(G) // 64) * 64), np.complex64)
+    Ch[:, :len(G)] = C
+    Cd, Gd = torch.from_numpy(Ch).cuda(), torch.from_numpy(np.ascontiguousarray(G, np.int32)).cuda()
+    w = rng.uniform(0.1, 1.0, nband)
+    w[nband // 2 + 1:] = 0.0
+    tol = 1e-14 if precision == "fp64" else 4e-7
+    got = {}
+    try:
+        for kern in (2, 3):
+            ctx.set_param("rs_kernel", kern)
+            for remove in (False, True):
+                for st in (False, True):
+                    out = torch.zeros((nband,) + tuple(fftg), dtype=torch.complex128, device="cuda") if st else None
+                    dens = torch.zeros(tuple(fftg), dtype=torch.float64, device="cuda")
+                    B.realspace_states(ctx, plan, k, Gd, Cd, proj, states_out=out, density_out=dens, weights=w,
+                                       remove_phase=remove, precision=precision)
+                    got[kern, remove, st] = (dens.cpu().numpy(), out.cpu().numpy() if st else None)
+    finally:
+        ctx.set_param("rs_kernel", 3)
+    for remove in (False, True):
+        for st in (False, True):
+            (d2, s2), (d3, s3) = got[2, remove, st], got[3, remove, st]
+            assert normwise(d3, d2) < tol, (remove, st)
+            if st:
+                for b in range(nband):
+                    assert normwise(s3[b], s2[b]) < tol, (remove, b)
+    plan.close()
+
+
 def test_wrapping_boxes_fp32_atomics(ctx):
     """Atomic adds of the FP32 chunk where site boxes wrap onto themselves."""
     from pawpyseed_amd.core import batched as B
