@@ -384,6 +384,36 @@ __device__ __forceinline__ f32x4 ld4(const float *x, long off, long left) {
   }
 }
 
+// Quarter `mi` of the staging of 8 reals of a row: one pair is split; the
+// last quarter stores the planes (plane stride ls, 16-bit words) and loads
+// the values `off` reals into the row.  Planes operands (CVT false) are
+// stored and loaded in the last quarter alone.
+template <bool WH, bool CVT, bool F16, int NT, int HP>
+__device__ __forceinline__ void stage(int mi, f32x4 &f0, f32x4 &f1, u32x4 (&g)[NT][HP], int q, float sc,
+                                      const float *x, const unsigned short *p, long sp, long off, long left,
+                                      unsigned short *lds, int ls) {
+  if constexpr (CVT) {
+    unsigned w[2];
+    const f32x4 &f = mi < 2 ? f0 : f1;
+    split_pair<2, F16>(f32x2{f[2 * (mi & 1)], f[2 * (mi & 1) + 1]}, sc, w);
+    g[0][q][mi] = w[0];
+    g[1][q][mi] = w[1];
+  }
+  if (mi == 3) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      *reinterpret_cast<u32x4 *>(lds + t * ls) = g[t][q];
+    if constexpr (CVT) {
+      f0 = ld4<WH>(x, off + q * 8, left);
+      f1 = ld4<WH>(x, off + q * 8 + 4, left);
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+        g[t][q] = *reinterpret_cast<const u32x4 *>(p + t * sp + off + q * 8);
+    }
+  }
+}
+
 // Operands: CVT false -- NT chunk-major planes of 16-bit values
 // (k_split_planes): rows of lda = ldb = 2048 reals per chunk block, block
 // stride cs, plane stride sp; CVT true (two-plane
@@ -511,7 +541,18 @@ __global__ __launch_bounds__(128 * TMW) __attribute__((amdgpu_waves_per_eu(WPE, 
   const int sub = lane & 15, kq = lane >> 4;
   // step s: compute from LDS buffer s & 1 while step s + 1 goes from
   // registers into the other buffer and step s + 2 is loaded (the last
-  // steps re-load the chunk's last step and fill a buffer no one reads)
+  // steps re-load the chunk's last step and fill a buffer no one reads).  A
+  // step is NBLK blocks of 16 columns; beside each block one unit is staged
+  // (a row pass of A or B, piece of 8 reals of the step): a quarter of it
+  // after every row tile's products, held there by the scheduling barriers,
+  // so that the split's vector instructions issue while the matrix core works
+  // on the wavefront's own products.  Split after all of a step's products, the
+  // GEMM of 512 x 512 bands, K = 116,329, took 843 (fp16x3), 709 (bf16x3) and
+  // 1616 us (bf16x6) where it takes 785, 660 and 1440.  Half of the cycles
+  // are MFMA, at 1.7 to 1.9 of 2.4 GHz: neither operands that hit the L2
+  // nor LDS rows without bank conflicts (18% of the cycles) changed the time.
+  constexpr int NU = (RA + RB) * HP, NBLK = 4 * (KS / 32);
+  static_assert(NU <= NBLK, "at most one unit per block of columns");
 #define PP_KLOOP(WH)                                                                                             \
   {                                                                                                              \
     PP_FETCH(0, WH);                                                                                             \
@@ -520,28 +561,46 @@ __global__ __launch_bounds__(128 * TMW) __attribute__((amdgpu_waves_per_eu(WPE, 
     PP_FETCH(1, WH);                                                                                             \
     for (int s = 0; s < nsteps; s++) {                                                                           \
       const int buf = s & 1;                                                                                     \
-      _Pragma("unroll") for (int kk = 0; kk < KS; kk += 32) {                                                    \
-        const int kc = kk + kq * 8;                                                                              \
-        u32x4 a[NT][4];                                                                                          \
-        _Pragma("unroll") for (int t = 0; t < NT; t++) _Pragma("unroll") for (int mi = 0; mi < 4; mi++) a[t][mi] = \
-            *reinterpret_cast<const u32x4 *>(&As[buf][t][wm * 64 + mi * 16 + sub][kc]);                        \
-        _Pragma("unroll") for (int nj = 0; nj < 4; nj++) {                                                       \
-          const int col = wn * 64 + nj * 16 + sub;                                                               \
-          u32x4 b[NT], q[NT];                                                                                    \
-          _Pragma("unroll") for (int t = 0; t < NT; t++) {                                                       \
-            b[t] = *reinterpret_cast<const u32x4 *>(&Bs[buf][t][col][kc]);                                       \
-            q[t] = qswap(b[t]);                                                                                  \
+      const long off_ = (long)min(s + 2, nsteps - 1) * KS;                                                       \
+      u32x4 a[NT][4], bn[NT];                                                                                    \
+      _Pragma("unroll") for (int t = 0; t < NT; t++) bn[t] =                                                     \
+          *reinterpret_cast<const u32x4 *>(&Bs[buf][t][wn * 64 + sub][kq * 8]);                                  \
+      _Pragma("unroll") for (int blk = 0; blk < NBLK; blk++) {                                                   \
+        const int kc = blk / 4 * 32 + kq * 8, nj = blk % 4;                                                      \
+        if (nj == 0) {                                                                                           \
+          _Pragma("unroll") for (int t = 0; t < NT; t++) _Pragma("unroll") for (int mi = 0; mi < 4; mi++)        \
+              a[t][mi] = *reinterpret_cast<const u32x4 *>(&As[buf][t][wm * 64 + mi * 16 + sub][kc]);             \
+        }                                                                                                        \
+        u32x4 b[NT], q[NT];                                                                                      \
+        _Pragma("unroll") for (int t = 0; t < NT; t++) {                                                         \
+          b[t] = bn[t];                                                                                          \
+          q[t] = qswap(b[t]);                                                                                    \
+        }                                                                                                        \
+        if (blk + 1 < NBLK) {                                                                                    \
+          _Pragma("unroll") for (int t = 0; t < NT; t++) bn[t] = *reinterpret_cast<const u32x4 *>(               \
+              &Bs[buf][t][wn * 64 + (blk + 1) % 4 * 16 + sub][(blk + 1) / 4 * 32 + kq * 8]);                     \
+        }                                                                                                        \
+        _Pragma("unroll") for (int mi = 0; mi < 4; mi++) {                                                       \
+          _Pragma("unroll") for (int d = NT - 1; d >= 0; d--) _Pragma("unroll") for (int i = d; i >= 0; i--) {   \
+            cr[mi][nj] = mfma16<F16>(a[i][mi], b[d - i], cr[mi][nj]);                                            \
+            ci[mi][nj] = mfma16<F16>(a[i][mi], q[d - i], ci[mi][nj]);                                            \
           }                                                                                                      \
-          _Pragma("unroll") for (int mi = 0; mi < 4; mi++) {                                                     \
-            _Pragma("unroll") for (int d = NT - 1; d >= 0; d--) _Pragma("unroll") for (int i = d; i >= 0; i--) { \
-              cr[mi][nj] = mfma16<F16>(a[i][mi], b[d - i], cr[mi][nj]);                                          \
-              ci[mi][nj] = mfma16<F16>(a[i][mi], q[d - i], ci[mi][nj]);                                          \
-            }                                                                                                    \
+          if (blk < NU) {                                                                                        \
+            const int h_ = blk / HP, q_ = blk % HP;                                                              \
+            if (h_ < RA)                                                                                         \
+              stage<WH, CVT, F16, NT, HP>(                                                                       \
+                    mi, fa[h_ % RA][2 * q_], fa[h_ % RA][2 * q_ + 1], ga[h_ % RA], q_, sa[h_ % RA],              \
+                    xa[h_ % RA], pa[h_ % RA], sp, off_, nreal_left,                                              \
+                    &As[buf ^ 1][0][h_ % RA * RS + lrow][part * (KS / 4) + q_ * 8], TM * LS);                    \
+            else                                                                                                 \
+              stage<WH, CVT, F16, NT, HP>(                                                                       \
+                    mi, fb[(h_ - RA) % RB][2 * q_], fb[(h_ - RA) % RB][2 * q_ + 1], gb[(h_ - RA) % RB],          \
+                    q_, sb[(h_ - RA) % RB], xb[(h_ - RA) % RB], pb[(h_ - RA) % RB], sp, off_, nreal_left,        \
+                    &Bs[buf ^ 1][0][(h_ - RA) % RB * RS + lrow][part * (KS / 4) + q_ * 8], 128 * LS);            \
           }                                                                                                      \
+          __builtin_amdgcn_sched_barrier(0);                                                                     \
         }                                                                                                        \
       }                                                                                                          \
-      PP_STASH(buf ^ 1);                                                                                         \
-      PP_FETCH(min(s + 2, nsteps - 1), WH);                                                                      \
       __syncthreads();                                                                                           \
     }                                                                                                            \
   }
