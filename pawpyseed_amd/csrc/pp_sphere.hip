@@ -56,125 +56,107 @@ __device__ __forceinline__ bool inside(const SiteGeo &s, const Lat9 &L, const in
   return sqrt(cv[0] * cv[0] + cv[1] * cv[1] + cv[2] * cv[2]) < s.R0;
 }
 
-// Candidate c of a site's box is inside its sphere.
-__device__ __forceinline__ bool cand_inside(const SiteGeo &s, const Lat9 &L, const int *fftg, int c, double *cv) {
+// The lists of a site are made by one work-group of SITE_W wavefronts, which
+// take 63 consecutive candidates at a time and lane 0 the one before them, so
+// that a wavefront's two ballots hold its inside flags and segment starts and
+// only the counts cross wavefronts.  Bound by the chain of tiles of a site:
+// 256 threads with shared flags and scans took 28 us to count and 88 to fill
+// for 215 sites of 5,900 points where these take 21 and 35, and for 8 sites 6
+// and 14 where these take 4 and 6.  A segment starts at an inside candidate
+// that is the first of its line or follows an outside one.
+constexpr int SITE_W = 16;
+struct SiteBallot {
+  unsigned long long in, start;  // of lanes 1..63
+  bool mine, first;              // the lane's own bits
   int i, j, k;
-  box_ijk(s, c, i, j, k);
-  return inside(s, L, fftg, i, j, k, cv);
+  double cv[3];
+};
+__device__ __forceinline__ SiteBallot site_ballot(const SiteGeo &s, const Lat9 &L, const int *fftg, int c0, int ncand) {
+  SiteBallot q;
+  const int lane = threadIdx.x & 63, c = c0 + lane - 1;
+  bool in = false;
+  if (c >= 0 && c < ncand) {
+    box_ijk(s, c, q.i, q.j, q.k);
+    in = inside(s, L, fftg, q.i, q.j, q.k, q.cv);
+  }
+  const unsigned long long m = __ballot(in);
+  q.mine = in && lane > 0;
+  q.first = q.mine && (c % (2 * s.g[0] + 1) == 0 || !(m >> (lane - 1) & 1));
+  q.in = m & ~1ull;
+  q.start = __ballot(q.first);
+  return q;
 }
 
-// points (counts[s]) and segments (counts[nsites + s]) of every site.  The
-// candidates are visited in tiles of 256 consecutive ones; a segment starts
-// at an inside candidate that is the first of its line or follows an
-// outside one, judged from the same inside flags as the points.
-__global__ __launch_bounds__(256) void k_site_count(const SiteGeo *__restrict__ geo, Lat9 L, int f0, int f1, int f2,
-                                                    int nsites, int *__restrict__ counts) {
+// points (counts[s]) and segments (counts[nsites + s]) of every site
+__global__ __launch_bounds__(64 * SITE_W) void k_site_count(const SiteGeo *__restrict__ geo, Lat9 L, int f0, int f1,
+                                                            int f2, int nsites, int *__restrict__ counts) {
   const SiteGeo s = geo[blockIdx.x];
   const int fftg[3] = {f0, f1, f2};
-  const int w0 = 2 * s.g[0] + 1;
-  const int ncand = w0 * (2 * s.g[1] + 1) * (2 * s.g[2] + 1);
-  __shared__ int flags[256], red[256], reds[256];
-  __shared__ int prev_last;
-  if (threadIdx.x == 0)
-    prev_last = 0;
+  const int ncand = (2 * s.g[0] + 1) * (2 * s.g[1] + 1) * (2 * s.g[2] + 1);
+  const int wave = threadIdx.x >> 6;
+  __shared__ int red[2][SITE_W];
   int cnt = 0, nseg = 0;
-  for (int c0 = 0; c0 < ncand; c0 += 256) {
-    const int c = c0 + threadIdx.x;
-    double cv[3];
-    const int in = (c < ncand && cand_inside(s, L, fftg, c, cv)) ? 1 : 0;
-    flags[threadIdx.x] = in;
-    __syncthreads();
-    const int prev = threadIdx.x > 0 ? flags[threadIdx.x - 1] : prev_last;
-    cnt += in;
-    nseg += (in && (c % w0 == 0 || !prev)) ? 1 : 0;
-    __syncthreads();
-    if (threadIdx.x == 255)
-      prev_last = flags[255];
-    __syncthreads();
+  for (int c0 = 63 * wave; c0 < ncand; c0 += 63 * SITE_W) {
+    const SiteBallot q = site_ballot(s, L, fftg, c0, ncand);
+    cnt += __popcll(q.in);
+    nseg += __popcll(q.start);
   }
-  red[threadIdx.x] = cnt;
-  reds[threadIdx.x] = nseg;
+  if ((threadIdx.x & 63) == 0) {
+    red[0][wave] = cnt;
+    red[1][wave] = nseg;
+  }
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      red[threadIdx.x] += red[threadIdx.x + o];
-      reds[threadIdx.x] += reds[threadIdx.x + o];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    counts[blockIdx.x] = red[0];
-    counts[nsites + blockIdx.x] = reds[0];
+  if (threadIdx.x < 2) {
+    int n = 0;
+    for (int w = 0; w < SITE_W; w++)
+      n += red[threadIdx.x][w];
+    counts[threadIdx.x * nsites + blockIdx.x] = n;
   }
 }
 
-// Ordered compaction of the inside candidates and of the segment starts
-// (block scans per tile of 256).  A segment is stored as (first point,
-// length, wrapped i of the first point, site) and its wrapped line
+// Ordered compaction of the inside candidates and of the segment starts, a
+// tile of 63 SITE_W candidates at a time.  A segment is stored as (first
+// point, length, wrapped i of the first point, site) and its wrapped line
 // j * N2 + k; the lengths are filled in by k_seg_len.
-__global__ __launch_bounds__(256) void k_site_fill(const SiteGeo *__restrict__ geo, Lat9 L, int f0, int f1, int f2,
-                                                   const int *__restrict__ site_pt, const int *__restrict__ seg_off,
-                                                   int *__restrict__ pidx, double *__restrict__ path,
-                                                   int4 *__restrict__ seg, int *__restrict__ segline) {
+__global__ __launch_bounds__(64 * SITE_W) void k_site_fill(const SiteGeo *__restrict__ geo, Lat9 L, int f0, int f1,
+                                                           int f2, const int *__restrict__ site_pt,
+                                                           const int *__restrict__ seg_off, int *__restrict__ pidx,
+                                                           double *__restrict__ path, int4 *__restrict__ seg,
+                                                           int *__restrict__ segline) {
   const SiteGeo s = geo[blockIdx.x];
   const int fftg[3] = {f0, f1, f2};
-  const int w0 = 2 * s.g[0] + 1;
-  const int ncand = w0 * (2 * s.g[1] + 1) * (2 * s.g[2] + 1);
-  __shared__ int flags[256], scan[256], scans[256];
-  __shared__ int running, running_s, prev_last;
-  if (threadIdx.x == 0) {
-    running = site_pt[blockIdx.x];
-    running_s = seg_off[blockIdx.x];
-    prev_last = 0;
-  }
-  __syncthreads();
-  for (int c0 = 0; c0 < ncand; c0 += 256) {
-    const int c = c0 + threadIdx.x;
-    int i = 0, j = 0, k = 0;
-    double cv[3] = {0, 0, 0};
-    int in = 0;
-    if (c < ncand) {
-      box_ijk(s, c, i, j, k);
-      in = inside(s, L, fftg, i, j, k, cv) ? 1 : 0;
+  const int ncand = (2 * s.g[0] + 1) * (2 * s.g[1] + 1) * (2 * s.g[2] + 1);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ int cnt[2][SITE_W];  // points, and segments << 16, of a tile's wavefronts
+  int run = site_pt[blockIdx.x], runs = seg_off[blockIdx.x];
+  for (int c0 = 0, p = 0; c0 < ncand; c0 += 63 * SITE_W, p ^= 1) {
+    const SiteBallot q = site_ballot(s, L, fftg, c0 + 63 * wave, ncand);
+    if (lane == 0)
+      cnt[p][wave] = __popcll(q.in) | __popcll(q.start) << 16;
+    __syncthreads();  // the next tile's counts go to the other half
+    int before = 0, all = 0;
+    for (int w = 0; w < SITE_W; w++) {
+      before += w < wave ? cnt[p][w] : 0;
+      all += cnt[p][w];
     }
-    flags[threadIdx.x] = in;
-    __syncthreads();
-    const int prev = threadIdx.x > 0 ? flags[threadIdx.x - 1] : prev_last;
-    const int st = (in && (c % w0 == 0 || !prev)) ? 1 : 0;
-    scan[threadIdx.x] = in;
-    scans[threadIdx.x] = st;
-    __syncthreads();
-    // Hillis-Steele inclusive scans
-    for (int o = 1; o < 256; o <<= 1) {
-      int v = threadIdx.x >= o ? scan[threadIdx.x - o] : 0;
-      int vs = threadIdx.x >= o ? scans[threadIdx.x - o] : 0;
-      __syncthreads();
-      scan[threadIdx.x] += v;
-      scans[threadIdx.x] += vs;
-      __syncthreads();
-    }
-    int pos = running + scan[threadIdx.x] - in;
-    if (in) {
-      int ii = (i % fftg[0] + fftg[0]) % fftg[0];
-      int jj = (j % fftg[1] + fftg[1]) % fftg[1];
-      int kk = (k % fftg[2] + fftg[2]) % fftg[2];
+    const unsigned long long below = (1ull << lane) - 1;
+    if (q.mine) {
+      const int pos = run + (before & 0xffff) + __popcll(q.in & below);
+      const int ii = (q.i % fftg[0] + fftg[0]) % fftg[0];
+      const int jj = (q.j % fftg[1] + fftg[1]) % fftg[1];
+      const int kk = (q.k % fftg[2] + fftg[2]) % fftg[2];
       pidx[pos] = (ii * fftg[1] + jj) * fftg[2] + kk;
-      path[3 * (long)pos + 0] = cv[0];
-      path[3 * (long)pos + 1] = cv[1];
-      path[3 * (long)pos + 2] = cv[2];
-      if (st) {
-        const int q = running_s + scans[threadIdx.x] - 1;
-        seg[q] = make_int4(pos, 0, ii, blockIdx.x);
-        segline[q] = jj * fftg[2] + kk;
+      path[3 * (long)pos + 0] = q.cv[0];
+      path[3 * (long)pos + 1] = q.cv[1];
+      path[3 * (long)pos + 2] = q.cv[2];
+      if (q.first) {
+        const int n = runs + (before >> 16) + __popcll(q.start & below);
+        seg[n] = make_int4(pos, 0, ii, blockIdx.x);
+        segline[n] = jj * fftg[2] + kk;
       }
     }
-    __syncthreads();
-    if (threadIdx.x == 255) {
-      running += scan[255];
-      running_s += scans[255];
-      prev_last = flags[255];
-    }
-    __syncthreads();
+    run += all & 0xffff;
+    runs += all >> 16;
   }
 }
 
@@ -225,15 +207,20 @@ __global__ __launch_bounds__(256) void k_site_values(const SiteGeo *__restrict__
   int ii = g / (fftg[1] * fftg[2]);
   double pf[3] = {(double)ii / fftg[0], (double)jj / fftg[1], (double)kk / fftg[2]};
   // minimum image of the wrapped point (utils.c:51-73, 566-576)
-  double best = INFINITY, v[3] = {0, 0, 0};
+  // (a square that is no smaller has no smaller root: few roots are taken)
+  double best = INFINITY, best2 = INFINITY, v[3] = {0, 0, 0};
   for (int a = -1; a <= 1; a++)
     for (int b = -1; b <= 1; b++)
       for (int c = -1; c <= 1; c++) {
         double fv[3] = {pf[0] + a - s.coord[0], pf[1] + b - s.coord[1], pf[2] + c - s.coord[2]}, cv[3];
         d_frac_to_cart(fv, L.m, cv);
-        double d = sqrt(cv[0] * cv[0] + cv[1] * cv[1] + cv[2] * cv[2]);
+        const double d2 = cv[0] * cv[0] + cv[1] * cv[1] + cv[2] * cv[2];
+        if (!(d2 < best2))
+          continue;
+        const double d = sqrt(d2);
         if (d < best) {
           best = d;
+          best2 = d2;
           v[0] = cv[0];
           v[1] = cv[1];
           v[2] = cv[2];
@@ -253,36 +240,55 @@ __global__ __launch_bounds__(256) void k_site_values(const SiteGeo *__restrict__
   const double *x = spl + s.spl_off;
   const int ts = table_stride(s.nproj, sizeof(T) == 4);
   T *out = table + tab_off[s_id] + (long)i * ts;
+  // place on the radial grid (utils.c:461-475), the same for every channel
+  const bool beyond = r > x[n - 1], below = r < x[0];
+  int id = 0;
+  double t = 0.0;
+  if (!beyond && !below) {
+    id = (int)(r / s.rmax * n);
+    if (id > n - 2)
+      id = n - 2;
+    t = r - x[id];
+  }
+  // Channels of one l in a row share their angular factors: four channels'
+  // radial values, then for each |m| the two real forms: slot m >= 0 holds
+  // A_|m| cos(|m| phi), slot -|m| holds A_|m| sin(|m| phi), with
+  // A_|m| = N_l|m| P_l^|m|(cos theta) radial.  Bound by its FP64 operations
+  // (215 sites of 5,900 points, two channels of l = 0, 1, 2: 143 us with the
+  // factors made for every slot and a root for each of the 27 images, 123 so).
+  constexpr int CR = 4;
   int p = 0;
-  for (int ch = 0; ch < s.nchan; ch++) {
+  for (int ch = 0; ch < s.nchan;) {
     const int l = chan_l[s.chan_off + ch];
-    const double *f = x + (long)(1 + ch) * n;
-    const double *bb = x + (long)(1 + s.nchan + ch) * n;
-    const double *cc = x + (long)(1 + 2 * s.nchan + ch) * n;
-    const double *dd = x + (long)(1 + 3 * s.nchan + ch) * n;
-    // utils.c:461-475
-    double radial;
-    if (r > x[n - 1]) {
-      radial = 0.0;
-    } else if (r < x[0]) {
-      radial = f[0];
-    } else {
-      int id = (int)(r / s.rmax * n);
-      if (id > n - 2)
-        id = n - 2;
-      double t = r - x[id];
-      radial = f[id] + t * (bb[id] + t * (cc[id] + t * dd[id]));
+    int nc = 1;
+    while (nc < CR && ch + nc < s.nchan && chan_l[s.chan_off + ch + nc] == l)
+      nc++;
+    double radial[CR];
+#pragma unroll
+    for (int q = 0; q < CR; q++) {
+      radial[q] = 0.0;
+      if (q < nc && !beyond) {
+        const double *f = x + (long)(1 + ch + q) * n;
+        const double *bb = f + (long)s.nchan * n, *cc = bb + (long)s.nchan * n, *dd = cc + (long)s.nchan * n;
+        radial[q] = below ? f[0] : f[id] + t * (bb[id] + t * (cc[id] + t * dd[id]));
+      }
     }
-    for (int m = -l; m <= l; m++, p++) {
-      // real form: slot m >= 0 holds A_|m| cos(|m| phi), slot -|m| holds
-      // A_|m| sin(|m| phi), with A_|m| = N_l|m| P_l^|m|(cos theta) radial
-      const int am = m < 0 ? -m : m;
-      double norm = sqrt((2 * l + 1) / (4.0 * M_PI) * d_fact(l - am) / d_fact(l + am));
-      double pl = norm * d_legendre(l, am, ct) * radial;
+    for (int am = 0; am <= l; am++) {
+      const double norm = sqrt((2 * l + 1) / (4.0 * M_PI) * d_fact(l - am) / d_fact(l + am));
+      const double a = norm * d_legendre(l, am, ct);
       double sn, cs;
       sincos(am * phi, &sn, &cs);
-      out[p] = (T)(m < 0 ? pl * sn : pl * cs);
+#pragma unroll
+      for (int q = 0; q < CR; q++)
+        if (q < nc) {
+          const double pl = a * radial[q];
+          out[p + q * (2 * l + 1) + l + am] = (T)(pl * cs);
+          if (am > 0)
+            out[p + q * (2 * l + 1) + l - am] = (T)(pl * sn);
+        }
     }
+    p += nc * (2 * l + 1);
+    ch += nc;
   }
   for (; p < ts; p++)
     out[p] = (T)0;
@@ -849,7 +855,7 @@ static int sphere_build(pp_sphere *sp) {
   PP_TRY(sp->d_counts.ensure(sizeof(int) * 2 * ns));
   hipEvent_t ev;
   tbegin(ctx, K_TABLE, &ev);
-  hipLaunchKernelGGL(k_site_count, dim3(ns), dim3(256), 0, ctx->stream, (const SiteGeo *)sp->d_sitemeta.p, L,
+  hipLaunchKernelGGL(k_site_count, dim3(ns), dim3(64 * SITE_W), 0, ctx->stream, (const SiteGeo *)sp->d_sitemeta.p, L,
                      sp->fftg[0], sp->fftg[1], sp->fftg[2], ns, (int *)sp->d_counts.p);
   tend(ctx, K_TABLE, ev);
   PP_CHECK_HIP(hipGetLastError());
@@ -896,7 +902,7 @@ static int sphere_build(pp_sphere *sp) {
   PP_CHECK_HIP(hipMemcpyAsync(sp->d_proj_off.p, sp->proj_off.data(), sizeof(int) * (ns + 1), hipMemcpyHostToDevice,
                               ctx->stream));
   tbegin(ctx, K_TABLE, &ev);
-  hipLaunchKernelGGL(k_site_fill, dim3(ns), dim3(256), 0, ctx->stream, (const SiteGeo *)sp->d_sitemeta.p, L,
+  hipLaunchKernelGGL(k_site_fill, dim3(ns), dim3(64 * SITE_W), 0, ctx->stream, (const SiteGeo *)sp->d_sitemeta.p, L,
                      sp->fftg[0], sp->fftg[1], sp->fftg[2], (const int *)sp->d_site_pt.p,
                      (const int *)sp->d_seg_off.p, (int *)sp->d_pidx.p, (double *)sp->d_path.p, (int4 *)sp->d_seg.p,
                      (int *)sp->d_segline.p);
