@@ -44,10 +44,10 @@ template <typename T> constexpr int fft2_lanes(int R1, int R2) {
   return sizeof(T) == 4 && (R1 > R2 ? R1 : R2) >= 16 ? 16 : 8;
 }
 // Band groups of a work-group: about 256 threads and at most 36 KiB of rows
-// (four or more work-groups per CU), but two where 52 KiB hold them: 256
-// contiguous bytes per element run faster than 128 (x pass of 108 in FP64
-// 465 -> 421 us, of 192 in FP32 1419 -> 1367; two of 216 leave two
-// work-groups per CU, 3216 -> 4090).
+// (four or more work-groups per CU), but two where 52 KiB hold them: the 256
+// contiguous bytes per element of two groups side by side run faster than
+// 128 (x pass of 108 in FP64 465 -> 421 us; two of 216 leave two work-groups
+// per CU, 3185 -> 3715).
 template <typename T> constexpr int fft2_lines(int R1, int R2) {
   const int rm = R1 > R2 ? R1 : R2, by_threads = 256 / (fft2_lanes<T>(R1, R2) * rm);
   const int row = R1 * R2 * 128, by_lds = 36 * 1024 / row, least = 2 * row <= 52 * 1024 ? 2 : 1;
@@ -148,10 +148,14 @@ __device__ __forceinline__ void fft2_tile(cplx<T> *__restrict__ g, const Fft2Arg
   const long u0 = (long)blk * LPW;  // units (line, band group), the groups of a line adjacent
   const int t = threadIdx.x, p = t % LR, q = t / LR;
   const bool masked = a.axis == 0 && bd.xm;
-  const int j2 = q % R2, lla = LPW == 1 ? 0 : q / R2, k1 = q % R1, llb = LPW == 1 ? 0 : q / R1;
-  const unsigned ua = (unsigned)(u0 + lla), ub = (unsigned)(u0 + llb), ng = (unsigned)a.ngroups;
+  // the units of an element next to each other, so that a wavefront's access
+  // to two band groups of a line is whole 256-byte rows (64 bands in FP32, z /
+  // y / x of 108: 45 / 95 / 167 us against 50 / 111 / 184 with a unit's
+  // elements next to each other, of 192: 123 / 410 / 893 against 142 / 449 /
+  // 1034; FP64 and one unit per work-group: the same)
+  const int j2 = q / LPW % R2, k1 = q / LPW % R1, ll = q % LPW;
+  const unsigned ua = (unsigned)(u0 + ll), ng = (unsigned)a.ngroups;
   const PassLine la = fft2_line(bd, a.axis, a.n2, a.s1, a.s2, ua / ng, a.nlines);
-  const PassLine lb = LPW == 1 ? la : fft2_line(bd, a.axis, a.n2, a.s1, a.s2, ub / ng, a.nlines);
   const bool ina = q < LPW * R2, inb = q < LPW * R1;
   // twiddles and coverage words are read into registers ahead of the line's
   // elements and written to LDS after those loads, so that all wait on one
@@ -209,17 +213,17 @@ __device__ __forceinline__ void fft2_tile(cplx<T> *__restrict__ g, const Fft2Arg
 #pragma unroll
         for (int c = 0; c < PK; c++)
           x.v[c] = k > 0 ? v[c][k] * w : v[c][k];
-        store_pack<T, PK>(buf + ((lla * N + k * R2 + j2) * LR + p) * PK, false, x);
+        store_pack<T, PK>(buf + (((k * R2 + j2) * LPW + ll) * LR + p) * PK, false, x);
       }
     }
   }
   __syncthreads();
-  if (!inb || !lb.on)
+  if (!inb || !la.on)
     return;
   cplx<T> v[PK][R2];
 #pragma unroll
   for (int j = 0; j < R2; j++) {
-    const BandPack<T, PK> x = load_pack<T, PK>(buf + ((llb * N + k1 * R2 + j) * LR + p) * PK, false);
+    const BandPack<T, PK> x = load_pack<T, PK>(buf + (((k1 * R2 + j) * LPW + ll) * LR + p) * PK, false);
 #pragma unroll
     for (int c = 0; c < PK; c++)
       v[c][j] = x.v[c];
@@ -227,12 +231,12 @@ __device__ __forceinline__ void fft2_tile(cplx<T> *__restrict__ g, const Fft2Arg
 #pragma unroll
   for (int c = 0; c < PK; c++)
     Dft<T, R2>::run(v[c]);
-  cplx<T> *dst = g + lb.base + (ub % ng) * ROW + p * PK + (long)k1 * a.es;
+  cplx<T> *dst = g + la.base + (ua % ng) * ROW + p * PK + (long)k1 * a.es;
   const long step = (long)R1 * a.es;
 #pragma unroll
   for (int k2 = 0; k2 < R2; k2++) {
     const int e = k1 + R1 * k2;
-    if (masked && !((msk[llb * MW + (e >> 5)] >> (e & 31)) & 1u))
+    if (masked && !((msk[ll * MW + (e >> 5)] >> (e & 31)) & 1u))
       continue;  // no projector sphere reads this point
     BandPack<T, PK> x;
 #pragma unroll
