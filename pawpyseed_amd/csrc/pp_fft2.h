@@ -39,9 +39,11 @@ namespace pp {
 template <typename T> constexpr int fft2_bands() { return 128 / (int)sizeof(cplx<T>); }
 // Lanes of a line's band group: 8 of 16 bytes each (FP32 two bands a lane),
 // or for long FP32 lines 16 of 8 bytes, which doubles the wavefronts that
-// share a line's LDS (y pass of 192: 474 -> 448 us per 64-band chunk).
+// share a line's LDS (y pass of 192: 474 -> 448 us per 64-band chunk), unless
+// one group fills the work-group alone (fft2_lines), whose rows of 128 bytes
+// want the wider accesses (x pass of 216: 1669 us, 2018 with 16 lanes).
 template <typename T> constexpr int fft2_lanes(int R1, int R2) {
-  return sizeof(T) == 4 && (R1 > R2 ? R1 : R2) >= 16 ? 16 : 8;
+  return sizeof(T) == 4 && (R1 > R2 ? R1 : R2) >= 16 && 2 * R1 * R2 * 128 <= 52 * 1024 ? 16 : 8;
 }
 // Band groups of a work-group: about 256 threads and at most 36 KiB of rows
 // (four or more work-groups per CU), but two where 52 KiB hold them: the 256
