@@ -401,6 +401,7 @@ def main():
     gemm_flops = 8.0 * nb * nb * float(nw.mean())
     timed_settings = dict(R.get("autotune") or {n: ctx.get_param(n) for n in B.TUNED})
     timed_settings["gemm_planes"] = ctx.get_param("gemm_planes")
+    timed_settings["fft_xmask"] = int(xmask_on)
     traffic = read_traffic(head, timed_settings)
     rl = {}
     for c, b in alg.items():
@@ -411,32 +412,33 @@ def main():
         rl[c] = {"bound": "hbm", "achieved": b / (ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                  "alg_bytes": b, "avg_launch_ms": ms, "ms_per_step": kc["ms_total"],
                  "traffic": traffic.get(c)}
-    # augmentation (O_M of all pairs): the gather of R's matched projector
-    # rows and dO applied to S's (read once, written once each), then an
-    # FP64 GEMM over the KM matched projectors per k
+    # augmentation (O_M of all pairs): dO applied to S's matched projector
+    # rows (read once, written once), then one FP64 GEMM over the KM matched
+    # projectors of every k, which gathers R's rows itself
     KM = int(sum(plans[head][1].proj_off[s + 1] - plans[head][1].proj_off[s] for s in wl.M_S))
-    aug_bytes = 32.0 * KM * (nb + nb)
+    aug_bytes = 32.0 * KM * nb
     kc = R["kernels"].get("aug_prep")
     if kc and kc["launches"]:
-        ms = kc["ms_total"] / kc["launches"]  # one timed pair of launches covers all k
+        ms = kc["ms_total"] / kc["launches"]  # one launch covers all k
         rl["aug_prep"] = {"bound": "hbm", "achieved": aug_bytes * nk / (ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9,
                           "unit": "GB/s", "alg_bytes": aug_bytes * nk, "avg_launch_ms": ms,
                           "ms_per_step": kc["ms_total"], "traffic": traffic.get("aug_prep"),
-                          "what": "k_aug_gather + k_aug_apply of one call (all k): 16 B per gathered / applied "
-                                  "value, read and written"}
+                          "what": "k_aug_apply of one call (all k): 16 B per applied value, read and written"}
     kc = R["kernels"].get("aug_gemm")
     if kc and kc["launches"]:
         ms = kc["ms_total"] / kc["launches"]
-        rl["aug_gemm"] = {"bound": "mfma", "achieved": 8.0 * nb * nb * KM / (ms * 1e-3) / 1e12,
-                          "peak": PEAK["fp64"] / 1e12, "unit": "TFLOP/s", "alg_flops": 8.0 * nb * nb * KM,
+        aug_flops = 8.0 * nb * nb * KM * nk / kc["launches"]  # a launch covers several k
+        rl["aug_gemm"] = {"bound": "mfma", "achieved": aug_flops / (ms * 1e-3) / 1e12,
+                          "peak": PEAK["fp64"] / 1e12, "unit": "TFLOP/s", "alg_flops": aug_flops,
                           "avg_launch_ms": ms, "ms_per_step": kc["ms_total"], "traffic": traffic.get("aug_gemm"),
-                          "what": "FP64 MFMA conj(X_R) Y^T of one k-point over the matched projectors"}
+                          "what": "FP64 MFMA conj(X_R) Y^T of all k-points over the matched projectors"}
     kc = R["kernels"].get("gemm")
     if kc and kc["launches"]:
         ms = kc["ms_total"] / kc["launches"]
-        rl["gemm"] = {"bound": "mfma", "achieved": gemm_flops / (ms * 1e-3) / 1e12,
+        per_launch = gemm_flops * nk / kc["launches"]  # FP32: one k-point; FP64: several
+        rl["gemm"] = {"bound": "mfma", "achieved": per_launch / (ms * 1e-3) / 1e12,
                       "peak": PEAK["fp32" if head != "fp64" else "fp64"] / 1e12, "unit": "TFLOP/s",
-                      "alg_flops": gemm_flops, "avg_launch_ms": ms, "ms_per_step": kc["ms_total"],
+                      "alg_flops": per_launch, "avg_launch_ms": ms, "ms_per_step": kc["ms_total"],
                       "traffic": traffic.get("gemm")}
     # split-plane overlap GEMMs: the plane GEMM on the MFMA peak of its
     # 16-bit arithmetic (products x 8 M N K flop per k-point), and the split

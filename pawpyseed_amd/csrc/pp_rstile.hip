@@ -15,7 +15,7 @@
 //
 // A read-modify-write of every sphere point per colour and a read of the
 // whole chunk for the density become one read: 216^3 x 64 bands in FP64,
-// 4.5 + 1.8 ms before, 3.5 now (13.9 GB, 4 TB/s).  What bounds it is the
+// 4.5 + 1.8 ms before, 3.5 now (13.2 GB, 3.9 TB/s).  What bounds it is the
 // latency of the loads at three wavefronts per SIMD: the matrix units are
 // busy a quarter of it.  Tiles of 8 bands with interleaved parts, 8-byte loads and
 // the blocks of x fastest took 5.8 ms, without the first entry's table values

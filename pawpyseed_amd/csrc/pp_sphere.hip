@@ -61,7 +61,7 @@ __device__ __forceinline__ bool inside(const SiteGeo &s, const Lat9 &L, const in
 // that a wavefront's two ballots hold its inside flags and segment starts and
 // only the counts cross wavefronts.  Bound by the chain of tiles of a site:
 // 256 threads with shared flags and scans took 28 us to count and 88 to fill
-// for 215 sites of 5,900 points where these take 21 and 35, and for 8 sites 6
+// for 215 sites of 4,900 points where these take 21 and 35, and for 8 sites 6
 // and 14 where these take 4 and 6.  A segment starts at an inside candidate
 // that is the first of its line or follows an outside one.
 constexpr int SITE_W = 16;
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256) void k_site_values(const SiteGeo *__restrict__
   // radial values, then for each |m| the two real forms: slot m >= 0 holds
   // A_|m| cos(|m| phi), slot -|m| holds A_|m| sin(|m| phi), with
   // A_|m| = N_l|m| P_l^|m|(cos theta) radial.  Bound by its FP64 operations
-  // (215 sites of 5,900 points, two channels of l = 0, 1, 2: 143 us with the
+  // (215 sites of 4,900 points, two channels of l = 0, 1, 2: 143 us with the
   // factors made for every slot and a root for each of the 27 images, 123 so).
   constexpr int CR = 4;
   int p = 0;
