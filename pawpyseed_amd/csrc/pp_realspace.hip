@@ -741,7 +741,7 @@ namespace pp {
 int rs_tile_ensure(pp_ctx *ctx, pp_rsplan *rp, bool *use);
 template <typename T>
 int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, const cplx<double> *proj, long ldp,
-                int remove_phase, bool states, const double *wts, double *dens, cplx<T> *grid);
+                int remove_phase, cplx<double> *states, long ldo, const double *wts, double *dens, cplx<T> *grid);
 }  // namespace pp
 
 namespace {
@@ -792,21 +792,16 @@ int rs_chunk(pp_ctx *ctx, pp_rsplan *rp, FftPlan *pl, const double *kf, int nw, 
              cplx<T> *grid, int NB, bool tiles) {
   const long npts = (long)rp->fftg[0] * rp->fftg[1] * rp->fftg[2];
   PP_TRY(fft_chunk<T>(ctx, pl, grid, NB, nw, gidx, C, ldc, nbc, bd));
-  double scl = 1.0 / sqrt(det3(rp->lattice));
   hipEvent_t ev;
-  int phase_on = remove_phase ? 0 : 1;
   if (tiles) {
-    // augmentation and density (or the finished states, scale and phase
-    // included) in one pass over the chunk
+    // augmentation, density and finished states in one pass over the chunk
     tbegin(ctx, K_RS_AUG, &ev);
-    const int st = rs_tile_run<T>(ctx, rp, kf, nbc, NB, proj, ldp, remove_phase, states != nullptr, wts, dens, grid);
+    const int st = rs_tile_run<T>(ctx, rp, kf, nbc, NB, proj, ldp, remove_phase, states, ldo, wts, dens, grid);
     tend(ctx, K_RS_AUG, ev);
-    PP_TRY(st);
-    if (!states)
-      return PP_OK;
-    scl = 1.0;
-    phase_on = 0;
-  } else if (rp->nsites && rp->ptot) {
+    return st;
+  }
+  const double scl = 1.0 / sqrt(det3(rp->lattice));
+  if (rp->nsites && rp->ptot) {
     tbegin(ctx, K_RS_AUG, &ev);
     const int ppb = 64;
     const size_t lds = sizeof(cplx<double>) * 64 * (size_t)std::max(1, rp->pmax);
@@ -876,11 +871,11 @@ int rs_chunk(pp_ctx *ctx, pp_rsplan *rp, FftPlan *pl, const double *kf, int nw, 
   tbegin(ctx, K_RS_EMIT, &ev);
   if (states) {
     hipLaunchKernelGGL(k_rs_state<T>, dim3((unsigned)((npts + RS_TP - 1) / RS_TP)), dim3(256), 0, ctx->stream, grid,
-                       NB, nbc, npts, scl, rp->fftg[0], rp->fftg[1], rp->fftg[2], kf[0], kf[1], kf[2], phase_on,
-                       states, ldo);
+                       NB, nbc, npts, scl, rp->fftg[0], rp->fftg[1], rp->fftg[2], kf[0], kf[1], kf[2],
+                       remove_phase ? 0 : 1, states, ldo);
     PP_CHECK_HIP(hipGetLastError());
   }
-  if (dens && !tiles) {
+  if (dens) {
     RsWeights W;
     for (int b = 0; b < 64; b++)
       W.w[b] = b < nbc ? wts[b] : 0.0;

@@ -10,8 +10,9 @@
 // as the complex form with half the products), c the site's projections in
 // that form times the phase of its lattice image, so the points need no phase
 // of their own.  The tiles then give the block's densities, weighted and
-// summed over the bands, or go back to the chunk as states.  Sites that share
-// points add into one accumulator in site order: no atomics and no colours.
+// summed over the bands, and the states in their band-major places.  Sites
+// that share points add into one accumulator in site order: no atomics and no
+// colours.
 //
 // A read-modify-write of every sphere point per colour and a read of the
 // whole chunk for the density become one read: 216^3 x 64 bands in FP64,
@@ -21,7 +22,7 @@
 // the blocks of x fastest took 5.8 ms, without the first entry's table values
 // loaded a step ahead 4.0 ms.  A form that also ran the x pass, so that
 // the chunk was never written, read each table row once per band group, 33 GB
-// where this reads 14, and took 8.8 ms against 3.2 (x pass) plus this.
+// where this reads 13, and took 8.8 ms against 3.2 (x pass) plus this.
 //
 // Work lists: an entry is a (site, lattice image) whose sphere holds points
 // of one block; its table holds the site's partial-wave differences at the
@@ -214,7 +215,9 @@ struct RsTileArgs {
   const cplx<double> *ph;
   int ks, nxb, NB, nbc, f0, f1, f2;
   double scl;
-  int states, unphase;
+  int unphase;
+  cplx<double> *states;  // [band][ldo]
+  long ldo;
   double *dens;
   RsWeights w;
 };
@@ -231,21 +234,38 @@ __device__ __forceinline__ double rs_row_sum(double v) {
   return rs_dpp_add<0x140>(rs_dpp_add<0x141>(rs_dpp_add<0x4E>(rs_dpp_add<0xB1>(v))));
 }
 
-// Work-group: RS_Z consecutive x-lines (y, z..) of one block of 16 x, so that
-// their densities are written as rows of RS_Z consecutive z; each of the four
-// wavefronts takes every fourth line, PL groups of 16 bands at a time: one
-// accumulator tile of the real parts and one of the imaginary parts for each
-// (a lane past the chunk's bands repeats its last one, unused).  KS: groups of
-// four projector slots (0: any number).
+// Work-group: RS_Z consecutive x-lines (y, z..) of one block of
+// 16 x, so that their densities are written as rows of RS_Z consecutive z; each
+// of the four wavefronts takes every fourth line, PL groups of 16 bands at a
+// time: one accumulator tile of the real parts and one of the imaginary parts
+// for each (a lane past the chunk's bands repeats its last one, unused).  KS:
+// groups of four projector slots (0: any number).  With ST the finished
+// states go straight from the FP64 accumulators to the band-major output, the
+// four wavefronts' lines together through LDS as rows of four consecutive z:
+// the chunk is not written, and no rounding follows an FP32 transform.  (Put
+// back into the chunk for a copy to the band-major output, the states of 64
+// bands on 108^3 with 18 projectors took 1540 us in FP32 and 2098 in FP64
+// where these take 1290 and 1680.)  Two LDS tiles leave one barrier a step;
+// the run-time form keeps to one tile and its occupancy (32 projectors, FP64:
+// 1980 us, 2190 with two).
 constexpr int RS_Z = 16;
 constexpr int RS_E = 8;  // entries of a line's block whose site images are kept in LDS
-template <typename T, int KS, int PL>
-__global__ __launch_bounds__(256, PL > 1 ? 3 : 4) void k_rs_tiles(cplx<T> *__restrict__ g, RsTileArgs L) {
+constexpr int RS_SB = 65;  // row of a band in the states' LDS tile: 16 x of 4 z, and one off the banks
+// Wavefronts per SIMD that the compiled forms are held to: with room for one
+// more the compiler saves registers by loading the coefficients in smaller
+// batches (108^3, 64 bands, 9 projectors, FP32 density: 852 us against 793).
+// The run-time form, whose loads wait anyway, takes what fits (32 projectors,
+// FP64 density: 1555 us, held to three 1616).
+constexpr int rs_waves(int KS, int PL, bool most) { return most && KS == 0 ? 8 : PL > 1 ? 3 : 4; }
+template <typename T, int KS, int PL, bool ST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rs_waves(KS, PL, false), rs_waves(KS, PL, true))))
+void k_rs_tiles(cplx<T> *__restrict__ g, RsTileArgs L) {
   typedef T vec2 __attribute__((ext_vector_type(2)));
   __shared__ double dl[16][RS_Z + 1];
   __shared__ double s_w[64];
   __shared__ int s_i0[RS_Z], s_i1[RS_Z], s_vid[RS_Z * RS_E];
   __shared__ cplx<double> s_ez[RS_Z];
+  __shared__ cplx<double> s_st2[KS > 0 ? 2 : 1][ST ? 16 * PL * RS_SB : 1];
   // z, then y, then the block of x: groups in flight together share 16 planes
   const int nzb = (L.f2 + RS_Z - 1) / RS_Z, nyz = L.f1 * nzb;
   const int xb = blockIdx.x / nyz, r = blockIdx.x % nyz;
@@ -278,18 +298,20 @@ __global__ __launch_bounds__(256, PL > 1 ? 3 : 4) void k_rs_tiles(cplx<T> *__res
   }
   const int ks = KS > 0 ? KS : L.ks, nh = (L.NB + 16 * PL - 1) / (16 * PL);
   // the wavefront's steps: its lines, PL groups at a time.  A step's chunk
-  // values are loaded during the step before.
-  const int nz = min(RS_Z, L.f2 - z0), nstep = (nz - wave + 3) / 4 * nh;
+  // values are loaded during the step before.  (With ST all wavefronts take
+  // as many steps, for the barriers; a line past the last repeats it.)
+  const int nz = min(RS_Z, L.f2 - z0), nstep = (ST ? (nz + 3) / 4 : (nz - wave + 3) / 4) * nh;
   vec2 u[PL][4];
   auto places = [&](int h, int (&at)[PL]) {
 #pragma unroll
     for (int c = 0; c < PL; c++)
       at[c] = min((h * PL + c) * 16 + col, L.NB - 1);
   };
+  auto line = [&](int s) { return ST ? min(wave + 4 * (s / nh), nz - 1) : wave + 4 * (s / nh); };
   auto values = [&](int s, vec2 (&w)[PL][4]) {
     int at[PL];
     places(s % nh, at);
-    const long zo = (long)(z0 + wave + 4 * (s / nh)) * L.NB;
+    const long zo = (long)(z0 + line(s)) * L.NB;
 #pragma unroll
     for (int v = 0; v < 4; v++)
 #pragma unroll
@@ -300,7 +322,7 @@ __global__ __launch_bounds__(256, PL > 1 ? 3 : 4) void k_rs_tiles(cplx<T> *__res
   double tf[KS > 0 ? KS : 1];
   auto table = [&](int s) {
     if (KS > 0) {
-      const int q = wave + 4 * (s / nh);
+      const int q = line(s);
       const double *ta = L.tab + (long)min(s_i0[q], max(s_i1[q] - 1, 0)) * KS * 64 + lane;
 #pragma unroll
       for (int j = 0; j < KS; j++)
@@ -313,7 +335,7 @@ __global__ __launch_bounds__(256, PL > 1 ? 3 : 4) void k_rs_tiles(cplx<T> *__res
   }
   double dens[4] = {0.0, 0.0, 0.0, 0.0};
   for (int st = 0; st < nstep; st++) {
-    const int zi = wave + 4 * (st / nh), z = z0 + zi, h = st % nh;
+    const int zi = line(st), h = st % nh;
     const int i0 = __builtin_amdgcn_readfirstlane(s_i0[zi]), i1 = __builtin_amdgcn_readfirstlane(s_i1[zi]);
     const cplx<double> ez = s_ez[zi];
     int at[PL];
@@ -384,7 +406,8 @@ __global__ __launch_bounds__(256, PL > 1 ? 3 : 4) void k_rs_tiles(cplx<T> *__res
         }
       }
     }
-    if (L.states) {
+    if constexpr (ST) {
+      cplx<double> *s_st = s_st2[KS > 0 ? st & 1 : 0];
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const cplx<double> e = ex[v] * ez;
@@ -395,17 +418,29 @@ __global__ __launch_bounds__(256, PL > 1 ? 3 : 4) void k_rs_tiles(cplx<T> *__res
             a = (dr[c][v] * e.x + di[c][v] * e.y) / L.scl;
             b = (di[c][v] * e.x - dr[c][v] * e.y) / L.scl;
           }
-          if (16 * xb + row + 4 * v < L.f0 && (h * PL + c) * 16 + col < L.NB)
-            gx[v][(long)z * L.NB + at[c]] = vec2{(T)a, (T)b};
+          s_st[(c * 16 + col) * RS_SB + (row + 4 * v) * 4 + wave] = mk<double>(a, b);
         }
       }
+      __syncthreads();
+      const int zl = 4 * (st / nh) + (threadIdx.x & 3), x = 16 * xb + (threadIdx.x >> 2 & 15);
+      if (zl < nz && x < L.f0) {
+        const long pt = ((long)x * L.f1 + y) * L.f2 + z0 + zl;
+#pragma unroll
+        for (int q = 0; q < 4 * PL; q++) {
+          const int band = (int)(threadIdx.x >> 6) + 4 * q, b = h * PL * 16 + band;
+          if (b < L.nbc)
+            L.states[b * L.ldo + pt] = s_st[band * RS_SB + (threadIdx.x & 63)];
+        }
+      }
+      if (KS == 0)
+        __syncthreads();
     }
   }
   if (!L.dens)
     return;
   __syncthreads();
   const int x = 16 * xb + (threadIdx.x >> 4), zi = threadIdx.x & 15;
-  if (x < L.f0 && z0 + zi < L.f2)
+  if (x < L.f0 && zi < nz)
     L.dens[((long)x * L.f1 + y) * L.f2 + z0 + zi] += dl[threadIdx.x >> 4][zi];
 }
 
@@ -501,17 +536,25 @@ int rs_tile_ensure(pp_ctx *ctx, pp_rsplan *rp, bool *use) {
 
 template <typename T, int KS>
 static void rs_tiles_launch(hipStream_t st, cplx<T> *grid, const RsTileArgs &L, unsigned blocks) {
-  if (L.NB <= 16)
-    hipLaunchKernelGGL((k_rs_tiles<T, KS, 1>), dim3(blocks), dim3(256), 0, st, grid, L);
-  else
-    hipLaunchKernelGGL((k_rs_tiles<T, KS, 2>), dim3(blocks), dim3(256), 0, st, grid, L);
+#define PP_RT(PL, ST) hipLaunchKernelGGL((k_rs_tiles<T, KS, PL, ST>), dim3(blocks), dim3(256), 0, st, grid, L)
+  if (L.NB <= 16) {
+    if (L.states)
+      PP_RT(1, true);
+    else
+      PP_RT(1, false);
+  } else if (L.states) {
+    PP_RT(2, true);
+  } else {
+    PP_RT(2, false);
+  }
+#undef PP_RT
 }
 
 // The augmentation of a transformed chunk: densities (wts, dens) and / or the
-// finished states in the chunk.
+// finished states, either of them null.
 template <typename T>
 int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, const cplx<double> *proj, long ldp,
-                int remove_phase, bool states, const double *wts, double *dens, cplx<T> *grid) {
+                int remove_phase, cplx<double> *states, long ldo, const double *wts, double *dens, cplx<T> *grid) {
   const int f0 = rp->fftg[0], f1 = rp->fftg[1], f2 = rp->fftg[2];
   DevBuf &qb = ctx->rs_coef[ctx->slot];
   const long nq = (long)rp->nvid * 4 * rp->ks * NB, nph = f0 + f1 + f2;
@@ -539,33 +582,28 @@ int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, c
   L.f1 = f1;
   L.f2 = f2;
   L.states = states;
-  L.unphase = states && remove_phase;
+  L.ldo = ldo;
+  L.unphase = remove_phase;
   L.dens = dens;
   for (int b = 0; b < 64; b++)
     L.w.w[b] = dens && b < nbc ? wts[b] : 0.0;
   const long blocks = (long)L.nxb * f1 * ((f2 + RS_Z - 1) / RS_Z);
   switch (rp->ks) {
-  case 1:
-    rs_tiles_launch<T, 1>(ctx->stream, grid, L, (unsigned)blocks);
+#define PP_KS(K)                                                        \
+  case K:                                                               \
+    rs_tiles_launch<T, K>(ctx->stream, grid, L, (unsigned)blocks);      \
     break;
-  case 2:
-    rs_tiles_launch<T, 2>(ctx->stream, grid, L, (unsigned)blocks);
-    break;
-  case 3:
-    rs_tiles_launch<T, 3>(ctx->stream, grid, L, (unsigned)blocks);
-    break;
-  case 5:
-    rs_tiles_launch<T, 5>(ctx->stream, grid, L, (unsigned)blocks);
-    break;
+    PP_KS(1) PP_KS(2) PP_KS(3) PP_KS(5)
+#undef PP_KS
   default:
     rs_tiles_launch<T, 0>(ctx->stream, grid, L, (unsigned)blocks);
   }
   PP_CHECK_HIP(hipGetLastError());
   return PP_OK;
 }
-template int rs_tile_run<float>(pp_ctx *, pp_rsplan *, const double *, int, int, const cplx<double> *, long, int, bool,
-                                const double *, double *, cplx<float> *);
-template int rs_tile_run<double>(pp_ctx *, pp_rsplan *, const double *, int, int, const cplx<double> *, long, int, bool,
-                                 const double *, double *, cplx<double> *);
+template int rs_tile_run<float>(pp_ctx *, pp_rsplan *, const double *, int, int, const cplx<double> *, long, int,
+                                cplx<double> *, long, const double *, double *, cplx<float> *);
+template int rs_tile_run<double>(pp_ctx *, pp_rsplan *, const double *, int, int, const cplx<double> *, long, int,
+                                 cplx<double> *, long, const double *, double *, cplx<double> *);
 
 }  // namespace pp

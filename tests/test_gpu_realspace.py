@@ -292,8 +292,8 @@ def test_blocks_of_x_agree_with_the_site_kernels(ctx, name, nband, precision):
     groups per step, several chunks, spheres on faces and boxes that wrap;
     states with and without their phase and the density, zero weights among
     the bands.  Both add the same FP64 terms to the same transform in another
-    order, a few roundings of 1.1e-16; an FP32 chunk rounds the sum once more
-    (6e-8 of its value, and as much where sites share points)."""
+    order, a few roundings of 1.1e-16; the per-site kernels also round each
+    site's sum into an FP32 chunk (6e-8 of its value)."""
     from pawpyseed_amd.core import batched as B
     rng = np.random.default_rng(23)
     lat, fftg, k, G, C, species, labels, coords = _case(name, nband, rng)
@@ -325,6 +325,50 @@ def test_blocks_of_x_agree_with_the_site_kernels(ctx, name, nband, precision):
             if st:
                 for b in range(nband):
                     assert normwise(s3[b], s2[b]) < tol, (remove, b)
+    plan.close()
+
+
+def _device(C, G, proj):
+    Ch = np.zeros((len(C), -(-len(G) // 64) * 64), np.complex64)
+    Ch[:, :len(G)] = C
+    return [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (Ch, G.astype(np.int32), proj)]
+
+
+def _by_kernel(ctx, plan, k, dev, nband, fftg, precision, remove=False, kernels=(2, 3)):
+    """States and density (weights 0.5 to 1.5) of the bands with each kernel."""
+    from pawpyseed_amd.core import batched as B
+    Cd, Gd, Pd = dev
+    out = []
+    try:
+        for kern in kernels:
+            ctx.set_param("rs_kernel", kern)
+            st = torch.zeros((nband,) + tuple(fftg), dtype=torch.complex128, device="cuda")
+            dens = torch.zeros(tuple(fftg), dtype=torch.float64, device="cuda")
+            torch.cuda.synchronize()
+            B.realspace_states(ctx, plan, k, Gd, Cd, Pd, states_out=st, remove_phase=remove, precision=precision)
+            B.realspace_states(ctx, plan, k, Gd, Cd, Pd, density_out=dens, weights=np.linspace(0.5, 1.5, nband),
+                               precision=precision)
+            out.append((st.cpu().numpy(), dens.cpu().numpy()))
+    finally:
+        ctx.set_param("rs_kernel", 3)
+    return out
+
+
+@pytest.mark.parametrize("nband", [5, 33])
+@pytest.mark.parametrize("remove", [False, True])
+def test_fp32_states_are_not_rounded_after_the_transform(ctx, nband, remove):
+    """The scale and the Bloch phase are applied to an FP32 transform's values
+    in FP64 on their way into the complex128 states: without projections both
+    augmentation kernels give the same states to a few roundings of 1.1e-16
+    (states rounded to FP32 once more differ by 3e-8)."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(29)
+    lat, fftg, k, G, C, species, labels, coords = _case("cubic", nband, rng)
+    plan = B.RealspacePlan(ctx, lat, fftg, coords, labels, species)
+    dev = _device(C, G, np.zeros((nband, plan.ptot), np.complex128))
+    (want, _), (got, _) = _by_kernel(ctx, plan, k, dev, nband, fftg, "fp32", remove)
+    for b in range(nband):
+        assert normwise(got[b], want[b]) < 2e-15
     plan.close()
 
 
