@@ -153,16 +153,31 @@ __global__ __launch_bounds__(256) void k_rst_values(const RsSite *__restrict__ g
     out[(p >> 2) * 64 + (p & 3) * 16] = 0.0;
 }
 
-// coef[((v * 4 ks + p) * NB + b) * 2 ..]: the coefficient of real-harmonic
-// slot p of site image v for band b, with P_m the band's projections:
+// What the pass over a chunk reads besides it, in one launch.  The first nb0
+// work-groups: ph = e^{2 pi i k_a i / n_a} of the three axes, the first times
+// the scale.  The others: coef[(v * 4 ks + p) * NB + b], the coefficient of
+// real-harmonic slot p of site image v for band b, with P_m the band's
+// projections:
 //   m > 0: P_m + (-1)^m P_-m,  slot -m: i (P_m - (-1)^m P_-m),  m = 0: P_0,
 // times e^{2 pi i k.(R - image)}; zero past the bands and the projectors.
-__global__ __launch_bounds__(256) void k_rst_coef(int nvid, const int2 *__restrict__ vsite,
+__global__ __launch_bounds__(256) void k_rst_coef(int nb0, int nvid, const int2 *__restrict__ vsite,
                                                   const RsSite *__restrict__ geo, const int *__restrict__ chan_l,
                                                   int ks, int NB, int nbc, const cplx<double> *__restrict__ proj,
-                                                  long ldp, double k0, double k1, double k2,
+                                                  long ldp, double k0, double k1, double k2, int f0, int f1, int f2,
+                                                  double scl, cplx<double> *__restrict__ ph,
                                                   cplx<double> *__restrict__ coef) {
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if ((int)blockIdx.x < nb0) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= f0 + f1 + f2)
+      return;
+    const double a = i < f0 ? k0 * i / f0 : i < f0 + f1 ? k1 * (i - f0) / f1 : k2 * (i - f0 - f1) / f2;
+    const double q = i < f0 ? scl : 1.0;
+    double sn, cs;
+    sincospi(2.0 * a, &sn, &cs);
+    ph[i] = mk<double>(q * cs, q * sn);
+    return;
+  }
+  const long t = (long)(blockIdx.x - nb0) * 256 + threadIdx.x;
   if (t >= (long)nvid * 4 * ks * NB)
     return;
   const int b = (int)(t % NB), p = (int)(t / NB % (4 * ks)), v = (int)(t / NB / (4 * ks));
@@ -194,19 +209,6 @@ __global__ __launch_bounds__(256) void k_rst_coef(int nvid, const int2 *__restri
 
 typedef double rs_doublex4 __attribute__((ext_vector_type(4)));
 
-// e^{2 pi i k_a i / n_a} of the three axes, the first times the scale.
-__global__ __launch_bounds__(256) void k_rst_phases(int f0, int f1, int f2, double k0, double k1, double k2, double scl,
-                                                    cplx<double> *__restrict__ ph) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= f0 + f1 + f2)
-    return;
-  const double a = i < f0 ? k0 * i / f0 : i < f0 + f1 ? k1 * (i - f0) / f1 : k2 * (i - f0 - f1) / f2;
-  const double s = i < f0 ? scl : 1.0;
-  double sn, cs;
-  sincospi(2.0 * a, &sn, &cs);
-  ph[i] = mk<double>(s * cs, s * sn);
-}
-
 struct RsTileArgs {
   const int *off;      // first entry of every (line, block of 16 x)
   const int4 *ent;     // entries: (site image, ...)
@@ -214,6 +216,7 @@ struct RsTileArgs {
   const cplx<double> *coef;  // [site image][4 ks][NB]
   const cplx<double> *ph;
   int ks, nxb, NB, nbc, f0, f1, f2;
+  int rz;  // x-lines of a work-group
   double scl;
   int unphase;
   cplx<double> *states;  // [band][ldo]
@@ -234,8 +237,8 @@ __device__ __forceinline__ double rs_row_sum(double v) {
   return rs_dpp_add<0x140>(rs_dpp_add<0x141>(rs_dpp_add<0x4E>(rs_dpp_add<0xB1>(v))));
 }
 
-// Work-group: RS_Z consecutive x-lines (y, z..) of one block of
-// 16 x, so that their densities are written as rows of RS_Z consecutive z; each
+// Work-group: rz (at most RS_Z) consecutive x-lines (y, z..) of one block of
+// 16 x, so that their densities are written as rows of rz consecutive z; each
 // of the four wavefronts takes every fourth line, PL groups of 16 bands at a
 // time: one accumulator tile of the real parts and one of the imaginary parts
 // for each (a lane past the chunk's bands repeats its last one, unused).  KS:
@@ -267,9 +270,9 @@ void k_rs_tiles(cplx<T> *__restrict__ g, RsTileArgs L) {
   __shared__ cplx<double> s_ez[RS_Z];
   __shared__ cplx<double> s_st2[KS > 0 ? 2 : 1][ST ? 16 * PL * RS_SB : 1];
   // z, then y, then the block of x: groups in flight together share 16 planes
-  const int nzb = (L.f2 + RS_Z - 1) / RS_Z, nyz = L.f1 * nzb;
+  const int nzb = (L.f2 + L.rz - 1) / L.rz, nyz = L.f1 * nzb;
   const int xb = blockIdx.x / nyz, r = blockIdx.x % nyz;
-  const int y = r / nzb, z0 = (r % nzb) * RS_Z;
+  const int y = r / nzb, z0 = (r % nzb) * L.rz;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, row = lane >> 4;
   if (threadIdx.x < 64)
@@ -300,7 +303,7 @@ void k_rs_tiles(cplx<T> *__restrict__ g, RsTileArgs L) {
   // the wavefront's steps: its lines, PL groups at a time.  A step's chunk
   // values are loaded during the step before.  (With ST all wavefronts take
   // as many steps, for the barriers; a line past the last repeats it.)
-  const int nz = min(RS_Z, L.f2 - z0), nstep = (ST ? (nz + 3) / 4 : (nz - wave + 3) / 4) * nh;
+  const int nz = min(L.rz, L.f2 - z0), nstep = (ST ? (nz + 3) / 4 : (nz - wave + 3) / 4) * nh;
   vec2 u[PL][4];
   auto places = [&](int h, int (&at)[PL]) {
 #pragma unroll
@@ -562,12 +565,10 @@ int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, c
   cplx<double> *coef = (cplx<double> *)qb.p, *ph = coef + nq;
   RsTileArgs L{};
   L.scl = 1.0 / sqrt(det3(rp->lattice));
-  hipLaunchKernelGGL(k_rst_phases, dim3((unsigned)((nph + 255) / 256)), dim3(256), 0, ctx->stream, f0, f1, f2, kf[0],
-                     kf[1], kf[2], L.scl, ph);
-  if (nq)
-    hipLaunchKernelGGL(k_rst_coef, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, ctx->stream, rp->nvid,
-                       (const int2 *)rp->l_vid.p, (const RsSite *)rp->d_geo.p, (const int *)rp->d_chan_l.p, rp->ks, NB,
-                       nbc, proj, ldp, kf[0], kf[1], kf[2], coef);
+  const int nb0 = (int)((nph + 255) / 256);
+  hipLaunchKernelGGL(k_rst_coef, dim3((unsigned)(nb0 + (nq + 255) / 256)), dim3(256), 0, ctx->stream, nb0, rp->nvid,
+                     (const int2 *)rp->l_vid.p, (const RsSite *)rp->d_geo.p, (const int *)rp->d_chan_l.p, rp->ks, NB,
+                     nbc, proj, ldp, kf[0], kf[1], kf[2], f0, f1, f2, L.scl, ph, coef);
   PP_CHECK_HIP(hipGetLastError());
   L.off = (const int *)rp->l_off.p;
   L.ent = (const int4 *)rp->l_ent.p;
@@ -587,7 +588,15 @@ int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, c
   L.dens = dens;
   for (int b = 0; b < 64; b++)
     L.w.w[b] = dens && b < nbc ? wts[b] : 0.0;
-  const long blocks = (long)L.nxb * f1 * ((f2 + RS_Z - 1) / RS_Z);
+  // Four lines a work-group (one a wavefront) where 16 leave the chip short of
+  // work-groups (fewer than two per CU: 20^3, 64 bands, 18 projectors, states
+  // 125 -> 100 us), and for states of more than 16 bands, whose work-groups
+  // wait on each other's lines (90^3, FP32: 823 -> 769 us; 108^3: the same).
+  // Else 16, which read the lines' tables together (108^3, 4 bands: 378 us
+  // against 417).
+  const long cols = (long)L.nxb * f1;
+  L.rz = cols * ((f2 + RS_Z - 1) / RS_Z) < 512 || (states && NB > 16) ? 4 : RS_Z;
+  const long blocks = cols * ((f2 + L.rz - 1) / L.rz);
   switch (rp->ks) {
 #define PP_KS(K)                                                        \
   case K:                                                               \

@@ -372,6 +372,30 @@ def test_fp32_states_are_not_rounded_after_the_transform(ctx, nband, remove):
     plan.close()
 
 
+@pytest.mark.parametrize("fftg", [(50, 52, 54), (33, 49, 90)])
+@pytest.mark.parametrize("nband", [7, 20])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_lines_of_a_work_group(ctx, fftg, nband, precision):
+    """Grids of more than 512 blocks of 16 lines, where a work-group takes 16
+    lines for up to 16 bands and for densities and four for the states of more
+    (the smaller grids of the other tests take four throughout), y and z ending
+    inside a work-group's lines; bounds as the test above."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(31)
+    wl = synthetic.tiny_config(ls=(0, 0, 1, 1, 2, 2), alphas=(1.5, 3.0) * 3, rmax=1.3, fftg=fftg, nband=nband)
+    assert (fftg[0] + 15) // 16 * fftg[1] * ((fftg[2] + 15) // 16) >= 512
+    k, G = np.array([0.25, -0.25, 0.1]), wl.ensure_gvecs()[0]
+    plan = B.RealspacePlan(ctx, wl.lattice, fftg, wl.frac_S, np.zeros(len(wl.frac_S), np.int32), [wl.species])
+    proj = rng.normal(size=(nband, plan.ptot)) + 1j * rng.normal(size=(nband, plan.ptot))
+    dev = _device(wl.coefficients("S", nband=nband)[0], G, proj)
+    (s2, d2), (s3, d3) = _by_kernel(ctx, plan, k, dev, nband, fftg, precision)
+    tol = 1e-14 if precision == "fp64" else 4e-7
+    assert normwise(d3, d2) < tol
+    for b in range(nband):
+        assert normwise(s3[b], s2[b]) < tol, b
+    plan.close()
+
+
 def test_wrapping_boxes_fp32_atomics(ctx):
     """Atomic adds of the FP32 chunk where site boxes wrap onto themselves."""
     from pawpyseed_amd.core import batched as B
