@@ -160,12 +160,18 @@ __global__ __launch_bounds__(256) void k_rst_values(const RsSite *__restrict__ g
 // projections:
 //   m > 0: P_m + (-1)^m P_-m,  slot -m: i (P_m - (-1)^m P_-m),  m = 0: P_0,
 // times e^{2 pi i k.(R - image)}; zero past the bands and the projectors.
+//
+// The tables are zero at a block's points outside a sphere, and zero times an
+// infinite or NaN coefficient would reach all of them: such a coefficient is
+// left zero and the band's values inside the site's sphere, where the sum is
+// not finite anyway, are made NaN in the chunk.
+template <typename T>
 __global__ __launch_bounds__(256) void k_rst_coef(int nb0, int nvid, const int2 *__restrict__ vsite,
                                                   const RsSite *__restrict__ geo, const int *__restrict__ chan_l,
                                                   int ks, int NB, int nbc, const cplx<double> *__restrict__ proj,
-                                                  long ldp, double k0, double k1, double k2, int f0, int f1, int f2,
-                                                  double scl, cplx<double> *__restrict__ ph,
-                                                  cplx<double> *__restrict__ coef) {
+                                                  long ldp, double k0, double k1, double k2, RsLat L, int f0, int f1,
+                                                  int f2, double scl, cplx<double> *__restrict__ ph,
+                                                  cplx<double> *__restrict__ coef, cplx<T> *__restrict__ grid) {
   if ((int)blockIdx.x < nb0) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= f0 + f1 + f2)
@@ -203,6 +209,18 @@ __global__ __launch_bounds__(256) void k_rst_coef(int nb0, int nvid, const int2 
     double sn, cs;
     sincospi(2.0 * (k0 * (g.R[0] - s0) + k1 * (g.R[1] - s1) + k2 * (g.R[2] - s2)), &sn, &cs);
     c = c * mk<double>(cs, sn);
+    if (!(isfinite(c.x) && isfinite(c.y))) {
+      c = mk<double>(0, 0);
+      for (int q = 0; q < (2 * g.g[0] + 1) * (2 * g.g[1] + 1) * (2 * g.g[2] + 1); q++) {
+        int i, j, k;
+        rs_cand(g, q, i, j, k);
+        double d[3];
+        if (!(rs_vec(g, L, f0, f1, f2, i, j, k, d) < g.rmax))
+          continue;
+        const long pt = ((long)((i + f0) % f0) * f1 + (j + f1) % f1) * f2 + (k + f2) % f2;
+        grid[pt * NB + b] = mk<T>((T)NAN, (T)NAN);
+      }
+    }
   }
   coef[t] = c;
 }
@@ -565,10 +583,12 @@ int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, c
   cplx<double> *coef = (cplx<double> *)qb.p, *ph = coef + nq;
   RsTileArgs L{};
   L.scl = 1.0 / sqrt(det3(rp->lattice));
+  RsLat lat;
+  memcpy(lat.m, rp->lattice, sizeof(lat.m));
   const int nb0 = (int)((nph + 255) / 256);
-  hipLaunchKernelGGL(k_rst_coef, dim3((unsigned)(nb0 + (nq + 255) / 256)), dim3(256), 0, ctx->stream, nb0, rp->nvid,
+  hipLaunchKernelGGL(k_rst_coef<T>, dim3((unsigned)(nb0 + (nq + 255) / 256)), dim3(256), 0, ctx->stream, nb0, rp->nvid,
                      (const int2 *)rp->l_vid.p, (const RsSite *)rp->d_geo.p, (const int *)rp->d_chan_l.p, rp->ks, NB,
-                     nbc, proj, ldp, kf[0], kf[1], kf[2], f0, f1, f2, L.scl, ph, coef);
+                     nbc, proj, ldp, kf[0], kf[1], kf[2], lat, f0, f1, f2, L.scl, ph, coef, grid);
   PP_CHECK_HIP(hipGetLastError());
   L.off = (const int *)rp->l_off.p;
   L.ent = (const int4 *)rp->l_ent.p;

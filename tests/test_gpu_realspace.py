@@ -396,6 +396,37 @@ def test_lines_of_a_work_group(ctx, fftg, nband, precision):
     plan.close()
 
 
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 1e308])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_non_finite_projections_stay_in_their_spheres(ctx, bad, precision):
+    """An infinite, NaN or overflowing projection of one site and band makes
+    that band not finite inside the site's sphere and nowhere else, as with the
+    per-site kernels; other bands are as they were.  (1e308: finite itself,
+    its sum with the partner of -m is not.)"""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(37)
+    nband = 19
+    lat, fftg, k, G, C, species, labels, coords = _case("skewed", nband, rng)
+    plan = B.RealspacePlan(ctx, lat, fftg, coords, labels, species)
+    proj = rng.normal(size=(nband, plan.ptot)) + 1j * rng.normal(size=(nband, plan.ptot))
+    clean = _by_kernel(ctx, plan, k, _device(C, G, proj), nband, fftg, precision, kernels=(3,))[0][0]
+    p = int(plan.proj_off[1])  # the d channel of the second site, m = -2 .. 2
+    proj[17, p:p + 5] = bad * (1 + 1j)
+    (s2, d2), (s3, d3) = _by_kernel(ctx, plan, k, _device(C, G, proj), nband, fftg, precision)
+    nans = np.where((np.arange(nband) == 17)[:, None] & (np.arange(plan.ptot) == p), np.nan, proj)
+    inside = ~np.isfinite(_by_kernel(ctx, plan, k, _device(C, G, nans), nband, fftg, precision, kernels=(2,))[0][0][17])
+    assert 0 < inside.sum() < inside.size // 4
+    if bad != 1e308:  # (the per-site sums overflow at some of the points only)
+        assert np.array_equal(~np.isfinite(s2[17]), inside)
+    assert np.array_equal(~np.isfinite(s3[17]), inside)
+    assert np.array_equal(~np.isfinite(d3), inside)
+    out = ~inside
+    assert normwise(s3[17][out], clean[17][out]) < 1e-14
+    for b in (0, 16, 18):
+        assert np.array_equal(s3[b], clean[b])
+    plan.close()
+
+
 def test_wrapping_boxes_fp32_atomics(ctx):
     """Atomic adds of the FP32 chunk where site boxes wrap onto themselves."""
     from pawpyseed_amd.core import batched as B
