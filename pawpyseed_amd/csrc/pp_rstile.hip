@@ -622,7 +622,7 @@ int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, c
   case K:                                                               \
     rs_tiles_launch<T, K>(ctx->stream, grid, L, (unsigned)blocks);      \
     break;
-    PP_KS(1) PP_KS(2) PP_KS(3) PP_KS(5)
+    PP_KS(1) PP_KS(2) PP_KS(3) PP_KS(4) PP_KS(5)
 #undef PP_KS
   default:
     rs_tiles_launch<T, 0>(ctx->stream, grid, L, (unsigned)blocks);

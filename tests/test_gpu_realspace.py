@@ -427,6 +427,53 @@ def test_non_finite_projections_stay_in_their_spheres(ctx, bad, precision):
     plan.close()
 
 
+def _entries(lat, fftg, species, labels, coords):
+    """Most (site, lattice image) pairs whose spheres hold points of one block
+    of 16 x of a line."""
+    count = np.zeros((-(-fftg[0] // 16), fftg[1], fftg[2]), int)
+    ax = [np.arange(-n, 2 * n) for n in fftg]
+    f = np.stack(np.meshgrid(*[a / n for a, n in zip(ax, fftg)], indexing="ij"), axis=-1)
+    for e, c in zip(labels, coords):
+        i, j, k = np.nonzero(np.linalg.norm((f - c) @ lat, axis=-1) < species[e].grid[-1])
+        xs, ys, zs = ax[0][i], ax[1][j], ax[2][k]
+        key = np.unique(np.stack([xs % fftg[0] // 16, ys % fftg[1], zs % fftg[2], xs // fftg[0], ys // fftg[1],
+                                  zs // fftg[2]]), axis=1)
+        np.add.at(count, tuple(key[:3]), 1)
+    return count.max()
+
+
+@pytest.mark.parametrize("ls,rmax", [((0, 0, 1, 1, 2), 1.3), ((0, 1, 2, 3), 1.3), ((0, 0, 1, 1, 2, 2), 1.3),
+                                     ((0, 1, 2, 3, 2, 1, 0), 1.3), ((0, 1, 2, 3) * 2, 1.3), ((0, 0, 1, 1, 2, 2), 2.6)])
+@pytest.mark.parametrize("nband", [4, 33])
+def test_projector_widths(ctx, ls, rmax, nband):
+    """States and densities of sites with 13 to 32 projectors (every compiled
+    number of groups of four beside the other tests' 4, 5 and 9, and the
+    run-time one), f channels among them, beside a species of 4 in the same
+    plan, up to 16 bands and more, and spheres so wide that a block lies in
+    more than eight of them, against the oracle."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(41)
+    fftg = (20, 18, 20)
+    wl = synthetic.tiny_config(fftg=fftg, nband=nband, kpts=[[0.25, -0.25, 0.1]])
+    species = [synthetic.make_species(list(ls), [1.5 + 0.2 * i for i in range(len(ls))], rmax),
+               synthetic.make_species([0, 1], [1.5, 3.0], 1.1)]
+    labels = (np.arange(len(wl.frac_S)) % 4 == 3).astype(np.int32)
+    k, G, C = np.asarray(wl.kpts[0]), wl.ensure_gvecs()[0], wl.coefficients("S", nband=nband)[0]
+    if rmax > 2:
+        assert _entries(wl.lattice, fftg, species, labels, wl.frac_S) > 8
+    plan = B.RealspacePlan(ctx, wl.lattice, fftg, wl.frac_S, labels, species)
+    proj = rng.normal(size=(nband, plan.ptot)) + 1j * rng.normal(size=(nband, plan.ptot))
+    W = orc.WaveData(species)
+    want = [orc.realspace_state(wl.lattice, fftg, k, G, C[b], W, labels, wl.frac_S, proj[b]) for b in range(nband)]
+    dens = sum(w * np.abs(x) ** 2 for w, x in zip(np.linspace(0.5, 1.5, nband), want))
+    for precision, tol in (("fp64", 1e-10), ("fp32", 1e-5)):
+        st, de = _by_kernel(ctx, plan, k, _device(C, G, proj), nband, fftg, precision, kernels=(3,))[0]
+        for b in range(nband):
+            assert normwise(st[b], want[b]) < tol, (precision, b)
+        assert normwise(de, dens) < tol, precision
+    plan.close()
+
+
 def test_wrapping_boxes_fp32_atomics(ctx):
     """Atomic adds of the FP32 chunk where site boxes wrap onto themselves."""
     from pawpyseed_amd.core import batched as B
