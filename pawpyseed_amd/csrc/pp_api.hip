@@ -150,7 +150,7 @@ static int setup_prepare(pp_ctx *ctx, pp_sphere *sp, int nk, const double *kfrac
                          int nband, SetupState &S, const PrepBufs &pb) {
   const int *fftg = sphere_fftg(sp);
   PP_TRY(get_fft_plan(ctx, fftg, &S.pl));
-  const int NB = chunk_bands(nband, ctx->tune_fft_bands, 128 / (int)sizeof(cplx<T>));
+  const int NB = chunk_width<T>(ctx, S.pl, nband, ctx->tune_fft_bands);
   S.NB = NB;
   const long npts_grid = (long)fftg[0] * fftg[1] * fftg[2];
   S.ptot = sphere_ptot(sp);
@@ -296,7 +296,7 @@ static int aug_freqs_batched(pp_ctx *ctx, pp_sphere *sp, int nk, const double *k
   const int *fftg = sphere_fftg(sp);
   FftPlan *pl = nullptr;
   PP_TRY(get_fft_plan(ctx, fftg, &pl));
-  const int NB = chunk_bands(nband, 0, 128 / (int)sizeof(cplx<T>));
+  const int NB = chunk_width<T>(ctx, pl, nband, 0);
   const long npts_grid = (long)fftg[0] * fftg[1] * fftg[2];
   const long npts_sph = std::max<long>(1, sphere_npts(sp));
   PP_TRY(ctx->grid.ensure(sizeof(cplx<T>) * (size_t)npts_grid * NB));

@@ -264,7 +264,7 @@ extern "C" int pp_fft3d_batched(pp_ctx *ctx, const double *lattice, const int *f
   PP_TRY(get_fft_plan(ctx, fftg, &pl));
   const long npts = (long)fftg[0] * fftg[1] * fftg[2];
   bool f64 = precision == PP_FP64;
-  const int NB = chunk_bands(nband, 0, f64 ? 8 : 16);
+  const int NB = f64 ? chunk_width<double>(ctx, pl, nband, 0) : chunk_width<float>(ctx, pl, nband, 0);
   size_t csz = f64 ? sizeof(cplx<double>) : sizeof(cplx<float>);
   PP_TRY(ctx->grid.ensure(csz * (size_t)npts * NB));
   PP_TRY(ctx->gidx.ensure(sizeof(int) * (size_t)std::max(1, nw)));

@@ -755,6 +755,24 @@ template <typename T> bool fft_masked_stores(pp_ctx *ctx, FftPlan *pl, int NB) {
 }
 template bool fft_masked_stores<double>(pp_ctx *, FftPlan *, int);
 template bool fft_masked_stores<float>(pp_ctx *, FftPlan *, int);
+// Whether half a band group is worth a whole one.  The empty half costs its
+// traffic and the two-DFT passes gain less than that unless the chunk stays in
+// the 256 MB cache: setups of 8 FP32 bands with and without, 60^3 142 / 158 us,
+// 108^3 311 / 330, 150^3 573 / 567, 216^3 1396 / 1342 (its transform alone
+// 2344 / 1467); 4 FP64 bands on 150^3 790 / 740; 8 FP32 bands with the staged
+// passes of 99^3 587 / 483.
+template <typename T> bool fft_half_groups(pp_ctx *ctx, FftPlan *pl) {
+  constexpr int group = fft2_bands<T>();
+  long bytes = 128;
+  for (const AxisPlan &ap : pl->ax) {
+    if (!fft2_pass(ctx, ap, group, group))
+      return false;
+    bytes *= ap.n;
+  }
+  return bytes <= 256L << 20;
+}
+template bool fft_half_groups<double>(pp_ctx *, FftPlan *);
+template bool fft_half_groups<float>(pp_ctx *, FftPlan *);
 // Streaming access of a pass: fft_nt 0..2 for every pass; 3 keeps the z
 // pass's stores cacheable (the y pass reads them next), streams the y
 // pass's stores and both directions of the x pass.

@@ -217,12 +217,13 @@ int zero_async(pp_ctx *ctx, void *p, size_t bytes);
 // columns past the bands are transformed as they are and read by nobody):
 // 70 bands run as 48 + 22 rather than 64 + 6, 45 as one chunk of 48 whose
 // passes take whole groups (45 fell to the one-band tiles).  Less than half
-// a group stays as it is.  tune > 0 forces the width.
-inline int chunk_bands(int nband, int tune, int group) {
+// a group stays as it is, and half a group too unless `half`
+// (fft_half_groups).  tune > 0 forces the width.
+inline int chunk_bands(int nband, int tune, int group, bool half) {
   if (tune > 0)
     return std::max(1, std::min(std::min(tune, 64), nband));
   const int nch = std::max(1, (nband + 63) / 64), per = (std::max(1, nband) + nch - 1) / nch;
-  return 2 * per < group ? per : (per + group - 1) / group * group;
+  return 2 * per < group + (half ? 0 : 1) ? per : (per + group - 1) / group * group;
 }
 
 // Band-fastest grid chunk pipeline pieces (pp_fft.hip).
@@ -236,6 +237,11 @@ int fft_chunk(pp_ctx *ctx, FftPlan *pl, cplx<T> *grid, int NB, int nw, const int
 template <typename T> const cplx<T> *fft_twiddles(FftPlan *pl, int axis);
 template <typename T> int fft_passes(pp_ctx *ctx, FftPlan *pl, cplx<T> *grid, int NB);
 template <typename T> bool fft_masked_stores(pp_ctx *ctx, FftPlan *pl, int NB);
+template <typename T> bool fft_half_groups(pp_ctx *ctx, FftPlan *pl);
+// chunk_bands of a plan's passes
+template <typename T> int chunk_width(pp_ctx *ctx, FftPlan *pl, int nband, int tune) {
+  return chunk_bands(nband, tune, 128 / (int)sizeof(cplx<T>), fft_half_groups<T>(ctx, pl));
+}
 template <typename T>
 int gather_conj(pp_ctx *ctx, const cplx<T> *grid, int NB, int nbc, const int *gidx, int nw, double scl,
                 cplx<double> *out, long ldo);

@@ -89,8 +89,7 @@ static int multi_prepare(pp_ctx *ctx, const MultiArgs &a, const MultiBufs &mb, M
   for (int i = 0; i < a.nstruct * a.nk; i++)
     maxnb = std::max(maxnb, a.nband[i]);
   // more than one chunk for some item: 64, as the items' counts differ
-  const int NB = maxnb > 64 ? chunk_bands(64, ctx->tune_fft_bands, 1)
-                            : chunk_bands(maxnb, ctx->tune_fft_bands, 128 / (int)sizeof(cplx<T>));
+  const int NB = chunk_width<T>(ctx, S.pl, std::min(64, maxnb), ctx->tune_fft_bands);
   S.NB = NB;
   if (!fft_items_supported<T>(ctx, S.pl, NB))
     return PP_ERR_UNSUPPORTED;

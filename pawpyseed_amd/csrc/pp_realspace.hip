@@ -911,8 +911,8 @@ extern "C" int pp_realspace_batched(pp_ctx *ctx, pp_rsplan *rp, const double *kf
   FftPlan *pl = nullptr;
   PP_TRY(get_fft_plan(ctx, rp->fftg, &pl));
   const bool f64 = precision == PP_FP64;
-  const int group = f64 ? 8 : 16;
-  const int nbmax = chunk_bands(nband, 0, group);
+  auto width = [&](int nb) { return f64 ? chunk_width<double>(ctx, pl, nb, 0) : chunk_width<float>(ctx, pl, nb, 0); };
+  const int nbmax = width(nband);
   const size_t csz = f64 ? sizeof(cplx<double>) : sizeof(cplx<float>);
   bool tiles = ctx->tune_rs_kernel == 3;
   if (tiles)
@@ -963,7 +963,7 @@ extern "C" int pp_realspace_batched(pp_ctx *ctx, pp_rsplan *rp, const double *kf
   for (size_t c = 0; c < starts.size() && st == PP_OK; c++) {
     const int b0 = starts[c];
     const int nbc = std::min(nbmax, nband - b0);
-    const int NB = nbmax % group ? nbc : (nbc + group - 1) / group * group;
+    const int NB = width(nbc);
     const int sl = two ? (int)(c & 1) : 0;
     ctx->stream = streams[sl];
     ctx->slot = sl;

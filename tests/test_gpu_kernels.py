@@ -679,6 +679,34 @@ def test_two_dft_pass_pruned(ctx, fftg, nb, precision, tol):
     plan.close()
 
 
+@pytest.mark.parametrize("fftg,whole", [((20, 24, 28), True), ((66, 50, 40), False), ((160, 112, 126), False)])
+@pytest.mark.parametrize("precision,nb,tol", [("fp64", 4, 5e-15), ("fp32", 8, 2e-6)])
+def test_half_a_band_group(ctx, fftg, whole, precision, nb, tol):
+    """Half a 128-byte band group of bands takes a whole one only where all
+    three axes have two-DFT passes and the chunk fits the 256 MB cache; else
+    the chunk holds the bands alone (on 216^3 eight FP32 bands as sixteen took
+    1.6 times as long).  The transform against numpy, bounds as
+    test_two_dft_pass_lengths, and the memory a fresh context takes."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(nb)
+    G = np.unique(rng.integers(-6, 7, (60, 3)), axis=0).astype(np.int32)
+    C = (rng.standard_normal((nb, len(G))) + 1j * rng.standard_normal((nb, len(G)))).astype(np.complex64)
+    x = np.zeros((nb, *fftg), np.complex128)
+    x[:, G[:, 0], G[:, 1], G[:, 2]] = C
+    want = np.fft.ifftn(x, axes=(1, 2, 3), norm="forward")
+    out = torch.empty((nb, *fftg), dtype=torch.complex128, device="cuda")
+    Gd, Cd = torch.from_numpy(G).cuda(), torch.from_numpy(C).cuda()
+    fresh = B.Context(0)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    B.fft3d(fresh, np.eye(3), fftg, Gd, Cd, out, precision)
+    used = free - torch.cuda.mem_get_info()[0]
+    fresh.close()
+    assert normwise(out.cpu().numpy(), want) < tol
+    if not whole:
+        assert used < 64 * np.prod(fftg) + (48 << 20)  # 64 bytes a point, and small buffers
+
+
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-9), ("fp32", 1e-5)])
 def test_projections_g_set_with_holes(ctx, precision, tol):
     """A plane-wave list that is not a cutoff sphere (a random subset of
