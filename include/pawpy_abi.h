@@ -236,7 +236,8 @@ int pp_ctx_set_timing(pp_ctx *ctx, int enable);
 int pp_ctx_timing_read(pp_ctx *ctx, int n, const char **names,
                        double *ms_total, long *launches);
 int pp_ctx_timing_reset(pp_ctx *ctx);
-/* Tuning knobs (0 = automatic): bands per FFT chunk (<= 64), bands per
+/* Tuning knobs (0 = automatic): bands per FFT chunk (at most this many and
+ * 64; even chunks, in whole band groups where those fit), bands per
  * FFT work-group tile (power of two <= 32), FFT pruning to the plane-wave
  * sphere (1 on, 2 off), sphere-sum parts per site, GEMM split-K factor. */
 int pp_ctx_set_tuning(pp_ctx *ctx, int fft_bands, int fft_tile, int fft_prune,
@@ -256,8 +257,8 @@ int pp_ctx_set_tuning(pp_ctx *ctx, int fft_bands, int fft_tile, int fft_prune,
  * plan allows -- it writes no real-space grid but measured slower on the
  * 216-atom workload), "fft_xcd" (1: FFT pass work-groups walk
  * XCD-contiguous line ranges), "fft_fixed" (1, default: FFT passes along
- * axes of a compiled length -- the even ones with factors 2, 3, 5 and 7 up
- * to 256 and their usual doubles -- run as two register-level DFTs with one
+ * axes of a compiled length -- the even ones from 8 to 256 with factors 2,
+ * 3, 5 and 7, and 270, 280, 288, 300, 320, 324, 360 -- run as two register-level DFTs with one
  * LDS exchange when the chunk holds whole 128-byte band groups; 0: the
  * staged passes, which the fft_tile, fft_threads, fft_radix, fft_persistent
  * and fft_pingpong settings are for; the two agree to rounding), "fft_nt" (FFT passes: 0 cached, 1

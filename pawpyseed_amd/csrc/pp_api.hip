@@ -698,10 +698,10 @@ int pp_autotune(pp_ctx *ctx, pp_sphere *sp, int nk, const double *kfrac, const i
       {"sphere_parts", {0, 4, 16}},
       {"fft_radix", {0, 1}},
       {"fft_xcd", {0, 1}},
-      {"fft_xmask", {0, 1}},
+      {"fft_xmask", {-1, 0, 1}},
       {"fft_nt", {0, 1, 2, 3}},
       {"sphere_nt", {0, 1}},
-      {"fft_bands", {64, 32}},
+      {"fft_bands", {0, 32}},
   };
   if (fp32)
     cands.push_back({"fused", {0, 1}});

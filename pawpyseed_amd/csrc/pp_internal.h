@@ -213,17 +213,20 @@ int get_fft_plan(pp_ctx *ctx, const int *fftg, FftPlan **out);
 int zero_async(pp_ctx *ctx, void *p, size_t bytes);
 
 // Bands of a chunk for nband bands of 2 sizeof(T) bytes: as few chunks of at
-// most 64 as hold them, even ones, in whole 128-byte band groups (the
+// most 64 (or the fft_bands setting `tune`) as hold them, even ones, in whole 128-byte band groups (the
 // columns past the bands are transformed as they are and read by nobody):
 // 70 bands run as 48 + 22 rather than 64 + 6, 45 as one chunk of 48 whose
 // passes take whole groups (45 fell to the one-band tiles).  Less than half
 // a group stays as it is, and half a group too unless `half`
-// (fft_half_groups).  tune > 0 forces the width.
+// (fft_half_groups).  Where `tune` is too narrow for whole groups it is the
+// width.
 inline int chunk_bands(int nband, int tune, int group, bool half) {
-  if (tune > 0)
-    return std::max(1, std::min(std::min(tune, 64), nband));
-  const int nch = std::max(1, (nband + 63) / 64), per = (std::max(1, nband) + nch - 1) / nch;
-  return 2 * per < group + (half ? 0 : 1) ? per : (per + group - 1) / group * group;
+  const int most = tune > 0 ? std::min(tune, 64) : 64;
+  const int nch = std::max(1, (nband + most - 1) / most), per = (std::max(1, nband) + nch - 1) / nch;
+  const int whole = (per + group - 1) / group * group;
+  if (whole > most)
+    return std::min(most, std::max(1, nband));
+  return 2 * per < group + (half ? 0 : 1) ? per : whole;
 }
 
 // Band-fastest grid chunk pipeline pieces (pp_fft.hip).

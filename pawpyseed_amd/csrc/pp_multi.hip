@@ -396,7 +396,7 @@ int pp_autotune_multi(pp_ctx *ctx, int nstruct, pp_sphere *const *plans, int nk,
       {"sphere_parts", {0, 4, 16}},
       {"fft_nt", {0, 1, 2, 3}},
       {"sphere_nt", {0, 1}},
-      {"fft_xmask", {0, 1}},
+      {"fft_xmask", {-1, 0, 1}},
   };
   return autotune_core(
       ctx, cands,

@@ -103,6 +103,61 @@ def test_autotune_keeps_results(ctx):
         plan.close()
 
 
+def test_autotune_tries_the_defaults(ctx):
+    """The library's own choices (fft_bands 0, fft_xmask -1) are among the
+    values that both autotuners try, so that they can be the ones kept."""
+    from pawpyseed_amd.core import batched as B
+    wl, Gs, Cs, want = _case(nband=20)
+    Cd, Gd, gofs, nw = device_inputs(Gs, Cs)
+    labels = np.zeros(len(wl.frac_S), np.int32)
+    plan = B.SpherePlan(ctx, wl.lattice, wl.fftg, wl.frac_S, labels, [wl.species], "fp32")
+    out = torch.zeros((len(Gs), 20, plan.ptot), dtype=torch.complex128, device="cuda")
+    names = B.TUNED + ("multi_items",)
+    before = {n: ctx.get_param(n) for n in names}
+    assert before["fft_bands"] == 0 and before["fft_xmask"] == -1
+    try:
+        _, single = B.autotune(ctx, plan, wl.kpts, gofs, Gd, Cd, out, "fp32", repeats=1)
+        for n, v in before.items():
+            ctx.set_param(n, v)
+        _, multi = B.autotune_multi(ctx, [plan], wl.kpts, gofs, Gd, [[Cd[0], Cd[1]]], [[out[0], out[1]]], "fp32", repeats=1)
+    finally:
+        for n, v in before.items():
+            ctx.set_param(n, v)
+        plan.close()
+    assert 0 in [v for n, v, _ in single if n == "fft_bands"]
+    for trials in (single, multi):
+        assert -1 in [v for n, v, _ in trials if n == "fft_xmask"]
+
+
+@pytest.mark.parametrize("nband", [20, 45, 70])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_fft_bands_bounds_the_chunk(ctx, nband, precision):
+    """fft_bands = 64 bounds the chunk as 0 does and leaves its width to the
+    library, so a context tuned at one band count takes whole band groups at
+    another: the projections are the same bits as without it (the staged
+    passes, which other widths fall to, round differently).  A narrower bound
+    (24, 7) gives the same projections to rounding."""
+    from pawpyseed_amd.core import batched as B
+    wl, Gs, Cs, want = _case(nband)
+    Cd, Gd, gofs, nw = device_inputs(Gs, Cs)
+    labels = np.zeros(len(wl.frac_S), np.int32)
+    plan = B.SpherePlan(ctx, wl.lattice, wl.fftg, wl.frac_S, labels, [wl.species], precision)
+    outs = {}
+    try:
+        for bands in (0, 64, 24, 7):
+            ctx.set_param("fft_bands", bands)
+            out = torch.zeros((len(Gs), nband, plan.ptot), dtype=torch.complex128, device="cuda")
+            torch.cuda.synchronize()
+            B.setup_projections(ctx, plan, wl.kpts, gofs, Gd, Cd, out, precision)
+            outs[bands] = out.cpu().numpy()
+    finally:
+        ctx.set_param("fft_bands", 0)
+        plan.close()
+    assert np.array_equal(outs[64], outs[0])
+    for bands in (24, 7):
+        assert normwise(outs[bands], want) < (1e-9 if precision == "fp64" else 1e-5)
+
+
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-9), ("fp32", 1e-5)])
 def test_graph_replay_after_other_inputs(ctx, precision, tol):
     """A replay after eager calls on the same context with other k-points,
