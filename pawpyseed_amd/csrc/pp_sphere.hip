@@ -458,8 +458,8 @@ __device__ __forceinline__ void mfma_group(const float (&tab)[Q], const cplx<flo
 // projector guard in the loop, and 2Q MFMAs of 8 cycles per point where the
 // VALU form issued 8Q FMAs of 4.  Register v of accumulator q holds table
 // slot 4q + v of the lane's band.  A group's tail points repeat the last
-// point with phase 0 (the table values past the site's rows are other
-// sites' rows or the buffer's padding, both finite).
+// point, its table row included, with phase 0 (another site's row, or what
+// lies past the last one, need not be finite).
 template <int Q>
 __device__ __forceinline__ void sphere_sum_mfma(const cplx<float> *__restrict__ g, int NB, int p0, int len,
                                                 const int *__restrict__ pidx, const cplx<float> *__restrict__ phase,
@@ -481,10 +481,18 @@ __device__ __forceinline__ void sphere_sum_mfma(const cplx<float> *__restrict__ 
     idx = pidx[pt];
     const cplx<float> v = phase[pt];
     ph = l16 < n ? v : mk<float>(0, 0);
-    const float *ts = tsite + (long)(g0 - p0) * (4 * Q) + lane;
+    const float *ts = tsite + (long)(g0 - p0) * (4 * Q);
+    if (n == 16) {
 #pragma unroll
-    for (int r = 0; r < Q; r++)
-      tab[r] = ts[r * 64];
+      for (int r = 0; r < Q; r++)
+        tab[r] = ts[r * 64 + lane];
+    } else {
+#pragma unroll
+      for (int r = 0; r < Q; r++) {
+        const int at = r * 64 + lane;
+        tab[r] = ts[min(at / (4 * Q), n - 1) * (4 * Q) + at % (4 * Q)];
+      }
+    }
   };
   int g0 = a + wave * 16;
   if (g0 < e)
@@ -885,10 +893,7 @@ static int sphere_build(pp_sphere *sp) {
   PP_TRY(sp->d_proj_off.ensure(sizeof(int) * (ns + 1)));
   PP_TRY(sp->d_pidx.ensure(sizeof(int) * std::max<long>(1, sp->npts)));
   PP_TRY(sp->d_path.ensure(sizeof(double) * 3 * std::max<long>(1, sp->npts)));
-  // the FP32 sums read whole groups of 16 rows: padding past the last row
-  const long tpad = 16 * 64;
-  PP_TRY(sp->d_table.ensure(csz * (to + tpad)));
-  PP_TRY(zero_async(ctx, (char *)sp->d_table.p + csz * to, csz * tpad));
+  PP_TRY(sp->d_table.ensure(csz * std::max<long>(1, to)));
   PP_TRY(sp->d_seg_off.ensure(sizeof(int) * (ns + 1)));
   PP_TRY(sp->d_seg.ensure(sizeof(int4) * std::max<long>(1, sp->nseg)));
   PP_TRY(sp->d_segline.ensure(sizeof(int) * std::max<long>(1, sp->nseg)));

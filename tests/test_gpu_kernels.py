@@ -526,6 +526,34 @@ def test_augmentation_dense_delta_o_cfg0(ctx):
     assert e_or < 1e-11 and e_l < 1e-13
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_non_finite_projector_tables_stay_with_their_sites(ctx, precision):
+    """A species whose projector functions are NaN or infinite leaves the
+    projections of the other species' sites as they are: sums in groups of 16
+    points read no row of another site's table, nor past the last one."""
+    from pawpyseed_amd.core import batched as B
+    wl = synthetic.tiny_config(encut=150.0, fftg=(20, 20, 20), nband=5)
+    good, bad = wl.species, synthetic.make_species([0, 1, 2], [1.0, 2.0, 1.5], 1.0)
+    labels = (np.arange(len(wl.frac_S)) % 2).astype(np.int32)
+    Gs, Cs = wl.ensure_gvecs(), wl.coefficients("S", nband=5)
+    Cd, Gd, gofs, nw = device_inputs(Gs, Cs)
+    outs = []
+    for value in (None, np.nan, np.inf):
+        if value is not None:
+            bad.realprojs = [np.full_like(p, value) for p in bad.realprojs]
+        plan = B.SpherePlan(ctx, wl.lattice, wl.fftg, wl.frac_S, labels, [good, bad], precision)
+        out = torch.zeros((1, 5, plan.ptot), dtype=torch.complex128, device="cuda")
+        torch.cuda.synchronize()
+        B.setup_projections(ctx, plan, wl.kpts, gofs, Gd, Cd, out, precision)
+        outs.append(out.cpu().numpy())
+        off = plan.proj_off
+        plan.close()
+    mine = np.concatenate([np.arange(off[s], off[s + 1]) for s in range(len(labels)) if labels[s] == 0])
+    for o in outs[1:]:
+        assert np.array_equal(o[..., mine], outs[0][..., mine])
+        assert not np.isfinite(np.delete(o, mine, axis=2)).any()
+
+
 def test_empty_and_invalid_inputs(ctx):
     from pawpyseed_amd.core import batched as B
     from pawpyseed_amd.core._lib import PAWpyError
