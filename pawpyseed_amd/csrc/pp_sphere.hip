@@ -308,20 +308,20 @@ __global__ __launch_bounds__(256) void k_phase(long npts, const double *__restri
 }
 
 // Sphere sums of one (site, part of its points) by a work-group of 4
-// wavefronts, FP64; lane b of every wavefront accumulates the site's PM
-// table slots for band b of the chunk.  Tiles of TP points stage their
+// wavefronts, FP64; lane b of every wavefront accumulates PM table slots of
+// the site, from slot s0 of its rows of RW, for band b of the chunk.  Tiles of TP points stage their
 // table rows, phases and grid indices in LDS with coalesced loads; each
 // wavefront then takes every fourth point of the tile, U points per step
 // with their grid loads in flight together, and reads the table values as
 // LDS broadcasts.  The four wavefronts' sums are added in LDS at the end;
 // partial[(blk * PMX + j) * NB + b].
-template <typename T, int PM, int U>
+template <typename T, int PM, int U, int RW = PM>
 __device__ __forceinline__ void sphere_sum_valu(const cplx<T> *__restrict__ g, int NB, int p0, int len,
                                                 const int *__restrict__ pidx, const cplx<T> *__restrict__ phase,
                                                 const T *__restrict__ tsite, int a, int e,
                                                 cplx<T> *__restrict__ partial, int streaming,
                                                 T *__restrict__ s_tab, cplx<T> *__restrict__ s_ph,
-                                                int *__restrict__ s_idx) {
+                                                int *__restrict__ s_idx, int s0 = 0) {
   constexpr int TP = 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool active = lane < NB;
@@ -337,11 +337,11 @@ __device__ __forceinline__ void sphere_sum_valu(const cplx<T> *__restrict__ g, i
   cplx<T> pv = mk<T>(0, 0);
   for (int t0 = a; t0 < e; t0 += TP) {
     const int n = min(TP, e - t0);
-    const T *tsrc = tsite + (long)(t0 - p0) * PM;
+    const T *tsrc = tsite + (long)(t0 - p0) * RW + s0;
 #pragma unroll
     for (int u = 0; u < SL; u++) {
       const int q = tid + u * 256;
-      tv[u] = q < n * PM ? tsrc[q] : (T)0;
+      tv[u] = q < n * PM ? tsrc[RW == PM ? q : q / PM * RW + q % PM] : (T)0;
     }
     if (tid < n) {
       iv = pidx[t0 + tid];
@@ -415,7 +415,7 @@ __device__ __forceinline__ void sphere_sum_valu(const cplx<T> *__restrict__ g, i
   if (wave == 0 && active) {
 #pragma unroll
     for (int j = 0; j < PM; j++)
-      partial[(long)j * NB + lane] = acc[j];
+      partial[(long)(s0 + j) * NB + lane] = acc[j];
   }
 }
 
@@ -571,14 +571,35 @@ __device__ __forceinline__ void sphere_sum_block(const cplx<T> *__restrict__ g, 
   cplx<T> *o = partial + (long)blk * PM * NB;
   if constexpr (sizeof(T) == 4) {
     __shared__ float red[PM * 2 * 64];
-#define PP_BODY(C)                                                                                         if constexpr (C <= PM) {                                                                                   if (ts == C) {                                                                                             sphere_sum_mfma<C / 4>(g, NB, p0, len, pidx, phase, tsite, a, e, o, streaming, red);                     return;                                                                                                }                                                                                                      }
+#define PP_BODY(C)                                                                               \
+  if constexpr (C <= PM) {                                                                       \
+    if (ts == C) {                                                                               \
+      sphere_sum_mfma<C / 4>(g, NB, p0, len, pidx, phase, tsite, a, e, o, streaming, red);       \
+      return;                                                                                    \
+    }                                                                                            \
+  }
     PP_STRIDES_F32(PP_BODY)
 #undef PP_BODY
   } else {
-    __shared__ __align__(16) T s_tab[64 * (PM + 1)];
+    // Rows of 64 in two halves, which read the grid twice: the sums of 64
+    // slots take 512 registers a lane and spilled (64 sites of 845 points, 64
+    // bands, 64 projectors: setup of 768 us, in halves 503).
+    constexpr int PH = PM > 48 ? 48 : PM;
+    __shared__ __align__(16) T s_tab[64 * (PH + 1)];
     __shared__ cplx<T> s_ph[64];
     __shared__ int s_idx[64];
-#define PP_BODY(C)                                                                                         if constexpr (C <= PM) {                                                                                   if (ts == C) {                                                                                             sphere_sum_valu<T, C, U>(g, NB, p0, len, pidx, phase, tsite, a, e, o, streaming, s_tab, s_ph, s_idx);       return;                                                                                                }                                                                                                      }
+#define PP_BODY(C)                                                                                                   \
+  if constexpr (C <= PM) {                                                                                           \
+    if (ts == C) {                                                                                                   \
+      if constexpr (C > 48) {                                                                                        \
+        for (int s0 = 0; s0 < C; s0 += C / 2)                                                                        \
+          sphere_sum_valu<T, C / 2, U, C>(g, NB, p0, len, pidx, phase, tsite, a, e, o, streaming, s_tab, s_ph, s_idx, s0); \
+      } else {                                                                                                       \
+        sphere_sum_valu<T, C, U>(g, NB, p0, len, pidx, phase, tsite, a, e, o, streaming, s_tab, s_ph, s_idx);        \
+      }                                                                                                              \
+      return;                                                                                                        \
+    }                                                                                                                \
+  }
     PP_STRIDES_F64(PP_BODY)
 #undef PP_BODY
   }
