@@ -13,11 +13,12 @@
 
 namespace pp {
 
-template <typename TA, typename TB>
+// (with GA, column k of A is column acol[k] of its rows, as k_zgemm_mfma64)
+template <typename TA, typename TB, bool GA>
 __global__ __launch_bounds__(256) void k_zgemm_f64(int M, int N, int kbeg_stride, int K, int nsplit,
                                                    const cplx<TA> *__restrict__ A, long lda,
-                                                   const cplx<TB> *__restrict__ B, long ldb,
-                                                   cplx<double> *__restrict__ C, long ldc, long sSplit) {
+                                                   const int *__restrict__ acol, const cplx<TB> *__restrict__ B,
+                                                   long ldb, cplx<double> *__restrict__ C, long ldc, long sSplit) {
   __shared__ cplx<double> As[16][64 + 1];
   __shared__ cplx<double> Bs[16][64 + 1];
   const int tilesN = (N + 63) / 64;
@@ -44,7 +45,7 @@ __global__ __launch_bounds__(256) void k_zgemm_f64(int M, int N, int kbeg_stride
       cplx<double> va = mk<double>(0, 0), vb = mk<double>(0, 0);
       if (gk < k1) {
         if (gm < M)
-          va = cvt<double>(A[(long)gm * lda + gk]);
+          va = cvt<double>(A[(long)gm * lda + (GA ? acol[gk] : gk)]);
         if (gn < N)
           vb = cvt<double>(B[(long)gn * ldb + gk]);
       }
@@ -344,21 +345,25 @@ int launch_zgemm64(hipStream_t st, int M, int N, const GemmBatch &gb, int atype,
   return PP_OK;
 }
 
-// The VALU form of one batch (the gemm_f64_valu option).
-int launch_zgemm64_valu(hipStream_t st, int M, int N, int K, int atype, const void *A, long lda, int btype,
-                        const void *B, long ldb, cplx<double> *dst, long dld, long sSplit, int nsplit, int kchunk) {
+// The VALU form of one batch (the gemm_f64_valu option); acol as
+// launch_zgemm64.
+int launch_zgemm64_valu(hipStream_t st, int M, int N, int K, int atype, const void *A, long lda, const int *acol,
+                        int btype, const void *B, long ldb, cplx<double> *dst, long dld, long sSplit, int nsplit,
+                        int kchunk) {
   const dim3 grd = gemm_grid(((M + 63) / 64) * ((N + 63) / 64), nsplit);
-#define PP_MV(TA, TB)                                                                                          \
-  hipLaunchKernelGGL((k_zgemm_f64<TA, TB>), grd, dim3(256), 0, st, M, N, kchunk, K, nsplit, (const cplx<TA> *)A, lda, \
-                     (const cplx<TB> *)B, ldb, dst, dld, sSplit)
-  if (atype == 1 && btype == 1)
-    PP_MV(float, float);
+#define PP_MV(TA, TB, GA)                                                                                      \
+  hipLaunchKernelGGL((k_zgemm_f64<TA, TB, GA>), grd, dim3(256), 0, st, M, N, kchunk, K, nsplit, (const cplx<TA> *)A, \
+                     lda, acol, (const cplx<TB> *)B, ldb, dst, dld, sSplit)
+  if (acol)
+    PP_MV(double, double, true);
+  else if (atype == 1 && btype == 1)
+    PP_MV(float, float, false);
   else if (atype == 0 && btype == 0)
-    PP_MV(double, double);
+    PP_MV(double, double, false);
   else if (atype == 0 && btype == 1)
-    PP_MV(double, float);
+    PP_MV(double, float, false);
   else
-    PP_MV(float, double);
+    PP_MV(float, double, false);
 #undef PP_MV
   PP_CHECK_HIP(hipGetLastError());
   return PP_OK;
@@ -381,7 +386,7 @@ int launch_splitk_reduce(hipStream_t st, int M, int N, int nsplit, const void *P
 static int zgemm64_group(pp_ctx *ctx, int M, int N, const GemmBatch &gb, int atype, const void *A, long lda, long sA,
                          const int *acol, int btype, const void *B, long ldb, long sB, cplx<double> *C, long ldc,
                          long sC, bool accumulate, int cls) {
-  const bool valu = ctx->tune_gemm_f64_valu != 0 && !acol && gb.n == 1;
+  const bool valu = ctx->tune_gemm_f64_valu != 0;  // one batch a launch (zgemm64_nt)
   int nsplit, kchunk;
   zgemm64_split(M, N, gb, ctx->tune_splitk, atype == 0 && btype == 0, nsplit, kchunk);
   const bool direct = nsplit == 1 && !(valu && accumulate);
@@ -397,7 +402,7 @@ static int zgemm64_group(pp_ctx *ctx, int M, int N, const GemmBatch &gb, int aty
   const size_t ea = atype == 0 ? 16 : 8, eb = btype == 0 ? 16 : 8;
   hipEvent_t ev;
   tbegin(ctx, cls, &ev);
-  int st = valu ? launch_zgemm64_valu(ctx->stream, M, N, gb.k[0], atype, (const char *)A + gb.a[0] * sA * ea, lda,
+  int st = valu ? launch_zgemm64_valu(ctx->stream, M, N, gb.k[0], atype, (const char *)A + gb.a[0] * sA * ea, lda, acol,
                                       btype, (const char *)B + gb.b[0] * sB * eb, ldb, dst, dld, sSplit, nsplit, kchunk)
                 : launch_zgemm64(ctx->stream, M, N, gb, atype, A, lda, sA, acol, btype, B, ldb, sB, dst, dld, sSplit,
                                  sBatch, nsplit, kchunk, direct && accumulate);
@@ -416,7 +421,7 @@ int zgemm64_nt(pp_ctx *ctx, int M, int N, int K, int atype, const void *A, long 
                const int *amap, const int *bmap, const int *klen, bool accumulate) {
   if (M <= 0 || N <= 0)
     return PP_OK;
-  const int most = ctx->tune_gemm_f64_valu && !acol ? 1 : GemmBatch::MAX;
+  const int most = ctx->tune_gemm_f64_valu ? 1 : GemmBatch::MAX;
   for (int b0 = 0; b0 < nbatch; b0 += most) {
     GemmBatch gb;
     gb.n = std::min(most, nbatch - b0);

@@ -30,8 +30,9 @@ int launch_zgemm64(hipStream_t st, int M, int N, const GemmBatch &gb, int atype,
                    const int *acol, int btype, const void *B, long ldb, long sB, cplx<double> *dst, long dld,
                    long sSplit, long sBatch, int nsplit, int kchunk, bool accumulate);
 void zgemm64_split(int M, int N, const GemmBatch &gb, int tune, bool c128, int &nsplit, int &kchunk);
-int launch_zgemm64_valu(hipStream_t st, int M, int N, int K, int atype, const void *A, long lda, int btype,
-                        const void *B, long ldb, cplx<double> *dst, long dld, long sSplit, int nsplit, int kchunk);
+int launch_zgemm64_valu(hipStream_t st, int M, int N, int K, int atype, const void *A, long lda, const int *acol,
+                        int btype, const void *B, long ldb, cplx<double> *dst, long dld, long sSplit, int nsplit,
+                        int kchunk);
 int launch_splitk_reduce(hipStream_t st, int M, int N, int nsplit, const void *P, bool fp32_partials,
                          cplx<double> *C, long ldc, bool accumulate, int nbatch, long sP, long sC);
 
@@ -142,7 +143,7 @@ int pp_overlap_gemm_noalloc(pp_ctx *ctx, int nwk, int nspin, int flip, const int
       kchunk = (K + nsplit - 1) / nsplit;
       kchunk = std::max(16, (kchunk + 15) / 16 * 16);
       nsplit = std::max(1, (K + kchunk - 1) / kchunk);
-      PP_TRY(launch_zgemm64_valu(st, nbR, nbS, K, 1, A, ldR, 1, B, ldS, P, (long)nbS, (long)nbR * nbS, nsplit,
+      PP_TRY(launch_zgemm64_valu(st, nbR, nbS, K, 1, A, ldR, nullptr, 1, B, ldS, P, (long)nbS, (long)nbR * nbS, nsplit,
                                  kchunk));
     }
     // the next k-point's GEMM overwrites the partials only after this

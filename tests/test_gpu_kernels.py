@@ -554,6 +554,30 @@ def test_non_finite_projector_tables_stay_with_their_sites(ctx, precision):
         assert not np.isfinite(np.delete(o, mine, axis=2)).any()
 
 
+def test_f64_valu_option_reaches_the_augmentation(ctx):
+    """gemm_f64_valu = 1 takes the augmentation's GEMM too (columns of the
+    reference's projections gathered): the VALU form adds a term's two real
+    products in a row, 2^53 + 1 - 2^53 = 0 here, the matrix cores the first
+    products of four terms and then the second ones, which gives 1."""
+    from pawpyseed_amd.core import batched as B
+    sp = synthetic.make_species([0], [1.5], 1.1)
+    PR = torch.tensor([[[5.0, 2.0 ** 53 + 1j, -2.0 ** 53 + 0j]]], dtype=torch.complex128, device="cuda")
+    PS = torch.full((1, 1, 2), 1 + 1j, dtype=torch.complex128, device="cuda")
+    off, lab = np.arange(4, dtype=np.int32), np.zeros(3, np.int32)
+    got = {}
+    try:
+        for valu in (0, 1):
+            ctx.set_param("gemm_f64_valu", valu)
+            out = torch.zeros((1, 1, 1), dtype=torch.complex128, device="cuda")
+            torch.cuda.synchronize()
+            B.augmentation(ctx, 1, 1, False, PR, off, lab, PS, off[:3], lab[:2], np.array([1, 2], np.int32),
+                           np.array([0, 1], np.int32), [sp], [np.ones((1, 1))], out)
+            got[valu] = out.cpu().numpy()[0, 0, 0].real
+    finally:
+        ctx.set_param("gemm_f64_valu", 0)
+    assert got == {0: 1.0, 1: 0.0}
+
+
 def test_empty_and_invalid_inputs(ctx):
     from pawpyseed_amd.core import batched as B
     from pawpyseed_amd.core._lib import PAWpyError
