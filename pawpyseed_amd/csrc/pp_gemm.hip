@@ -318,6 +318,14 @@ void zgemm64_split(int M, int N, const GemmBatch &gb, int tune, bool c128, int &
   nsplit = std::max(1, (K + kchunk - 1) / kchunk);
 }
 
+// Batches of a launch.  A forced chunk count holds that many partial sums for
+// each of them: no more batches than keep those within what the policy's own
+// counts take (1536 tiles, 96 MiB), or one.
+int zgemm64_batches(int M, int N, int tune) {
+  const long part = 16L * M * N * std::max(1, tune);
+  return tune > 1 ? (int)std::max(1L, std::min<long>(GemmBatch::MAX, (96L << 20) / part)) : GemmBatch::MAX;
+}
+
 // FP64 MFMA GEMM of the batches gb: partials dst + batch * sBatch + split *
 // sSplit, or with nsplit == 1 the outputs themselves; kchunk a multiple of
 // 16.  acol (optional, FP64 operands): column map of A.  No allocation.
@@ -421,7 +429,7 @@ int zgemm64_nt(pp_ctx *ctx, int M, int N, int K, int atype, const void *A, long 
                const int *amap, const int *bmap, const int *klen, bool accumulate) {
   if (M <= 0 || N <= 0)
     return PP_OK;
-  const int most = ctx->tune_gemm_f64_valu ? 1 : GemmBatch::MAX;
+  const int most = ctx->tune_gemm_f64_valu ? 1 : zgemm64_batches(M, N, ctx->tune_splitk);
   for (int b0 = 0; b0 < nbatch; b0 += most) {
     GemmBatch gb;
     gb.n = std::min(most, nbatch - b0);

@@ -578,6 +578,30 @@ def test_f64_valu_option_reaches_the_augmentation(ctx):
     assert got == {0: 1.0, 1: 0.0}
 
 
+@pytest.mark.parametrize("nk,nb,splitk", [(16, 512, 64), (9, 40, 7), (20, 300, 3)])
+def test_forced_splitk_workspace(ctx, nk, nb, splitk):
+    """A forced chunk count holds the partial sums of no more k-points at once
+    than 96 MiB take, or of one: the memory a fresh context takes, and the
+    overlaps against numpy (1e-13 of the 2 nw that |a|^2 |b|^2 sum to)."""
+    from pawpyseed_amd.core import batched as B
+    nw = (1024 - 16 * np.arange(nk)).astype(np.int32)
+    gen = torch.Generator(device="cuda").manual_seed(nk)
+    R, S = (torch.randn((nk, nb, 1024), dtype=torch.complex64, device="cuda", generator=gen) for _ in range(2))
+    out = torch.zeros((nk, nb, nb), dtype=torch.complex128, device="cuda")
+    want = [(R[k, :, :n].to(torch.complex128).conj() @ S[k, :, :n].to(torch.complex128).T.contiguous())
+            for k, n in enumerate(int(n) for n in nw)]
+    fresh = B.Context(0)
+    fresh.set_param("gemm_splitk", splitk)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    B.overlap_gemm(fresh, nk, 1, False, nw, R, S, out, "fp64")
+    used = free - torch.cuda.mem_get_info()[0]
+    fresh.close()
+    for k in range(nk):
+        assert (out[k] - want[k]).abs().max().item() < 1e-13 * 2 * nw[k]
+    assert used < max(96 << 20, 16 * splitk * nb * nb) + (64 << 20)
+
+
 def test_empty_and_invalid_inputs(ctx):
     from pawpyseed_amd.core import batched as B
     from pawpyseed_amd.core._lib import PAWpyError
