@@ -30,6 +30,7 @@ int launch_zgemm64(hipStream_t st, int M, int N, const GemmBatch &gb, int atype,
                    const int *acol, int btype, const void *B, long ldb, long sB, cplx<double> *dst, long dld,
                    long sSplit, long sBatch, int nsplit, int kchunk, bool accumulate);
 void zgemm64_split(int M, int N, const GemmBatch &gb, int tune, bool c128, int &nsplit, int &kchunk);
+int zgemm64_batches(int M, int N, int tune);
 int launch_zgemm64_valu(hipStream_t st, int M, int N, int K, int atype, const void *A, long lda, const int *acol,
                         int btype, const void *B, long ldb, cplx<double> *dst, long dld, long sSplit, int nsplit,
                         int kchunk);
@@ -90,30 +91,39 @@ int pp_overlap_gemm_noalloc(pp_ctx *ctx, int nwk, int nspin, int flip, const int
   const int max_split64 = (int)(kScratchBytes / plane);  // FP64 partial planes that fit
   hipStream_t st = ctx->stream;
   if (precision == PP_FP64 && !ctx->tune_gemm_f64_valu) {
-    // the k-points of one launch and their K chunks as pp_overlap_gemm takes
-    // them where the partials fit the array; fewer of either where not
-    for (int k0 = 0; k0 < nkt;) {
-      GemmBatch gb;
-      gb.n = std::min({nkt - k0, (int)GemmBatch::MAX, max_split64});
-      for (int i = 0; i < gb.n; i++) {
+    // the K chunks of pp_overlap_gemm's groups of k-points, fewer where one
+    // k-point's partials would not fit the array; a group in as many launches
+    // as its partials take
+    const int most = zgemm64_batches(nbR, nbS, ctx->tune_splitk);
+    const long mn = (long)nbR * nbS;
+    for (int k0 = 0; k0 < nkt; k0 += most) {
+      GemmBatch all;
+      all.n = std::min(nkt - k0, most);
+      for (int i = 0; i < all.n; i++) {
         const int k = k0 + i;
-        gb.a[i] = (flip && nspin == 2) ? (k < nwk ? k + nwk : k - nwk) : k;
-        gb.b[i] = k;
-        gb.k[i] = nw[k];
+        all.a[i] = (flip && nspin == 2) ? (k < nwk ? k + nwk : k - nwk) : k;
+        all.b[i] = k;
+        all.k[i] = nw[k];
       }
       int nsplit, kchunk;
-      zgemm64_split(nbR, nbS, gb, ctx->tune_splitk, false, nsplit, kchunk);
-      if (nsplit > max_split64 / gb.n)
-        zgemm64_split(nbR, nbS, gb, max_split64 / gb.n, false, nsplit, kchunk);
-      const long mn = (long)nbR * nbS;
-      cplx<double> *C = (cplx<double> *)out_dev + k0 * mn;
+      zgemm64_split(nbR, nbS, all, ctx->tune_splitk, false, nsplit, kchunk);
+      if (nsplit > max_split64)
+        zgemm64_split(nbR, nbS, all, max_split64, false, nsplit, kchunk);
       const bool direct = nsplit == 1;
-      PP_TRY(launch_zgemm64(st, nbR, nbS, gb, 1, CR_dev, ldR, (long)nbR * ldR, nullptr, 1, CS_dev, ldS,
-                            (long)nbS * ldS, direct ? C : P, (long)nbS, mn, direct ? mn : mn * nsplit, nsplit, kchunk,
-                            false));
-      if (!direct)
-        PP_TRY(launch_splitk_reduce(st, nbR, nbS, nsplit, P, false, C, nbS, false, gb.n, mn * nsplit, mn));
-      k0 += gb.n;
+      const int part = direct ? all.n : max_split64 / nsplit;
+      for (int i0 = 0; i0 < all.n; i0 += part) {
+        GemmBatch gb;
+        gb.n = std::min(part, all.n - i0);
+        std::copy_n(all.a + i0, gb.n, gb.a);
+        std::copy_n(all.b + i0, gb.n, gb.b);
+        std::copy_n(all.k + i0, gb.n, gb.k);
+        cplx<double> *C = (cplx<double> *)out_dev + (k0 + i0) * mn;
+        PP_TRY(launch_zgemm64(st, nbR, nbS, gb, 1, CR_dev, ldR, (long)nbR * ldR, nullptr, 1, CS_dev, ldS,
+                              (long)nbS * ldS, direct ? C : P, (long)nbS, mn, direct ? mn : mn * nsplit, nsplit,
+                              kchunk, false));
+        if (!direct)
+          PP_TRY(launch_splitk_reduce(st, nbR, nbS, nsplit, P, false, C, nbS, false, gb.n, mn * nsplit, mn));
+      }
     }
     return PP_OK;
   }

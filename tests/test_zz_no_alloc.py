@@ -53,7 +53,7 @@ def test_noalloc_matches_overlap_gemm(ctx, prec):
         CR, CS, nw = _inputs(seed, nwk * nspin, nbR, nbS, W, ld)
         ref = torch.zeros((nwk * nspin, nbR, nbS), dtype=torch.complex128, device="cuda")
         got = torch.full_like(ref, complex(7.0, -7.0))
-        ctx.synchronize()
+        torch.cuda.synchronize()  # torch's stream makes the inputs, the context's reads them
         assert _call("pp_overlap_gemm", ctx, nwk, nspin, flip, nw, CR, CS, ref, prec) == 0
         assert _call("pp_overlap_gemm_noalloc", ctx, nwk, nspin, flip, nw, CR, CS, got, prec) == 0
         ctx.synchronize()
@@ -71,6 +71,30 @@ def test_noalloc_matches_overlap_gemm(ctx, prec):
                 want = a.conj() @ b.T
                 err = np.abs(got[k].cpu().numpy() - want).max() / np.abs(want).max()
                 assert err < 1e-12, (call, k, err)
+
+
+@pytest.mark.parametrize("nkt,nb,splitk", [(14, 600, 0), (18, 130, 0), (18, 130, 5), (5, 700, 12)])
+def test_noalloc_splits_as_overlap_gemm(ctx, nkt, nb, splitk):
+    """FP64: the K chunks are those of pp_overlap_gemm's groups of k-points
+    also where a group's partials take several launches (14 k-points of 600
+    bands: 11 planes fit the array), so the results are the same bits; as many
+    chunks as fit where even one k-point's do not (700 bands, 12 chunks: 8)."""
+    CR, CS, nw = _inputs(7, nkt, nb, nb, 2000, 2048)
+    ref = torch.zeros((nkt, nb, nb), dtype=torch.complex128, device="cuda")
+    got = torch.full_like(ref, complex(7.0, -7.0))
+    ctx.set_param("gemm_splitk", splitk)
+    try:
+        ctx.synchronize()
+        torch.cuda.synchronize()
+        assert _call("pp_overlap_gemm", ctx, nkt, 1, 0, nw, CR, CS, ref, 0) == 0
+        assert _call("pp_overlap_gemm_noalloc", ctx, nkt, 1, 0, nw, CR, CS, got, 0) == 0
+        ctx.synchronize()
+    finally:
+        ctx.set_param("gemm_splitk", 0)
+    if nb < 700:
+        assert torch.equal(got, ref)
+    else:
+        assert ((got - ref).abs().max() / ref.abs().max()).item() < 1e-12
 
 
 def test_noalloc_refuses_beyond_scratch(ctx):
