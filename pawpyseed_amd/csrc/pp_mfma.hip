@@ -421,7 +421,7 @@ __device__ __forceinline__ void stage(int mi, f32x4 &f0, f32x4 &f1, u32x4 (&g)[N
 // complex terms each), split into hi / lo planes on their way into LDS with
 // the same arithmetic, so that no plane buffer goes through HBM (fp16: the
 // exponents EA / EB of an exponent-only k_split_planes pass).
-template <int NT, int KS, bool F16, int CH, int WPE, bool CVT, int TMW>
+template <int NT, int KS, bool F16, int CH, int WPE, bool CVT, int TMW, bool ILV>
 __global__ __launch_bounds__(128 * TMW) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void k_cgemm_planes(
     int M, int N, int nsplit, int K, const void *__restrict__ Av, long lda, const void *__restrict__ Bv, long ldb,
     long sp, long cs, const int *__restrict__ EA, const int *__restrict__ EB, long sE, cplx<float> *__restrict__ C,
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(128 * TMW) __attribute__((amdgpu_waves_per_eu(WPE, 
             cr[mi][nj] = mfma16<F16>(a[i][mi], b[d - i], cr[mi][nj]);                                            \
             ci[mi][nj] = mfma16<F16>(a[i][mi], q[d - i], ci[mi][nj]);                                            \
           }                                                                                                      \
-          if (blk < NU) {                                                                                        \
+          if (ILV && blk < NU) {                                                                                 \
             const int h_ = blk / HP, q_ = blk % HP;                                                              \
             if (h_ < RA)                                                                                         \
               stage<WH, CVT, F16, NT, HP>(                                                                       \
@@ -598,8 +598,13 @@ __global__ __launch_bounds__(128 * TMW) __attribute__((amdgpu_waves_per_eu(WPE, 
                     q_, sb[(h_ - RA) % RB], xb[(h_ - RA) % RB], pb[(h_ - RA) % RB], sp, off_, nreal_left,        \
                     &Bs[buf ^ 1][0][(h_ - RA) % RB * RS + lrow][part * (KS / 4) + q_ * 8], 128 * LS);            \
           }                                                                                                      \
-          __builtin_amdgcn_sched_barrier(0);                                                                     \
+          if (ILV)                                                                                               \
+            __builtin_amdgcn_sched_barrier(0);                                                                   \
         }                                                                                                        \
+      }                                                                                                          \
+      if (!ILV) {                                                                                                \
+        PP_STASH(buf ^ 1);                                                                                       \
+        PP_FETCH(min(s + 2, nsteps - 1), WH);                                                                    \
       }                                                                                                          \
       __syncthreads();                                                                                           \
     }                                                                                                            \
@@ -763,10 +768,10 @@ int launch_plane_gemm(hipStream_t st, int precision, int M, int N, int K, const 
   const long sE = M + N;
   constexpr int CH = kPlaneChunk / 2;
 #define PP_PG(NTV, KSV, F, WPEV, CVTV, AA, LA, BB, LB, EE)                                                      \
-  hipLaunchKernelGGL((k_cgemm_planes<NTV, KSV, F, CH, WPEV, CVTV, 2>), grd, dim3(256), 0, st, M, N, nsplit, K, AA, LA,  \
+  hipLaunchKernelGGL((k_cgemm_planes<NTV, KSV, F, CH, WPEV, CVTV, 2, true>), grd, dim3(256), 0, st, M, N, nsplit, K, AA, LA,  \
                      BB, LB, sp, cs, EE, EE ? EE + M : nullptr, sE, P, ldp_out, sSplit)
 #define PP_PG4(F, AA, LA, BB, LB, EE)                                                                          \
-  hipLaunchKernelGGL((k_cgemm_planes<2, 32, F, CH, 2, true, 4>), grd4, dim3(512), 0, st, M, N, nsplit, K, AA, LA, BB, \
+  hipLaunchKernelGGL((k_cgemm_planes<2, 32, F, CH, 2, true, 4, true>), grd4, dim3(512), 0, st, M, N, nsplit, K, AA, LA, BB, \
                      LB, sp, cs, EE, EE ? EE + M : nullptr, sE, P, ldp_out, sSplit)
   const dim3 grd4 = gemm_grid(((M + 255) / 256) * ((N + 127) / 128), nsplit);
   const int *noE = nullptr;
@@ -774,6 +779,12 @@ int launch_plane_gemm(hipStream_t st, int precision, int M, int N, int K, const 
     PP_PG4(true, A, lda, B, ldb, E);
   else if (cvt && variant >= 4)
     PP_PG4(false, A, lda, B, ldb, noE);
+  else if (cvt && precision == PP_FP16X3 && (long)tiles * nsplit <= 256)
+    // at most one work-group per CU: nothing else runs beside a wavefront's
+    // products and the scheduling barriers only hold its loads back (512 x 512,
+    // K = 2000, 64 work-groups, six k-points: 983 us interleaved, 903 so)
+    hipLaunchKernelGGL((k_cgemm_planes<2, 32, true, CH, 2, true, 2, false>), grd, dim3(256), 0, st, M, N, nsplit, K, A,
+                       lda, B, ldb, sp, cs, E, E + M, sE, P, ldp_out, sSplit);
   else if (cvt && precision == PP_FP16X3)
     PP_PG(2, 32, true, 2, true, A, lda, B, ldb, E);
   else if (cvt)

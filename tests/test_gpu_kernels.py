@@ -602,6 +602,30 @@ def test_forced_splitk_workspace(ctx, nk, nb, splitk):
     assert used < max(96 << 20, 16 * splitk * nb * nb) + (64 << 20)
 
 
+@pytest.mark.parametrize("nw", [100, 32700, 33000])
+def test_overlap_fp16x3_loop_orders(ctx, nw):
+    """The GEMM that splits FP32 operands itself runs one loop order on at
+    most 256 work-groups (130 bands: 4 tiles of 2 to 64 chunks) and another
+    on more (66 chunks): both bit-identical to the one with planes split
+    beforehand."""
+    from pawpyseed_amd.core import batched as B
+    ld = -(-nw // 64) * 64
+    gen = torch.Generator(device="cuda").manual_seed(nw)
+    R, S = (torch.randn((1, 130, ld), dtype=torch.complex64, device="cuda", generator=gen) for _ in range(2))
+    got = []
+    before = ctx.get_param("gemm_planes")
+    try:
+        for gp in (2, 3):
+            ctx.set_param("gemm_planes", gp)
+            out = torch.zeros((1, 130, 130), dtype=torch.complex128, device="cuda")
+            torch.cuda.synchronize()
+            B.overlap_gemm(ctx, 1, 1, False, np.array([nw], np.int32), R, S, out, "fp16x3")
+            got.append(out.cpu().numpy())
+    finally:
+        ctx.set_param("gemm_planes", before)
+    assert np.array_equal(got[0], got[1])
+
+
 def test_empty_and_invalid_inputs(ctx):
     from pawpyseed_amd.core import batched as B
     from pawpyseed_amd.core._lib import PAWpyError
