@@ -739,10 +739,12 @@ int compute_gidx(pp_ctx *ctx, const int *fftg, int nw, const int *G_dev, int *gi
 
 // The two-DFT pass of an axis, where the length has one, the chunk holds
 // whole band groups and the staged forms are not asked for.
-static const Fft2Entry *fft2_pass(pp_ctx *ctx, const AxisPlan &ap, int NB, int bands) {
-  if (!ctx->tune_fft_fixed || ctx->tune_fft_pingpong || ctx->tune_fft_persistent || ctx->tune_fft_radix || NB % bands)
+template <typename T> static const Fft2Entry *fft2_pass(pp_ctx *ctx, const AxisPlan &ap, int NB) {
+  if (!ctx->tune_fft_fixed || ctx->tune_fft_pingpong || ctx->tune_fft_persistent || ctx->tune_fft_radix ||
+      NB % fft2_bands<T>())
     return nullptr;
-  return fft2_entry(ap.n);
+  const Fft2Entry *fe = fft2_entry(ap.n);
+  return fe && (sizeof(T) == 4 || fe->f64) ? fe : nullptr;
 }
 // Whether the x pass of a setup stores covered points only: fft_xmask, or by
 // itself with the two-DFT pass, whose stores the test costs nothing (216
@@ -751,7 +753,7 @@ static const Fft2Entry *fft2_pass(pp_ctx *ctx, const AxisPlan &ap, int NB, int b
 template <typename T> bool fft_masked_stores(pp_ctx *ctx, FftPlan *pl, int NB) {
   if (ctx->tune_fft_xmask >= 0)
     return ctx->tune_fft_xmask != 0;
-  return fft2_pass(ctx, pl->ax[0], NB, fft2_bands<T>()) != nullptr;
+  return fft2_pass<T>(ctx, pl->ax[0], NB) != nullptr;
 }
 template bool fft_masked_stores<double>(pp_ctx *, FftPlan *, int);
 template bool fft_masked_stores<float>(pp_ctx *, FftPlan *, int);
@@ -762,10 +764,9 @@ template bool fft_masked_stores<float>(pp_ctx *, FftPlan *, int);
 // 2344 / 1467); 4 FP64 bands on 150^3 790 / 740; 8 FP32 bands with the staged
 // passes of 99^3 587 / 483.
 template <typename T> bool fft_half_groups(pp_ctx *ctx, FftPlan *pl) {
-  constexpr int group = fft2_bands<T>();
   long bytes = 128;
   for (const AxisPlan &ap : pl->ax) {
-    if (!fft2_pass(ctx, ap, group, group))
+    if (!fft2_pass<T>(ctx, ap, fft2_bands<T>()))
       return false;
     bytes *= ap.n;
   }
@@ -897,7 +898,7 @@ static int launch_pass(pp_ctx *ctx, cplx<T> *grid, const AxisPlan &ap, const cpl
 template <typename T, int AXIS>
 static int run_pass(pp_ctx *ctx, cplx<T> *grid, const AxisPlan &ap, const cplx<T> *tw, long es, long s1, long s2,
                     int n1, int n2, int NB, int cls, const SphereBounds &bd) {
-  if (const Fft2Entry *fe = fft2_pass(ctx, ap, NB, fft2_bands<T>())) {
+  if (const Fft2Entry *fe = fft2_pass<T>(ctx, ap, NB)) {
     const long nlines = pass_lines(bd, AXIS);
     if (nlines == 0)
       return PP_OK;
@@ -1003,7 +1004,7 @@ static int launch_pass_items(pp_ctx *ctx, const ChunkItem *items, int nitems, lo
 template <typename T, int AXIS>
 static int run_pass_items(pp_ctx *ctx, const ChunkItem *items, int nitems, long maxlines, const AxisPlan &ap,
                           const cplx<T> *tw, long es, long s1, long s2, int n2, int NB, int cls) {
-  if (const Fft2Entry *fe = fft2_pass(ctx, ap, NB, fft2_bands<T>())) {
+  if (const Fft2Entry *fe = fft2_pass<T>(ctx, ap, NB)) {
     if (maxlines == 0 || nitems == 0)
       return PP_OK;
     const Fft2Args<T> a = fft2_args<T>(ctx, ap, tw, AXIS, es, s1, s2, n2, NB, maxlines);
@@ -1040,7 +1041,7 @@ template <typename T> bool fft_items_supported(pp_ctx *ctx, FftPlan *pl, int NB)
   int nbw = ctx->tune_fft_tile > 0 ? ctx->tune_fft_tile : (sizeof(T) == 4 ? 16 : 8);
   for (int a = 0; a < 3; a++) {
     const AxisPlan &ap = pl->ax[a];
-    if (fft2_pass(ctx, ap, NB, fft2_bands<T>()))
+    if (fft2_pass<T>(ctx, ap, NB))
       continue;
     int w = nbw;
     while (w > 1 && (NB % w != 0 || (size_t)2 * ap.n * w * sizeof(cplx<T>) > 64 * 1024))

@@ -21,8 +21,11 @@
 
 namespace pp {
 
-// Lengths with a pass, as X(N, R1, R2): the even lengths with factors 2, 3,
-// 5 and 7 up to 256 and their usual doubles, R1 and R2 at most 25.
+// Lengths with a pass, as X(N, R1, R2): the 50 even lengths from 8 to 256 with
+// factors 2, 3, 5 and 7, and above them seven of the doubled grids (270, 280,
+// 288, 300, 320, 324, 360).  294, 336, 378, 384 and 392 are no products of two
+// of the radices with a register-level DFT (at most 25); they, 350 and 400 run
+// the staged passes.
 #define PP_FFT2_A(X) X(8, 4, 2) X(10, 5, 2) X(12, 4, 3) X(14, 7, 2) X(16, 4, 4) X(18, 6, 3) X(20, 5, 4) X(24, 6, 4) \
   X(28, 7, 4) X(30, 6, 5) X(32, 8, 4) X(36, 6, 6) X(40, 8, 5) X(42, 7, 6) X(48, 8, 6)
 #define PP_FFT2_B(X) X(50, 10, 5) X(54, 9, 6) X(56, 8, 7) X(60, 10, 6) X(64, 8, 8) X(70, 10, 7) X(72, 9, 8) X(80, 10, 8)
@@ -49,12 +52,16 @@ template <typename T> constexpr int fft2_lanes(int R1, int R2) {
 // (four or more work-groups per CU), but two where 52 KiB hold them: the 256
 // contiguous bytes per element of two groups side by side run faster than
 // 128 (x pass of 108 in FP64 465 -> 421 us; two of 216 leave two work-groups
-// per CU, 3185 -> 3715).
+// per CU, 3185 -> 3715).  Two FP64 units of more than 256 threads do not get
+// two work-groups into a CU's registers and take turns with nobody: one (32
+// bands in FP64, z / y / x of 200: 200 / 576 / 1103 us against 282 / 796 /
+// 1629, of 162: 171 / 391 / 676 against 248 / 578 / 971).
 template <typename T> constexpr int fft2_lines(int R1, int R2) {
   const int rm = R1 > R2 ? R1 : R2, by_threads = 256 / (fft2_lanes<T>(R1, R2) * rm);
   const int row = R1 * R2 * 128, by_lds = 36 * 1024 / row, least = 2 * row <= 52 * 1024 ? 2 : 1;
   const int n = by_threads < by_lds ? by_threads : by_lds;
-  return n > least ? n : least;
+  const bool one = sizeof(T) == 8 && 2 * fft2_lanes<T>(R1, R2) * rm > 256;
+  return n > least ? n : one ? (n > 1 ? n : 1) : least;
 }
 template <typename T> constexpr int fft2_threads(int R1, int R2) {
   return fft2_lines<T>(R1, R2) * fft2_lanes<T>(R1, R2) * (R1 > R2 ? R1 : R2);
@@ -300,7 +307,7 @@ __global__ __launch_bounds__(fft2_threads<T>(R1, R2)) void k_fft2_items(const Ch
   fft2_tile<T, R1, R2>((cplx<T> *)it->grid, a, bd, (int)blockIdx.x, buf, twl, msk);
 }
 
-// Launchers of one length.
+// Launchers of one length (f64, items64: nullptr where FP64 has no such pass).
 struct Fft2Entry {
   int n, r1, r2;
   void (*f32)(hipStream_t, cplx<float> *, const Fft2Args<float> &, const SphereBounds &, bool);
@@ -323,9 +330,25 @@ void fft2_launch_items(hipStream_t st, const ChunkItem *items, int nitems, const
   hipLaunchKernelGGL((k_fft2_items<T, R1, R2>), dim3((unsigned)nblk, (unsigned)nitems), dim3(fft2_threads<T>(R1, R2)), 0,
                      st, items, a);
 }
-#define PP_FFT2_ENTRY(N, R1, R2)                                                                       \
-  {N, R1, R2, fft2_launch<float, R1, R2>, fft2_launch<double, R1, R2>, fft2_launch_items<float, R1, R2>, \
-   fft2_launch_items<double, R1, R2>},
+// FP64 passes stop at radix 20: the 25 complex values of a radix-25 half take
+// 210 registers, which leave two wavefronts per SIMD, and the staged pass is
+// the faster (32 bands in FP64, z / y / x of 250: 342 / 1309 / 3657 us against
+// 302 / 1023 / 2776; FP32 145 / 539 / 1518 against 178 / 602 / 1668).
+template <int R1, int R2> constexpr auto fft2_f64() {
+  if constexpr (R1 <= 20)
+    return fft2_launch<double, R1, R2>;
+  else
+    return nullptr;
+}
+template <int R1, int R2> constexpr auto fft2_items_f64() {
+  if constexpr (R1 <= 20)
+    return fft2_launch_items<double, R1, R2>;
+  else
+    return nullptr;
+}
+#define PP_FFT2_ENTRY(N, R1, R2)                                                                            \
+  {N, R1, R2, fft2_launch<float, R1, R2>, fft2_f64<R1, R2>(), fft2_launch_items<float, R1, R2>, \
+   fft2_items_f64<R1, R2>()},
 // A translation unit's entries (the lengths are spread over several so that
 // they compile in parallel), closed by n = 0.
 #define PP_FFT2_TABLE(NAME, LIST)                                  \

@@ -682,13 +682,11 @@ def test_xmask_writes_only_covered_points(ctx, precision):
 @pytest.mark.parametrize("fftg", [(108, 60, 216), (192, 108, 60)])
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-9), ("fp32", 1e-5)])
 def test_fixed_length_passes(ctx, fftg, precision, tol, wide):
-    """The FFT passes compiled for the axis lengths 60, 108, 192 and 216
-    (fft_fixed = 1, the default), with the default band tile (16 FP32, 8
-    FP64) and twice it, give the projections of the generic passes
-    (fft_fixed = 0) to rounding (the compiler contracts the complex
-    products into FMAs differently in the two forms, so they are not
-    bit-identical) and the oracle's (first 8 bands).  64 bands: a full
-    chunk, so the tiles are the ones the fixed passes are compiled for."""
+    """The two-DFT passes of a full chunk of 64 bands (fft_fixed = 1, the
+    default) give the projections of the staged passes (fft_fixed = 0), with
+    the staged passes' default band tile (16 FP32, 8 FP64) and twice it, to
+    rounding, and the oracle's (first 8 bands).  The tile changes the staged
+    passes alone: the two-DFT results are the same bits with either."""
     from pawpyseed_amd.core import batched as B
     nb = 64
     wl = synthetic.tiny_config(encut=150.0, fftg=fftg, nband=nb, kpts=[[0.25, -0.25, 0.1]], ls=(0, 1, 2),
@@ -701,19 +699,23 @@ def test_fixed_length_passes(ctx, fftg, precision, tol, wide):
     Cd, Gd, gofs, nw = device_inputs(Gs, Cs)
     plan = B.SpherePlan(ctx, wl.lattice, wl.fftg, wl.frac_S, labels, [wl.species], precision)
     outs = []
-    ctx.set_param("fft_tile", (32 if precision == "fp32" else 16) if wide else 0)
-    for fx in (0, 1):
-        ctx.set_param("fft_fixed", fx)
-        out = torch.zeros((1, nb, plan.ptot), dtype=torch.complex128, device="cuda")
-        B.setup_projections(ctx, plan, wl.kpts, gofs, Gd, Cd, out, precision)
-        torch.cuda.synchronize()
-        outs.append(out.cpu().numpy())
-    ctx.set_param("fft_fixed", 1)
-    ctx.set_param("fft_tile", 0)
+    tile = (32 if precision == "fp32" else 16) if wide else 0
+    try:
+        for fx, ft in ((0, tile), (1, tile), (1, 0)):
+            ctx.set_param("fft_fixed", fx)
+            ctx.set_param("fft_tile", ft)
+            out = torch.zeros((1, nb, plan.ptot), dtype=torch.complex128, device="cuda")
+            torch.cuda.synchronize()
+            B.setup_projections(ctx, plan, wl.kpts, gofs, Gd, Cd, out, precision)
+            outs.append(out.cpu().numpy())
+    finally:
+        ctx.set_param("fft_fixed", 1)
+        ctx.set_param("fft_tile", 0)
     err = normwise(outs[1][:, :8], want)
     diff = normwise(outs[1], outs[0])
-    print("fixed-length passes", fftg, precision, "wide" if wide else "", err, "against generic", diff, flush=True)
-    assert diff < tol / 10
+    print("two-DFT passes", fftg, precision, "wide" if wide else "", err, "against staged", diff, flush=True)
+    assert 0 < diff < tol / 10
+    assert np.array_equal(outs[2], outs[1])
     assert err < tol
     plan.close()
 
@@ -723,31 +725,67 @@ FFT2_LENGTHS = (8, 10, 12, 14, 16, 18, 20, 24, 28, 30, 32, 36, 40, 42, 48, 50, 5
                 252, 256, 270, 280, 288, 300, 320, 324, 360)
 
 
-@pytest.mark.parametrize("axis", [0, 1, 2])
-def test_two_dft_pass_lengths(ctx, axis):
-    """Every axis length with a two-DFT pass, on each axis, FP64 and FP32, in
-    chunks of whole band groups, of a rounded-up band count and of fewer
-    bands than half a group (the staged passes): the transform of random
-    coefficients at random G against numpy.  A length-n FP64 (FP32)
-    transform rounds by a few log2(n) times 1.1e-16 (6e-8), normwise."""
+def _transform_error(ctx, fftg, nb, precision, rng):
+    """normwise error of fft3d of random coefficients at random G against numpy"""
     from pawpyseed_amd.core import batched as B
+    G = np.unique(rng.integers([-(m // 2 - 1) for m in fftg], [m // 2 for m in fftg], (60, 3)), axis=0).astype(np.int32)
+    C = (rng.standard_normal((nb, len(G))) + 1j * rng.standard_normal((nb, len(G)))).astype(np.complex64)
+    x = np.zeros((nb, *fftg), np.complex128)
+    x[:, G[:, 0], G[:, 1], G[:, 2]] = C
+    want = np.fft.ifftn(x, axes=(1, 2, 3), norm="forward")
+    out = torch.empty((nb, *fftg), dtype=torch.complex128, device="cuda")
+    Gd, Cd = torch.from_numpy(G).cuda(), torch.from_numpy(C).cuda()
+    torch.cuda.synchronize()
+    B.fft3d(ctx, np.eye(3), fftg, Gd, Cd, out, precision)
+    return normwise(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("nb", [32, 13])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_two_dft_pass_lengths(ctx, axis, nb):
+    """Every axis length with a two-DFT pass, on each axis, FP64 and FP32, in
+    chunks of whole band groups (two in FP32, four in FP64) and of a
+    rounded-up band count.  A length-n FP64 (FP32) transform rounds by a few
+    log2(n) times 1.1e-16 (6e-8), normwise."""
     rng = np.random.default_rng(axis)
-    for i, n in enumerate(FFT2_LENGTHS):
+    for n in FFT2_LENGTHS:
         fftg = [10, 12, 14]
         fftg[axis] = n
-        nb = (64, 16, 13, 3)[i % 4]
-        G = np.unique(rng.integers([-(m // 2 - 1) for m in fftg], [m // 2 for m in fftg], (60, 3)), axis=0).astype(np.int32)
-        C = (rng.standard_normal((nb, len(G))) + 1j * rng.standard_normal((nb, len(G)))).astype(np.complex64)
-        x = np.zeros((nb, *fftg), np.complex128)
-        x[:, G[:, 0], G[:, 1], G[:, 2]] = C
-        want = np.fft.ifftn(x, axes=(1, 2, 3), norm="forward")
-        out = torch.empty((nb, *fftg), dtype=torch.complex128, device="cuda")
-        Gd, Cd = torch.from_numpy(G).cuda(), torch.from_numpy(C).cuda()
-        torch.cuda.synchronize()
         for precision, tol in (("fp64", 5e-15), ("fp32", 2e-6)):
-            B.fft3d(ctx, np.eye(3), fftg, Gd, Cd, out, precision)
-            err = normwise(out.cpu().numpy(), want)
+            err = _transform_error(ctx, fftg, nb, precision, rng)
             assert err < tol, (fftg, nb, precision, err)
+
+
+@pytest.mark.parametrize("fftg", [(14, 100, 36), (250, 84, 10), (12, 16, 324)])
+def test_staged_pass_lengths(ctx, fftg):
+    """Fewer bands than half a group take the staged passes on any length."""
+    rng = np.random.default_rng(fftg[0])
+    for precision, tol in (("fp64", 5e-15), ("fp32", 2e-6)):
+        assert _transform_error(ctx, fftg, 3, precision, rng) < tol
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_radix_25_passes_are_fp32_only(ctx, precision):
+    """A length-250 axis has a two-DFT pass in FP32 alone: in FP64 fft_fixed
+    changes nothing on it."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(43)
+    fftg, nb = (250, 11, 13), 16
+    G = np.unique(rng.integers(-4, 5, (60, 3)), axis=0).astype(np.int32)
+    C = (rng.standard_normal((nb, len(G))) + 1j * rng.standard_normal((nb, len(G)))).astype(np.complex64)
+    Gd, Cd = torch.from_numpy(G).cuda(), torch.from_numpy(C).cuda()
+    got = []
+    try:
+        for fx in (0, 1):
+            ctx.set_param("fft_fixed", fx)
+            out = torch.empty((nb, *fftg), dtype=torch.complex128, device="cuda")
+            torch.cuda.synchronize()
+            B.fft3d(ctx, np.eye(3), fftg, Gd, Cd, out, precision)
+            got.append(out.cpu().numpy())
+    finally:
+        ctx.set_param("fft_fixed", 1)
+    assert np.array_equal(got[0], got[1]) == (precision == "fp64")
+    assert normwise(got[1], got[0]) < (1e-14 if precision == "fp64" else 2e-6)
 
 
 @pytest.mark.parametrize("fftg", [(80, 54, 56), (54, 98, 30), (126, 28, 50), (36, 42, 150)])
