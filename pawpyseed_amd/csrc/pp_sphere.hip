@@ -487,11 +487,11 @@ __device__ __forceinline__ void sphere_sum_mfma(const cplx<float> *__restrict__ 
       for (int r = 0; r < Q; r++)
         tab[r] = ts[r * 64 + lane];
     } else {
+      int l = lane;
+      asm volatile("" : "+v"(l));  // keeps this branch's indices out of the loop's registers
 #pragma unroll
-      for (int r = 0; r < Q; r++) {
-        const int at = r * 64 + lane;
-        tab[r] = ts[min(at / (4 * Q), n - 1) * (4 * Q) + at % (4 * Q)];
-      }
+      for (int r = 0; r < Q; r++)
+        tab[r] = ts[min((r * 64 + l) / (4 * Q), n - 1) * (4 * Q) + (r * 64 + l) % (4 * Q)];
     }
   };
   int g0 = a + wave * 16;
