@@ -515,7 +515,7 @@ __device__ __forceinline__ void sphere_sum_mfma(const cplx<float> *__restrict__ 
       fetch(g0 + 64);
     mfma_group<Q>(tc, x, pc, ar, ai);
   }
-  // add the four wavefronts' sums: 2, 3 onto 0, 1, then 1 onto 0
+  // add the four wavefronts' sums: 3, 2 and 1 onto 0, in turn
   auto put = [&](float *dst) {
 #pragma unroll
     for (int q = 0; q < Q; q++)
@@ -1027,13 +1027,21 @@ int sphere_sums(pp_ctx *ctx, pp_sphere *sp, const cplx<T> *grid, int NB, int nbc
 // Sphere-sum parts per site of a plan: the tuning value, else enough for
 // about 2048 work-groups (eight per CU), of at least 64 points each (one
 // group of 16 per wavefront): a cell of 8 sites of 270 points runs 32
-// work-groups of one group per wavefront instead of 8 of four.
+// work-groups of one group per wavefront instead of 8 of four.  FP32 takes
+// nine per CU: the matrix cores' sums are a little further from the FP64 ones
+// than fused multiply-adds were, and the parts are added in FP64 (215 sites of
+// 4,853 points, error of the projections with VALU sums in 10 parts 1.110e-7,
+// on the matrix cores in 10 / 11 / 14 parts 1.131e-7 / 1.105e-7 / 1.058e-7,
+// sums and reduction of a chunk 151 / 150 / 149 us, of eight chunks in one
+// launch 7.71 / 7.75 / 8.02 ms; 512 sites of 11,499 in 4 and 5 parts 2.10e-7
+// and 1.84e-7, 733 and 736 us).
 int sphere_parts_of(pp_ctx *ctx, pp_sphere *sp) {
   if (ctx->tune_sphere_parts > 0)
     return ctx->tune_sphere_parts;
   const int ns = std::max(1, sp->nsites);
   const long most = std::max<long>(1, sp->npts / ns / 64);
-  return (int)std::min<long>((2048 + ns - 1) / ns, most);
+  const int wgs = sp->precision == PP_FP64 ? 2048 : 2304;
+  return (int)std::min<long>((wgs + ns - 1) / ns, most);
 }
 // Widest table row of a plan: the sum kernel that serves it.
 int sphere_pm_of(pp_sphere *sp) { return table_stride(sp->pmax, sp->precision != PP_FP64); }

@@ -626,6 +626,34 @@ def test_overlap_fp16x3_loop_orders(ctx, nw):
     assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("ncell,n,nb,tol", [(3, 108, 16, 1.11e-7), (4, 192, 8, 2.0e-7)])
+def test_fp32_projection_error(ctx, ncell, n, nb, tol):
+    """FP32 projections of the 216- and 512-atom cells against the FP64 ones,
+    2-norm: no further off than with VALU sums in 10 and 4 parts a site after
+    staged transforms (1.115e-7 and 2.05e-7 here)."""
+    from pawpyseed_amd.core import batched as B
+    rng = np.random.default_rng(3)
+    lattice, frac = synthetic.diamond_cell(ncell)
+    frac = np.mod(frac + rng.normal(0, 0.05, frac.shape) @ np.linalg.inv(lattice), 1.0)
+    kp = np.array([[0.25, -0.1, 0.3]])
+    G = synthetic.gvectors(lattice, kp[0], 520.0)
+    env = np.exp(-2.0 * (np.linalg.norm(G, axis=1) / np.linalg.norm(G, axis=1).max()) ** 2)
+    C = ((rng.standard_normal((nb, len(G))) + 1j * rng.standard_normal((nb, len(G)))) * env).astype(np.complex64)
+    Cd, Gd, gofs, nw = device_inputs([G], [C])
+    sp = synthetic.make_species([0, 0, 1, 1, 2, 2], [1.5, 3.0] * 3, 1.6)
+    outs = []
+    for precision in ("fp64", "fp32"):
+        plan = B.SpherePlan(ctx, lattice, np.full(3, n, np.int32), frac, np.zeros(len(frac), np.int32), [sp], precision)
+        out = torch.zeros((1, nb, plan.ptot), dtype=torch.complex128, device="cuda")
+        torch.cuda.synchronize()
+        B.setup_projections(ctx, plan, kp, gofs, Gd, Cd, out, precision)
+        outs.append(out)
+        plan.close()
+    err = ((outs[1] - outs[0]).norm() / outs[0].norm()).item()
+    print("FP32 projections", n, "error", err, flush=True)
+    assert err < tol
+
+
 def test_empty_and_invalid_inputs(ctx):
     from pawpyseed_amd.core import batched as B
     from pawpyseed_amd.core._lib import PAWpyError
