@@ -534,8 +534,8 @@ typedef struct pp_rsplan pp_rsplan;
  * partial-wave differences diffwave = r (phi - phi~) on it (projector.c:
  * 84-99; [nchan][wave_n] per species, concatenated).  A site's sphere
  * holds the box points (density.c:266-284) within the last point of its
- * wave grid; the table of (diffwave/r) Y_lm per point and projector is
- * built once.  Projectors of a site: channels in order, m = -l..l. */
+ * wave grid; tables of (diffwave/r) Y_lm per point and projector are
+ * built on its first use.  Projectors of a site: channels in order, m = -l..l. */
 int pp_rs_plan_create(pp_ctx *ctx, pp_rsplan **out, const double *lattice,
                       const int *fftg, int num_sites, const int *labels,
                       const double *frac_coords, int num_elems,
@@ -555,7 +555,9 @@ int pp_rs_plan_info(pp_rsplan *plan, int *total_projs, long *total_points,
  * partial-wave differences weighted by proj_dev (c128 [nband][ldp], the
  * plan's projector order).  Outputs (either may be NULL): states_dev c128
  * [nband][ldo] (x slowest) and density_dev f64 [N^3] += sum_b weights[b]
- * |psi_b|^2 (weights: host [nband]).  precision: PP_FP64 or PP_FP32 FFT.
+ * |psi_b|^2 (weights: host [nband]).  precision: PP_FP64 or PP_FP32 FFT
+ * (scale, Bloch phase and augmentation are FP64 either way).  The tables of
+ * the augmentation kernel in use are built on a plan's first call.
  * Asynchronous on the context's stream after one host synchronisation
  * (the plane-wave bounds); with the "streams" parameter at 2 two 64-band
  * chunks are in flight on two streams, joined into the context's stream

@@ -378,13 +378,27 @@ void k_rs_tiles(cplx<T> *__restrict__ g, RsTileArgs L) {
     if (KS > 0 && i < i1) {
       const int vid = __builtin_amdgcn_readfirstlane(s_vid[zi * RS_E]);
       const cplx<double> *cb = L.coef + ((long)vid * ks * 4 + row) * L.NB;
+      // a group's coefficients are loaded before the products of the group
+      // before it (left alone the compiler waits for each load ahead of its two
+      // products: density of 64 bands and 18 projectors on 108^3, FP64 1466
+      // against 1306 us, FP32 990 against 890; one group at a time keeps to the
+      // registers of three wavefronts per SIMD, all groups at once spill)
+      cplx<double> q[2][PL];
+      auto coefs = [&](int j) {
+#pragma unroll
+        for (int c = 0; c < PL; c++)
+          q[j & 1][c] = cb[j * 4 * L.NB + at[c]];
+      };
+      coefs(0);
 #pragma unroll
       for (int j = 0; j < KS; j++) {
+        if (j + 1 < KS)
+          coefs(j + 1);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 0; c < PL; c++) {
-          const cplx<double> q = cb[j * 4 * L.NB + at[c]];
-          dr[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(tf[j], q.x, dr[c], 0, 0, 0);
-          di[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(tf[j], q.y, di[c], 0, 0, 0);
+          dr[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(tf[j], q[j & 1][c].x, dr[c], 0, 0, 0);
+          di[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(tf[j], q[j & 1][c].y, di[c], 0, 0, 0);
         }
       }
       i++;
@@ -395,14 +409,36 @@ void k_rs_tiles(cplx<T> *__restrict__ g, RsTileArgs L) {
       const int vid = __builtin_amdgcn_readfirstlane(i - i0 < RS_E ? s_vid[zi * RS_E + i - i0] : L.ent[i].x);
       const double *ta = L.tab + (long)i * ks * 64 + lane;
       const cplx<double> *cb = L.coef + ((long)vid * ks * 4 + row) * L.NB;
+      if constexpr (KS > 0) {
+        cplx<double> q[2][PL];
+        double av[2];
+        auto load = [&](int j) {
+          av[j & 1] = ta[j * 64];
 #pragma unroll
-      for (int j = 0; j < ks; j++) {
-        const double av = ta[j * 64];
+          for (int c = 0; c < PL; c++)
+            q[j & 1][c] = cb[j * 4 * L.NB + at[c]];
+        };
+        load(0);
 #pragma unroll
-        for (int c = 0; c < PL; c++) {
-          const cplx<double> q = cb[j * 4 * L.NB + at[c]];
-          dr[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, q.x, dr[c], 0, 0, 0);
-          di[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, q.y, di[c], 0, 0, 0);
+        for (int j = 0; j < KS; j++) {
+          if (j + 1 < KS)
+            load(j + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int c = 0; c < PL; c++) {
+            dr[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[j & 1], q[j & 1][c].x, dr[c], 0, 0, 0);
+            di[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[j & 1], q[j & 1][c].y, di[c], 0, 0, 0);
+          }
+        }
+      } else {
+        for (int j = 0; j < ks; j++) {
+          const double av = ta[j * 64];
+#pragma unroll
+          for (int c = 0; c < PL; c++) {
+            const cplx<double> q = cb[j * 4 * L.NB + at[c]];
+            dr[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, q.x, dr[c], 0, 0, 0);
+            di[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, q.y, di[c], 0, 0, 0);
+          }
         }
       }
     }
