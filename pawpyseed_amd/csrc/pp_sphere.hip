@@ -188,6 +188,10 @@ __global__ __launch_bounds__(256) void k_seg_len(int4 *__restrict__ seg, long ns
   seg[q].y = end - sg.x;
 }
 
+// Rows of zeros behind a site's FP32 table: the sums read its rows in whole
+// groups of 16.  (Clamping the rows in the sums instead cost them 3%: 216^3,
+// 215 sites, 16 bands 676 -> 693 us.)
+constexpr int TAB_PAD = 15;
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_site_values(const SiteGeo *__restrict__ geo, Lat9 L, int f0, int f1, int f2,
@@ -198,8 +202,13 @@ __global__ __launch_bounds__(256) void k_site_values(const SiteGeo *__restrict__
   const SiteGeo s = geo[s_id];
   const int p0 = site_pt[s_id], np = site_pt[s_id + 1] - p0;
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= np)
+  if (i >= np) {
+    const int w = table_stride(s.nproj, sizeof(T) == 4);
+    if (sizeof(T) == 4 && i < np + TAB_PAD)
+      for (int p = 0; p < w; p++)
+        table[tab_off[s_id] + (long)i * w + p] = (T)0;
     return;
+  }
   const int fftg[3] = {f0, f1, f2};
   int g = pidx[p0 + i];
   int kk = g % fftg[2];
@@ -458,8 +467,8 @@ __device__ __forceinline__ void mfma_group(const float (&tab)[Q], const cplx<flo
 // projector guard in the loop, and 2Q MFMAs of 8 cycles per point where the
 // VALU form issued 8Q FMAs of 4.  Register v of accumulator q holds table
 // slot 4q + v of the lane's band.  A group's tail points repeat the last
-// point, its table row included, with phase 0 (another site's row, or what
-// lies past the last one, need not be finite).
+// point with phase 0; their table rows are the next part's of the site or the
+// zeros behind its last one (TAB_PAD), since another site's need not be finite.
 template <int Q>
 __device__ __forceinline__ void sphere_sum_mfma(const cplx<float> *__restrict__ g, int NB, int p0, int len,
                                                 const int *__restrict__ pidx, const cplx<float> *__restrict__ phase,
@@ -481,18 +490,10 @@ __device__ __forceinline__ void sphere_sum_mfma(const cplx<float> *__restrict__ 
     idx = pidx[pt];
     const cplx<float> v = phase[pt];
     ph = l16 < n ? v : mk<float>(0, 0);
-    const float *ts = tsite + (long)(g0 - p0) * (4 * Q);
-    if (n == 16) {
+    const float *ts = tsite + (long)(g0 - p0) * (4 * Q) + lane;
 #pragma unroll
-      for (int r = 0; r < Q; r++)
-        tab[r] = ts[r * 64 + lane];
-    } else {
-      int l = lane;
-      asm volatile("" : "+v"(l));  // keeps this branch's indices out of the loop's registers
-#pragma unroll
-      for (int r = 0; r < Q; r++)
-        tab[r] = ts[min((r * 64 + l) / (4 * Q), n - 1) * (4 * Q) + (r * 64 + l) % (4 * Q)];
-    }
+    for (int r = 0; r < Q; r++)
+      tab[r] = ts[r * 64];
   };
   int g0 = a + wave * 16;
   if (g0 < e)
@@ -901,7 +902,8 @@ static int sphere_build(pp_sphere *sp) {
     sp->site_pt_h[s + 1] = sp->site_pt_h[s] + counts[s];
     sp->seg_off_h[s + 1] = sp->seg_off_h[s] + counts[ns + s];
     tab_off[s] = to;
-    to += (long)counts[s] * table_stride(sp->nproj_site[s], sp->precision != PP_FP64);
+    to += (long)(counts[s] + (sp->precision != PP_FP64 ? TAB_PAD : 0)) *
+          table_stride(sp->nproj_site[s], sp->precision != PP_FP64);
     if (counts[s] > maxcount)
       maxcount = counts[s];
   }
@@ -949,7 +951,7 @@ static int sphere_build(pp_sphere *sp) {
     PP_CHECK_HIP(hipGetLastError());
   }
   if (maxcount > 0) {
-    dim3 grd((maxcount + 255) / 256, ns);
+    dim3 grd((maxcount + TAB_PAD + 255) / 256, ns);
     tbegin(ctx, K_TABLE, &ev);
     if (sp->precision == PP_FP64)
       hipLaunchKernelGGL(k_site_values<double>, grd, dim3(256), 0, ctx->stream, (const SiteGeo *)sp->d_sitemeta.p,
