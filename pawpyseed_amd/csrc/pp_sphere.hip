@@ -1029,20 +1029,21 @@ int sphere_sums(pp_ctx *ctx, pp_sphere *sp, const cplx<T> *grid, int NB, int nbc
 // Sphere-sum parts per site of a plan: the tuning value, else enough for
 // about 2048 work-groups (eight per CU), of at least 64 points each (one
 // group of 16 per wavefront): a cell of 8 sites of 270 points runs 32
-// work-groups of one group per wavefront instead of 8 of four.  FP32 takes
-// nine per CU: the matrix cores' sums are a little further from the FP64 ones
+// work-groups of one group per wavefront instead of 8 of four.  FP32 rows of
+// up to 32 take nine per CU: the matrix cores' sums are a little further from the FP64 ones
 // than fused multiply-adds were, and the parts are added in FP64 (215 sites of
 // 4,853 points, error of the projections with VALU sums in 10 parts 1.110e-7,
 // on the matrix cores in 10 / 11 / 14 parts 1.131e-7 / 1.105e-7 / 1.058e-7,
 // sums and reduction of a chunk 151 / 150 / 149 us, of eight chunks in one
 // launch 7.71 / 7.75 / 8.02 ms; 512 sites of 11,499 in 4 and 5 parts 2.10e-7
-// and 1.84e-7, 733 and 736 us).
+// and 1.84e-7, 733 and 736 us).  Wider rows write as much in partial sums as
+// they gather (64 sites, 64 projectors: setup 275 us, with nine 287).
 int sphere_parts_of(pp_ctx *ctx, pp_sphere *sp) {
   if (ctx->tune_sphere_parts > 0)
     return ctx->tune_sphere_parts;
   const int ns = std::max(1, sp->nsites);
   const long most = std::max<long>(1, sp->npts / ns / 64);
-  const int wgs = sp->precision == PP_FP64 ? 2048 : 2304;
+  const int wgs = sp->precision == PP_FP64 || sp->pmax > 32 ? 2048 : 2304;
   return (int)std::min<long>((wgs + ns - 1) / ns, most);
 }
 // Widest table row of a plan: the sum kernel that serves it.
