@@ -748,8 +748,9 @@ template <typename T> static const Fft2Entry *fft2_pass(pp_ctx *ctx, const AxisP
 }
 // Whether the x pass of a setup stores covered points only: fft_xmask, or by
 // itself with the two-DFT pass, whose stores the test costs nothing (216
-// atoms: x pass 210 -> 181 us per chunk, 64 atoms FP64 89 -> 56); the staged
-// passes are bound by their instructions and lose (setup 20.6 -> 21.5 ms).
+// atoms: x pass 206 -> 165 us per chunk, 64 atoms FP64 83 -> 52).  The staged
+// passes are bound by their instructions, so that it saves them little (216
+// atoms 252 -> 245 us, 96 atoms 45.5 -> 46.6), and store every point.
 template <typename T> bool fft_masked_stores(pp_ctx *ctx, FftPlan *pl, int NB) {
   if (ctx->tune_fft_xmask >= 0)
     return ctx->tune_fft_xmask != 0;

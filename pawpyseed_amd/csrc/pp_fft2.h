@@ -9,11 +9,11 @@
 // element makes one LDS round trip and the work-group two barriers; the
 // staged form made one round trip and two barriers per radix plus one for
 // the line (four or five for the usual lengths).  Per 64-band FP32 chunk on
-// 80 x 54 x 54: x 46.9 -> 35.5 us, y 44.8 -> 23.8, z 29.1 -> 16.5 against the
-// run-time staged passes, which those lengths had; on 108^3 the passes move
-// at the memory's rate in both forms (x 232 -> 210, y 110 -> 109, z 54 -> 49).  Eight or sixteen lanes
-// hold a line's band group, so each of their global and LDS accesses is one
-// contiguous 128 bytes and LDS reads and writes are free of bank conflicts.
+// 80 x 54 x 54: x 45.5 -> 35.2 us, y 44.8 -> 23.2, z 28.8 -> 16.0 against the
+// run-time staged passes; on 108^3 x 252 -> 206, y 134 -> 96, z 64 -> 45, near
+// the memory's rate.  Eight or sixteen lanes hold a line's band group, so each
+// of their global and LDS accesses is one contiguous 128 bytes and LDS reads
+// and writes are free of bank conflicts.
 #pragma once
 #include "pp_dft.h"
 #include "pp_internal.h"

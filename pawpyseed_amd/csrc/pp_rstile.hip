@@ -16,9 +16,10 @@
 //
 // A read-modify-write of every sphere point per colour and a read of the
 // whole chunk for the density become one read: 216^3 x 64 bands in FP64,
-// 4.5 + 1.8 ms before, 3.5 now (13.2 GB, 3.9 TB/s).  What bounds it is the
-// latency of the loads at three wavefronts per SIMD: the matrix units are
-// busy a quarter of it.  Tiles of 8 bands with interleaved parts, 8-byte loads and
+// 4.5 + 1.8 ms before, 2.84 now (13.2 GB, 4.6 TB/s; 3.4 with the coefficients
+// loaded where they are used; FP32 2.29, 3.19).  What bounds it is the latency
+// of the loads at three wavefronts per SIMD: the matrix units are busy under a third
+// of it.  Tiles of 8 bands with interleaved parts, 8-byte loads and
 // the blocks of x fastest took 5.8 ms, without the first entry's table values
 // loaded a step ahead 4.0 ms.  A form that also ran the x pass, so that
 // the chunk was never written, read each table row once per band group, 33 GB
@@ -27,7 +28,7 @@
 // Work lists: an entry is a (site, lattice image) whose sphere holds points
 // of one block; its table holds the site's partial-wave differences at the
 // block's points, zero outside the sphere, laid out as the MFMA reads it.
-// The plan builds them once: every (site, y, z) of the sites' boxes counts
+// The plan's first use builds them once: every (site, y, z) of the sites' boxes counts
 // the blocks it reaches, the host scans the counts, and the entries of a
 // block are put in site order.
 #include <cstring>
