@@ -656,7 +656,8 @@ int rs_tile_run(pp_ctx *ctx, pp_rsplan *rp, const double *kf, int nbc, int NB, c
   // Four lines a work-group (one a wavefront) where 16 leave the chip short of
   // work-groups (fewer than two per CU: 20^3, 64 bands, 18 projectors, states
   // 125 -> 100 us), and for states of more than 16 bands, whose work-groups
-  // wait on each other's lines (90^3, FP32: 823 -> 769 us; 108^3: the same).
+  // wait on each other's lines (64 FP32 bands, 4 projectors: 90^3 749 -> 608 us,
+  // 108^3 1162 -> 1101).
   // Else 16, which read the lines' tables together (108^3, 4 bands: 378 us
   // against 417).
   const long cols = (long)L.nxb * f1;
